@@ -156,11 +156,15 @@ int strip_mlem_synchronize(strip_mlem_ctx* ctx);
  * threads_per_block must be a multiple of 64 (one wavefront per event). */
 int strip_mlem_set_launch(strip_mlem_ctx* ctx, int n_blocks,
                           int threads_per_block);
-/* Selects the hot-path implementation: 0 = automatic (row band when the
- * mode and grid allow it), 1 = bbox wavefront kernel (every mode), 2 =
- * row-band LDS kernels (Gaussian kernel, sensitivity none or numerator).
+/* Selects the hot-path implementation: 0 = automatic (row bands when the
+ * mode and grid allow it: in their moment form, which sums a row's run from a
+ * table instead of pixel by pixel, where every tiling knob below has its
+ * default value and the events are dense enough, else as 2), 1 = bbox
+ * wavefront kernel (every mode), 2 = row-band LDS kernels over the runs'
+ * pixels (Gaussian kernel, sensitivity none or numerator).
  * Returns STRIP_MLEM_ERR_UNSUPPORTED when the requested one cannot run the
- * context's mode or grid.  strip_mlem_get_algorithm returns the one in use. */
+ * context's mode or grid.  strip_mlem_get_algorithm returns the one in use (2
+ * for either form of the row bands). */
 int strip_mlem_set_algorithm(strip_mlem_ctx* ctx, int algorithm);
 int strip_mlem_get_algorithm(const strip_mlem_ctx* ctx);
 
@@ -215,9 +219,10 @@ int strip_mlem_set_backprojection_occupancy(strip_mlem_ctx* ctx,
 int strip_mlem_set_span_table(strip_mlem_ctx* ctx, int enable);
 int strip_mlem_get_span_table(strip_mlem_ctx* ctx, int* in_use);
 
-/* The plan in use: band rows of both kernels, the widest back-projection
- * task window (columns) and the number of (event, band) pairs of both
- * kernels. */
+/* The row-band tiling: band rows of both kernels, the widest
+ * back-projection task window (columns) and the number of (event, band) pairs
+ * of both kernels (where the moment form is in use, those its events would
+ * have). */
 int strip_mlem_get_band_tiling(strip_mlem_ctx* ctx, int* forward_rows,
                                int* backward_rows, int* window_columns,
                                int64_t* forward_pairs,

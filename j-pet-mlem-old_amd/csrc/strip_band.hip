@@ -1151,7 +1151,18 @@ bool band_window_fits(const DeviceGeometry& g) {
          kLdsLimit;
 }
 
+bool default_tuning(const BandTuning& t) {
+  const BandTuning d;
+  return t.fwd_rows == d.fwd_rows && t.bwd_rows == d.bwd_rows &&
+         t.bwd_waves == d.bwd_waves && t.bucket == d.bucket &&
+         t.fwd_pairs == d.fwd_pairs && t.bwd_pairs == d.bwd_pairs &&
+         t.fwd_group == d.fwd_group && t.bwd_group == d.bwd_group &&
+         t.auto_groups == d.auto_groups && t.bwd_cu_waves == d.bwd_cu_waves &&
+         t.recurrence == d.recurrence && t.spans == d.spans;
+}
+
 void band_release(BandPlan& plan) {
+  moment_release(plan.moment);
   free_list(plan.bwd);
   free_list(plan.fwd);
   free_ptr(plan.partial);
@@ -1189,6 +1200,7 @@ int band_prepare_once(BandPlan& plan, const DeviceGeometry& g,
   free_ptr(plan.records);
   free_ptr(plan.order);
   free_ptr(plan.spans);
+  moment_release(plan.moment);
   plan.ready = false;
   plan.n_events = n_events;
   if (!plan.rhoT[0]) {
@@ -1196,6 +1208,18 @@ int band_prepare_once(BandPlan& plan, const DeviceGeometry& g,
     BAND_TRY(hipMalloc(&plan.rhoT[1], sizeof(float) * n_pixels));
     BAND_TRY(hipMalloc(&plan.bpT, sizeof(float) * n_pixels));
     BAND_TRY(hipMemsetAsync(plan.bpT, 0, sizeof(float) * n_pixels, stream));
+  }
+  static std::atomic<int64_t> generations{0};
+  plan.generation = ++generations;
+  if (plan.tuning.moments && default_tuning(plan.tuning)) {
+    bool built = false;
+    if (moment_prepare(plan.moment, g, ev, n_events, plan.rhoT, plan.bpT,
+                       stream, &built, err))
+      return -1;
+    if (built) {
+      plan.ready = true;
+      return 0;
+    }
   }
   const int64_t n = n_events;
   const unsigned blocks = (unsigned)((n + 255) / 256);
@@ -1369,8 +1393,6 @@ int band_prepare_once(BandPlan& plan, const DeviceGeometry& g,
     BAND_TRY(hipMalloc(&plan.desc, sizeof(BandInstance) * kDescSlots));
   for (int k = 0; k < kDescSlots; ++k) plan.desc_host[k] = BandInstance{};
   plan.n_custom = 0;
-  static std::atomic<int64_t> generations{0};
-  plan.generation = ++generations;
   for (int c = 0; c < 2; ++c) plan.desc_host[c] = band_descriptor(plan, g, c);
   BAND_TRY(hipMemcpyAsync(plan.desc, plan.desc_host,
                           sizeof(BandInstance) * kDescSlots,
@@ -1525,6 +1547,18 @@ int band_iteration(BandPlan& plan, const DeviceGeometry& g,
     if (err) *err = "the band algorithm does not fold sensitivity into D";
     return -1;
   }
+  if (plan.moment.ready) {
+    if (moment_forward(plan.moment, plan.curT, stream, err)) return -1;
+    if (t_fwd) BAND_TRY(hipEventRecord(t_fwd, stream));
+    if (moment_inverse(plan.moment, guard_zero, plan.moment.inv, nullptr,
+                       stream, err) ||
+        moment_backward(plan.moment, plan.curT, stream, err))
+      return -1;
+    if (t_bwd) BAND_TRY(hipEventRecord(t_bwd, stream));
+    if (!finalize) return 0;
+    return band_finalize(plan, g, sensitivity_mode, stream, err, scale,
+                         bp_out);
+  }
   if (dispatch_forward(plan, g, 0, nullptr, stream, err)) return -1;
   if (t_fwd) BAND_TRY(hipEventRecord(t_fwd, stream));
   if (plan.n_events > 0) {
@@ -1544,6 +1578,19 @@ int band_iteration(BandPlan& plan, const DeviceGeometry& g,
 int band_forward_only(BandPlan& plan, const DeviceGeometry& g,
                       const EventSoA& ev, float* denominators,
                       hipStream_t stream, std::string* err) {
+  if (plan.moment.ready) {
+    const unsigned blocks = (unsigned)((plan.n_events + 255) / 256);
+    // D in record order into the weights (free between iterations), then
+    // back to the caller's event order
+    if (moment_forward(plan.moment, plan.curT, stream, err) ||
+        moment_inverse(plan.moment, 1, nullptr, plan.moment.inv, stream, err))
+      return -1;
+    hipLaunchKernelGGL(unpermute_kernel, dim3(blocks), dim3(256), 0, stream,
+                       plan.moment.inv, plan.moment.order, plan.n_events,
+                       denominators);
+    BAND_TRY(hipGetLastError());
+    return 0;
+  }
   if (dispatch_forward(plan, g, 0, nullptr, stream, err)) return -1;
   if (plan.n_events > 0) {
     const unsigned blocks = (unsigned)((plan.n_events + 255) / 256);
@@ -1592,6 +1639,8 @@ int band_backproject(BandPlan& plan, const DeviceGeometry& g,
 int band_count(BandPlan& plan, const DeviceGeometry& g, const EventSoA& ev,
                unsigned long long* d_total, hipStream_t stream,
                std::string* err) {
+  if (plan.moment.ready)
+    return moment_count(plan.moment, d_total, stream, err);
   return dispatch_forward(plan, g, 1, d_total, stream, err);
 }
 

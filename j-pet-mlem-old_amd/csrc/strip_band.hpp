@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "strip_device.hpp"
+#include "strip_moment.hpp"
 
 namespace strip {
 
@@ -61,7 +62,14 @@ struct BandTuning {
   // 1 = build the span table when it fits, 0 = solve every row's run in the
   // iteration kernels
   int spans = 1;
+  // 1 = the moment form (strip_moment.hpp) where every other knob has its
+  // default value and the events suit it, 0 = always the row-band lists
+  int moments = 1;
 };
+
+// Whether a caller has left every knob at its default, so that the form of
+// the iteration is free to choose.
+bool default_tuning(const BandTuning& t);
 
 // Per-event parameters of the row-band kernels, packed in one 32-byte record
 // so a pair costs one cache-line access: ellipse centre (cz, cy), quadratic
@@ -119,6 +127,9 @@ constexpr int kDescSlots = 6;
 
 struct BandPlan {
   bool ready = false;
+  // ready: the plan runs in the moment form and has no pair lists, records,
+  // span table or partials of its own
+  MomentPlan moment;
   BandTuning tuning;
   PairList fwd, bwd;
   int Wt = 0;         // bound on the task windows: bucket + widest bbox

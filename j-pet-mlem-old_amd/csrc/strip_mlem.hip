@@ -676,6 +676,10 @@ int adjoint_ready(strip_mlem_ctx* ctx, bool full_plan = true) {
   if (effective_algorithm(ctx) != 2)
     return strip::fail(STRIP_MLEM_ERR_UNSUPPORTED,
                        "gradients need the row-band algorithm");
+  if (ctx->band.tuning.moments) {
+    ctx->band.tuning.moments = 0;
+    ctx->band_dirty = ctx->subsets_dirty = true;
+  }
   if (!full_plan) return STRIP_MLEM_OK;
   int rc = ensure_band(ctx);
   if (rc) return rc;
@@ -828,6 +832,58 @@ int active_plans(strip_mlem_ctx* ctx,
     if (rc) return rc;
     plans.push_back(&ctx->band);
   }
+  return STRIP_MLEM_OK;
+}
+
+// The row-band tiling that the resident events' plans have, or, for plans in
+// the moment form, would have: those plans' lists are built, described and
+// released again.
+int describe_tiling(strip_mlem_ctx* ctx, int* forward_group,
+                    int* backward_group, int* forward_rows,
+                    int* backward_rows, int* window_columns,
+                    int64_t* forward_pairs, int64_t* backward_pairs) {
+  std::vector<const strip::BandPlan*> plans;
+  int rc = active_plans(ctx, plans);
+  if (rc) return rc;
+  int wt = 0;
+  int64_t nf = 0, nb = 0;
+  for (size_t i = 0; i < plans.size(); ++i) {
+    const strip::BandPlan* p = plans[i];
+    strip::BandPlan lists;
+    if (p->moment.ready) {
+      std::string err;
+      const int64_t parts = (int64_t)plans.size();
+      const int64_t lo = ctx->n_events * (int64_t)i / parts;
+      const EventSoA view{ctx->ev.a + lo, ctx->ev.b + lo, ctx->ev.c + lo,
+                          ctx->ev.box + lo};
+      lists.tuning = p->tuning;
+      lists.tuning.moments = 0;
+      lists.rhoT[0] = p->rhoT[0];
+      lists.rhoT[1] = p->rhoT[1];
+      lists.bpT = p->bpT;
+      lists.owns_images = false;
+      const int failed = strip::band_prepare(lists, ctx->g, view, p->n_events,
+                                             ctx->stream, &err);
+      p = &lists;
+      if (failed) {
+        strip::band_release(lists);
+        return strip::fail(STRIP_MLEM_ERR_HIP, "band plan: " + err);
+      }
+    }
+    if (i == 0) {
+      if (forward_group) *forward_group = p->fwd_group;
+      if (backward_group) *backward_group = p->bwd_group;
+      if (forward_rows) *forward_rows = p->fwd.H;
+      if (backward_rows) *backward_rows = p->bwd.H;
+    }
+    wt = std::max(wt, p->bwd.Wt);
+    nf += p->fwd.n_pairs;
+    nb += p->bwd.n_pairs;
+    if (p == &lists) strip::band_release(lists);
+  }
+  if (window_columns) *window_columns = wt;
+  if (forward_pairs) *forward_pairs = nf;
+  if (backward_pairs) *backward_pairs = nb;
   return STRIP_MLEM_OK;
 }
 
@@ -1383,6 +1439,12 @@ int strip_mlem_set_algorithm(strip_mlem_ctx* ctx, int algorithm) {
                        "ordered subsets run on the row-band algorithm: set "
                        "one subset before choosing the bbox kernel");
   ctx->algorithm = algorithm;
+  const int moments = algorithm == 2 ? 0 : 1;
+  if (ctx->band.tuning.moments != moments) {
+    ctx->band.tuning.moments = moments;
+    ctx->band_dirty = true;
+    ctx->subsets_dirty = true;
+  }
   return STRIP_MLEM_OK;
 }
 
@@ -1439,12 +1501,8 @@ int strip_mlem_get_band_groups(strip_mlem_ctx* ctx, int* forward_group,
   CTX_CHECK(ctx);
   if (effective_algorithm(ctx) != 2)
     return strip::fail(STRIP_MLEM_ERR_STATE, "row-band algorithm not in use");
-  std::vector<const strip::BandPlan*> plans;
-  int rc = active_plans(ctx, plans);
-  if (rc) return rc;
-  if (forward_group) *forward_group = plans[0]->fwd_group;
-  if (backward_group) *backward_group = plans[0]->bwd_group;
-  return STRIP_MLEM_OK;
+  return describe_tiling(ctx, forward_group, backward_group, nullptr, nullptr,
+                         nullptr, nullptr, nullptr);
 }
 
 int strip_mlem_set_backprojection_waves(strip_mlem_ctx* ctx, int waves) {
@@ -1476,6 +1534,11 @@ int strip_mlem_set_exp_mode(strip_mlem_ctx* ctx, int mode) {
   if (!ctx) return strip::fail(STRIP_MLEM_ERR_ARGUMENT, "ctx is NULL");
   if (mode != 0 && mode != 1)
     return strip::fail(STRIP_MLEM_ERR_ARGUMENT, "exp mode must be 0 or 1");
+  if (ctx->band.tuning.recurrence != mode && ctx->band.tuning.moments) {
+    // the knob leaves or regains its default: the plans' form may change
+    ctx->band_dirty = true;
+    ctx->subsets_dirty = true;
+  }
   ctx->band.tuning.recurrence = mode;
   for (auto& p : ctx->subsets) p.tuning.recurrence = mode;
   return STRIP_MLEM_OK;
@@ -1505,7 +1568,8 @@ int strip_mlem_get_span_table(strip_mlem_ctx* ctx, int* in_use) {
   for (const strip::BandPlan* p : plans)
     if (p->n_events > 0) {
       any = true;
-      all = all && p->spans != nullptr;
+      // (the moment form keeps every row's run with its pairs)
+      all = all && (p->spans != nullptr || p->moment.ready);
     }
   *in_use = any && all ? 1 : 0;
   return STRIP_MLEM_OK;
@@ -1518,22 +1582,8 @@ int strip_mlem_get_band_tiling(strip_mlem_ctx* ctx, int* forward_rows,
   CTX_CHECK(ctx);
   if (effective_algorithm(ctx) != 2)
     return strip::fail(STRIP_MLEM_ERR_STATE, "row-band algorithm not in use");
-  std::vector<const strip::BandPlan*> plans;
-  int rc = active_plans(ctx, plans);
-  if (rc) return rc;
-  if (forward_rows) *forward_rows = plans[0]->fwd.H;
-  if (backward_rows) *backward_rows = plans[0]->bwd.H;
-  int wt = 0;
-  int64_t nf = 0, nb = 0;
-  for (const strip::BandPlan* p : plans) {
-    wt = std::max(wt, p->bwd.Wt);
-    nf += p->fwd.n_pairs;
-    nb += p->bwd.n_pairs;
-  }
-  if (window_columns) *window_columns = wt;
-  if (forward_pairs) *forward_pairs = nf;
-  if (backward_pairs) *backward_pairs = nb;
-  return STRIP_MLEM_OK;
+  return describe_tiling(ctx, nullptr, nullptr, forward_rows, backward_rows,
+                         window_columns, forward_pairs, backward_pairs);
 }
 
 int strip_mlem_kernel_evaluations(strip_mlem_ctx* ctx, int64_t* count) {
@@ -2047,6 +2097,7 @@ int strip_mlem_batch_create(int device, strip_mlem_batch** out) {
     return strip::fail(STRIP_MLEM_ERR_HIP, "cannot create batch stream");
   }
   b->cu_count = prop.multiProcessorCount;
+  b->tuning.moments = 0;
   *out = b;
   return STRIP_MLEM_OK;
 }

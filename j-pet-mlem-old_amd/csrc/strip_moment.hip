@@ -1,0 +1,1134 @@
+// Moment-table form of the strip MLEM iteration (kernels + host driver); the
+// algorithm is described in strip_moment.hpp.
+#include <hip/hip_runtime.h>
+#include <hipcub/hipcub.hpp>
+
+#include <algorithm>
+#include <cmath>
+#include <string>
+#include <type_traits>
+#include <vector>
+
+#include "strip_band.hpp"
+#include "strip_band_device.hpp"
+#include "strip_device.hpp"
+#include "strip_moment.hpp"
+
+namespace strip {
+namespace {
+
+constexpr int R = kMomentRows;
+constexpr int kGroup = 16;  // pairs of one 1 KiB group
+
+// exp(v) ~ sum c_m v^m, m < NM, on [-1, 1] with the least largest relative
+// error, 1.9e-7 (a linear program over 2001 Chebyshev points).  The vertex may
+// then lie reach * sigma_z from the line, 2 (3 / sqrt 2 + reach) reach = 1, for
+// |C u delta| <= 1 on every u of a 3-sigma run.
+template <int NM>
+struct ExpPoly;
+template <>
+struct ExpPoly<8> {
+  static constexpr double reach = 0.2140;
+  static constexpr float c[8] = {
+      0.9999998808238608f,    1.000001053962846f,   0.5000048572256811f,
+      0.16665825143600693f,   0.04163906763089733f, 0.008348694726996652f,
+      0.0014365374436724502f, 0.00019297136769021376f};
+};
+constexpr double kRunHalf = 2.1213203435596424;  // 3 / sqrt 2, in sigma_z
+
+typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+
+// Half of the moments of one (row, side, position): one LDS access.  A cell
+// (side, position) is two halves of 16 rows each, so the 16 lanes of a band
+// read consecutive bytes.
+template <int NM>
+struct HalfCell {
+  static constexpr int W = NM / 2;
+  float w[W];
+  __device__ static HalfCell load(const float* p) {
+    HalfCell v;
+    if constexpr (W == 4) {
+      const float4v x = *reinterpret_cast<const float4v*>(p);
+      v.w[0] = x.x;
+      v.w[1] = x.y;
+      v.w[2] = x.z;
+      v.w[3] = x.w;
+    } else {
+      __builtin_memcpy(v.w, p, sizeof(v.w));
+    }
+    return v;
+  }
+  __device__ void store(float* p) const {
+    if constexpr (W == 4)
+      *reinterpret_cast<float4v*>(p) = float4v{w[0], w[1], w[2], w[3]};
+    else
+      __builtin_memcpy(p, w, sizeof(w));
+  }
+  __device__ static constexpr int half_words() { return R * W; }
+  __device__ static constexpr int cell_words() { return 2 * R * W; }
+};
+
+// The line of a bin on one row of its band and its column, evaluated alike in
+// every kernel (contraction off): runs are stored relative to `column`.
+struct LineRow {
+  float x;     // z coordinate
+  int column;  // nearest column, inside the columns a clamped bbox can hold
+};
+
+__device__ inline LineRow line_row(const MomentInstance& d, int bin, int row) {
+#pragma clang fp contract(off)
+  const int jt = bin % d.nt, rest = bin / d.nt;
+  const int ix = rest % d.nx, band = rest / d.nx;
+  const float xc = d.x_lo + ((float)ix + 0.5f) * d.dx;
+  const float tc = d.t_lo + ((float)jt + 0.5f) * d.dt;
+  LineRow l;
+  l.x = xc - tc * (((float)row - 0.5f * (R - 1)) * d.g.pixel_height);
+  const float col = rintf((l.x - d.g.tl_z_half_w) * d.g.inv_pixel_width);
+  l.column = (int)fminf(fmaxf(col, 0.0f), (float)max(d.g.n_z - 2, 0));
+  (void)band;
+  return l;
+}
+
+__device__ inline int bin_band(const MomentInstance& d, int bin) {
+  return bin / (d.nt * d.nx);
+}
+
+// lane i of each row of 16 lanes, in all of them (a DPP operand)
+template <int I>
+__device__ inline float row_lane(float v) {
+  return __builtin_bit_cast(
+      float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x150 + I,
+                                      0xF, 0xF, true));
+}
+template <int I>
+__device__ inline int row_lane(uint32_t v) {
+  return __builtin_amdgcn_mov_dpp((int)v, 0x150 + I, 0xF, 0xF, true);
+}
+
+// Keeps LDS accesses of one wavefront in program order across lanes: the
+// hardware executes them in order, so only the compiler must not move them.
+__device__ inline void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// ---------------------------------------------------------------------------
+// plan
+// ---------------------------------------------------------------------------
+
+struct PlanStats {
+  unsigned long long pairs;
+  int max_bands;
+  int max_tan;  // bit pattern of a non-negative float
+};
+
+__device__ inline int box_bands(const uint2 box) {
+  const int x0 = box.x & 0xffff, x1 = box.x >> 16;
+  const int y0 = box.y & 0xffff, y1 = box.y >> 16;
+  return (x1 > x0 && y1 > y0) ? (y1 - 1) / R - y0 / R + 1 : 0;
+}
+
+__global__ __launch_bounds__(256) void moment_stats_kernel(
+    const uint2* __restrict__ box, const float4* __restrict__ a, int64_t n,
+    PlanStats* __restrict__ stats) {
+  unsigned long long pairs = 0;
+  int bands = 0;
+  float tan = 0.0f;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
+       e += (int64_t)gridDim.x * blockDim.x) {
+    const int c = box_bands(box[e]);
+    pairs += (unsigned long long)c;
+    bands = max(bands, c);
+    // (a NaN stays out: such an event's box is empty or its bin is clamped)
+    if (c) tan = fmaxf(tan, fabsf(a[e].z));
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    pairs += __shfl_xor(pairs, o);
+    bands = max(bands, __shfl_xor(bands, o));
+    tan = fmaxf(tan, __shfl_xor(tan, o));
+  }
+  __shared__ unsigned long long sp[4];
+  __shared__ int sb[4], st[4];
+  if ((threadIdx.x & 63) == 0) {
+    const int w = threadIdx.x >> 6;
+    sp[w] = pairs;
+    sb[w] = bands;
+    st[w] = __builtin_bit_cast(int, tan);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 4; ++w) {
+      pairs += sp[w];
+      bands = max(bands, sb[w]);
+      st[0] = max(st[0], st[w]);
+    }
+    atomicAdd(&stats->pairs, pairs);
+    atomicMax(&stats->max_bands, bands);
+    atomicMax(&stats->max_tan, st[0]);
+  }
+}
+
+__global__ __launch_bounds__(256) void fill_words_kernel(uint32_t* p, int64_t n,
+                                                         uint32_t v) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    p[i] = v;
+}
+
+__device__ inline int tan_bin(const MomentInstance& d, float t) {
+  const float j = floorf((t - d.t_lo) / d.dt);
+  return (int)fminf(fmaxf(j, 0.0f), (float)(d.nt - 1));
+}
+
+// event order: tan bin, then the band of the bbox top, then the bbox's
+// column, so the pairs of a bin come from a few runs of neighbouring records
+__global__ __launch_bounds__(256) void moment_order_kernel(
+    MomentInstance d, const uint2* __restrict__ box,
+    const float4* __restrict__ a, int64_t n, uint32_t* __restrict__ keys,
+    int* __restrict__ values) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  const uint2 b = box[e];
+  keys[e] = ((uint32_t)min(tan_bin(d, a[e].z), 63) << 26) |
+            (((b.y & 0xffff) / R) << 15) | (b.x & 0x7fff);
+  values[e] = (int)e;
+}
+
+// records in that order, and their band counts
+__global__ __launch_bounds__(256) void moment_records_kernel(
+    EventSoA ev, const int* __restrict__ order, int64_t n,
+    BandRecord* __restrict__ rec, int* __restrict__ counts) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int e = order[i];
+  const float4 a = ev.a[e], b = ev.b[e], c = ev.c[e];
+  const uint2 box = ev.box[e];
+  BandRecord r;
+  r.cz = a.x;
+  r.cy = a.y;
+  r.A = b.x;
+  r.B = b.y;
+  r.P = c.x;
+  r.Q0 = c.y;
+  r.bx = box.x;
+  r.by = box.y;
+  rec[i] = r;
+  counts[i] = box_bands(box);
+}
+
+// (bin, record) of every pair
+__global__ __launch_bounds__(256) void moment_emit_kernel(
+    MomentInstance d, const BandRecord* __restrict__ rec,
+    const int* __restrict__ counts, const int* __restrict__ offsets, int64_t n,
+    uint32_t* __restrict__ keys, int* __restrict__ values) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int c = counts[i];
+  if (!c) return;
+  const BandRecord r = rec[i];
+  const float t = -r.B * d.g.inv_2c;
+  const int jt = tan_bin(d, t);
+  const int b0 = (int)(r.by & 0xffff) / R;
+  const int at = offsets[i];
+  for (int k = 0; k < c; ++k) {
+    const float yc = d.g.tl_y_half_h -
+                     ((float)((b0 + k) * R) + 0.5f * (R - 1)) *
+                         d.g.pixel_height;
+    const float x = r.cz + t * (yc - r.cy);
+    const float f = floorf((x - d.x_lo) / d.dx);
+    const int ix = (int)fminf(fmaxf(f, 0.0f), (float)(d.nx - 1));
+    keys[at + k] = (uint32_t)(((b0 + k) * d.nx + ix) * d.nt + jt);
+    values[at + k] = (int)i;
+  }
+}
+
+// first / end pair of every bin that has pairs
+__global__ __launch_bounds__(256) void moment_bins_kernel(
+    const uint32_t* __restrict__ keys, int64_t n, int* __restrict__ first,
+    int* __restrict__ end) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t k = keys[i];
+  if (i == 0 || keys[i - 1] != k) first[k] = (int)i;
+  if (i == n - 1 || keys[i + 1] != k) end[k] = (int)i + 1;
+}
+
+// pieces of `chunk` pairs each bin is cut into (0 at n_bins)
+__global__ __launch_bounds__(256) void moment_piece_count_kernel(
+    const int* __restrict__ first, const int* __restrict__ end, int n_bins,
+    int chunk, int* __restrict__ counts) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= n_bins)
+    counts[i] = i < n_bins ? (end[i] - first[i] + chunk - 1) / chunk : 0;
+}
+
+// groups[k] = (bin, first pair) of every 16-pair group
+__global__ __launch_bounds__(256) void moment_group_emit_kernel(
+    const int* __restrict__ first, const int* __restrict__ end, int n_bins,
+    const int* __restrict__ group_of, int2* __restrict__ groups) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n_bins) return;
+  int k = group_of[i];
+  for (int p = first[i]; p < end[i]; p += kGroup) groups[k++] = make_int2(i, p);
+}
+
+// tasks of a bin: its groups in nearly equal parts of at most `chunk` pairs
+__global__ __launch_bounds__(256) void moment_task_emit_kernel(
+    const int* __restrict__ first, const int* __restrict__ end, int n_bins,
+    int chunk, const int* __restrict__ group_of,
+    const int* __restrict__ offsets, int4* __restrict__ tasks) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n_bins) return;
+  const int total = end[i] - first[i];
+  const int groups = (total + kGroup - 1) / kGroup;
+  const int parts = (total + chunk - 1) / chunk;
+  for (int k = 0; k < parts; ++k) {
+    const int lo = (int)((int64_t)groups * k / parts);
+    const int hi = (int)((int64_t)groups * (k + 1) / parts);
+    tasks[offsets[i] + k] = make_int4(
+        i, group_of[i] + lo, min(total, hi * kGroup) - lo * kGroup, 0);
+  }
+}
+
+// The pairs' data in groups of 16 pairs of one bin, 1 KiB each, laid out as a
+// wavefront reads it: one 16-byte load per lane holds four steps of four pairs
+// (pair 4 s + g belongs to lane group g = lane / 16 of step s).  With i =
+// lane % 16:
+//   word s / 2, lanes i = 8 (s % 2) + k: field k of the pair of step s:
+//     cz, cy, tan, 4 id sec^2 (times the exp2 scale), P', Q0' of the record,
+//     the record's index and the index of its partial sum for this band;
+//   half-word s of words 2 and 3: the run of band row i: a | b << 8, a columns
+//     left of the line's column and b from it on, or, for a run that misses
+//     the line's column, 0x8000 | n << 8 | (offset + positions / 2), n
+//     columns, the first at the line's column + offset (both parts at most
+//     `positions`, so that either form addresses cells that exist).
+// Missing pairs of a last group are zero.
+__global__ __launch_bounds__(256) void moment_pack_kernel(
+    MomentInstance d, const BandRecord* __restrict__ rec,
+    const int2* __restrict__ groups, const int* __restrict__ end,
+    const int* __restrict__ values, int n_groups,
+    uint4* __restrict__ blocks, int* __restrict__ status) {
+  __shared__ uint32_t words[kGroup * 16];
+  const int pair = threadIdx.x >> 4, row = threadIdx.x & 15;
+  const int step = pair >> 2, grp = pair & 3;
+  for (int k = blockIdx.x; k < n_groups; k += gridDim.x) {
+    const int bin = groups[k].x, p = groups[k].y + pair;
+    uint32_t word = 0, field = 0;
+    if (p < end[bin]) {
+      const int e = values[p];
+      const BandRecord r = rec[e];
+      int x0, x1, y0, y1;
+      record_box(r, x0, x1, y0, y1);
+      const int band = bin_band(d, bin);
+      const LineRow l = line_row(d, bin, row);
+      const RowSpan s = row_span(d.g, r.cz, r.cy, r.A, r.B, r.P, r.Q0, x0, x1,
+                                 y0, y1, band * R + row);
+      if (s.n > 0) {
+        const int a = l.column - s.lo, b = s.lo + s.n - l.column;
+        const int off = s.lo - l.column + d.positions / 2;
+        if (a >= 0 && b >= 0 && a <= d.positions && b <= d.positions)
+          word = (uint32_t)(a | (b << 8));
+        else if (s.n <= d.positions && off >= 0 && off <= d.positions)
+          word = 0x8000u | ((uint32_t)s.n << 8) | (uint32_t)off;
+        else
+          *status = 1;  // does not fit: the host falls back
+      }
+      const float t = -r.B * d.g.inv_2c;
+      const float ad = 4.0f * d.g.inv_pow_sigma_dl * __builtin_fmaf(t, t, 1.0f);
+      switch (row) {
+        case 0: field = __builtin_bit_cast(uint32_t, r.cz); break;
+        case 1: field = __builtin_bit_cast(uint32_t, r.cy); break;
+        case 2: field = __builtin_bit_cast(uint32_t, t); break;
+        case 3: field = __builtin_bit_cast(uint32_t, ad * kExp2Scale); break;
+        case 4: field = __builtin_bit_cast(uint32_t, r.P); break;
+        case 5: field = __builtin_bit_cast(uint32_t, r.Q0); break;
+        case 6: field = (uint32_t)e; break;
+        case 7: field = (uint32_t)(e * d.max_bands + (band - y0 / R)); break;
+        default: break;
+      }
+    }
+    __syncthreads();  // the previous group has been written out
+    if (row < 8)
+      words[(grp * 16 + (step & 1) * 8 + row) * 4 + (step >> 1)] = field;
+    reinterpret_cast<uint16_t*>(words)[(grp * 16 + row) * 8 + 4 + step] =
+        (uint16_t)word;
+    __syncthreads();
+    if (threadIdx.x < 64)
+      blocks[(int64_t)k * 64 + threadIdx.x] =
+          reinterpret_cast<const uint4*>(words)[threadIdx.x];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// iteration
+// ---------------------------------------------------------------------------
+
+// Row terms of a pair on this lane.
+struct RowTerms {
+  float delta;   // vertex - line
+  float qa;      // exponent at the vertex
+  float pre;     // row prefactor
+  float w;       // pre exp2(exponent on the line): the polynomial's factor
+  uint32_t run;  // run word
+};
+
+// of step S of a group
+template <int S>
+__device__ inline RowTerms row_terms(const uint4v& v, float y, float y2,
+                                     float x, float qc) {
+  constexpr int F = 8 * (S & 1);
+  const uint32_t fields = S < 2 ? v.x : v.y, runs = S < 2 ? v.z : v.w;
+  const float f = __builtin_bit_cast(float, fields);
+  RowTerms r;
+  const float dy = y - row_lane<F + 1>(f);
+  r.delta = __builtin_fmaf(row_lane<F + 2>(f), dy, row_lane<F>(f) - x);
+  r.qa = row_lane<F + 3>(f) * dy * dy;
+  r.pre = __builtin_amdgcn_rsqf(
+      __builtin_fmaf(row_lane<F + 4>(f), y2, row_lane<F + 5>(f)));
+  const float q = __builtin_fmaf(qc * r.delta, r.delta, r.qa);
+  r.w = r.pre * __builtin_amdgcn_exp2f(q);
+  r.run = (S & 1) ? runs >> 16 : runs & 0xffff;
+  return r;
+}
+
+// Forward projection of one task: the workgroup tabulates the image around
+// the bin's line, then every wavefront step takes four pairs, 16 lanes each.
+// Bound by VALU issue (58 instructions per step of 64 rows, whatever the runs'
+// lengths; 0.64 per CU-cycle) and the waits around it.  2e7 events, 1000 x 400
+// at 1 mm: 6.4 ms, against 12.4 ms for the kernel that walks the runs' pixels
+// (33 columns per row, 6.9 lane operations each).
+template <int NM, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void moment_forward_kernel(
+    const MomentInstance* __restrict__ desc, const int4* __restrict__ tasks) {
+  using Half = HalfCell<NM>;
+  constexpr int W = Half::W, HALF = Half::half_words(),
+                CELL = Half::cell_words();
+  extern __shared__ float4v table4[];
+  float* const table = reinterpret_cast<float*>(table4);
+  const int4 task = tasks[blockIdx.x];
+  const MomentInstance& d = desc[task.w];
+  const int lane = threadIdx.x & 63;
+  const int row = lane & (R - 1);
+  const int grp = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int bin = task.x;
+  const int P = d.positions;
+  const int n_y = d.g.n_y, n_z = d.g.n_z;
+  const float w_px = d.g.pixel_width;
+  const int iy = bin_band(d, bin) * R + row;
+  const LineRow l = line_row(d, bin, row);
+  const float qc = d.g.C * kExp2Scale;
+  const float* __restrict__ rhoT = d.rhoT;
+  const int n_here = task.z;
+  const uint4v* __restrict__ base =
+      reinterpret_cast<const uint4v*>(d.blocks) + (int64_t)task.y * 64;
+  const int last = (n_here - 1) / kGroup;
+  uint4v next = gload(base + min(wave, last) * 64 + lane);
+  {
+    // thread = (row, side, MG consecutive moments); cell k of a side holds
+    // the sums over its first k columns outward from the line
+    constexpr int MG = (NM + 2 * WAVES - 1) / (2 * WAVES);
+    static_assert(W % MG == 0, "a thread's moments stay in one half");
+    const int side = grp & 1;
+    const int m0 = (int)(threadIdx.x >> 5) * MG;
+    if (m0 < NM) {
+      float* cell = table + (side * (P + 1)) * CELL + (m0 / W) * HALF +
+                    row * W + m0 % W;
+      float acc[MG], cm[MG];
+#pragma unroll
+      for (int i = 0; i < MG; ++i) {
+        acc[i] = 0.0f;
+        cm[i] = ExpPoly<NM>::c[m0 + i];
+        cell[i] = 0.0f;
+      }
+      const int dir = side ? 1 : -1;
+      int col = side ? l.column : l.column - 1;
+      const bool row_in = iy < n_y;
+      const float du = side ? w_px : -w_px;
+      const float inv_s = d.inv_s;
+      const float u0 = __builtin_fmaf((float)col, w_px, d.g.tl_z_half_w) - l.x;
+      // eight columns' pixels are in flight together
+      for (int k0 = 0; k0 < P; k0 += 8) {
+        float rho[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int x = col + k * dir;
+          const bool in = row_in && x >= 0 && x < n_z;
+          const float v = gload(rhoT + (in ? (int64_t)x * n_y + iy : 0));
+          rho[k] = in ? v : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          if (k0 + k >= P) break;
+          cell += CELL;
+          const float u = __builtin_fmaf((float)(k0 + k), du, u0);
+          const float v = u * inv_s;
+          float t = __builtin_amdgcn_exp2f(qc * u * u) * rho[k];
+          // (u / s)^m0
+          if constexpr (MG < NM) {
+            const float v2 = v * v;
+            if (MG % 2 == 1 && (m0 & 1)) t *= v;
+            if (MG % 4 != 0 && (m0 & 2)) t *= v2;
+            if (m0 & 4) t *= v2 * v2;
+          }
+#pragma unroll
+          for (int i = 0; i < MG; ++i) {
+            acc[i] = __builtin_fmaf(cm[i], t, acc[i]);
+            cell[i] = acc[i];
+            t *= v;
+          }
+        }
+        col += 8 * dir;
+      }
+    }
+  }
+  __syncthreads();
+  const float y = pixel_center_y(d.g, iy);
+  const float y2 = y * y;
+  const float cs = d.cs;
+  float* __restrict__ partial = d.partial;
+  const float* const left = table + row * W;
+  const float* const right = left + (P + 1) * CELL;
+  auto step = [&](auto tag, const uint4v& v, int j) {
+    constexpr int S = decltype(tag)::value;
+    const RowTerms r = row_terms<S>(v, y, y2, l.x, qc);
+    const float eta = cs * r.delta;
+    const int a = (int)(r.run & 0xff), b = (int)((r.run >> 8) & 0x7f);
+    const float* pl = left + a * CELL;
+    const float* pr = right + b * CELL;
+    const Half l0 = Half::load(pl), l1 = Half::load(pl + HALF);
+    const Half r0 = Half::load(pr), r1 = Half::load(pr + HALF);
+    float t = l1.w[W - 1] + r1.w[W - 1];
+#pragma unroll
+    for (int i = W - 2; i >= 0; --i)
+      t = __builtin_fmaf(t, eta, l1.w[i] + r1.w[i]);
+#pragma unroll
+    for (int i = W - 1; i >= 0; --i)
+      t = __builtin_fmaf(t, eta, l0.w[i] + r0.w[i]);
+    float s = t * r.w;
+    // runs that miss the line's column, and rows whose sum is not finite (an
+    // infinite pixel times powers of both signs), pixel by pixel
+    const bool direct = r.run >= 0x8000u;
+    if (direct || !(__builtin_fabsf(s) < __builtin_inff())) {
+      const int n = direct ? b : a + b;
+      const int col = l.column + (direct ? a - P / 2 : -a);
+      float dz = (__builtin_fmaf((float)col, w_px, d.g.tl_z_half_w) - l.x) -
+                 r.delta;
+      float acc = 0.0f;
+      const float* src = rhoT + (int64_t)col * n_y + iy;
+      for (int k = 0; k < n; ++k) {
+        acc = __builtin_fmaf(
+            __builtin_amdgcn_exp2f(__builtin_fmaf(qc * dz, dz, r.qa)),
+            gload(src), acc);
+        src += n_y;
+        dz += w_px;
+      }
+      s = n > 0 ? r.pre * acc : 0.0f;
+    }
+    s = group_total<R>(s);
+    // the lane that holds the partial's index stores it
+    if (row == 7 + 8 * (S & 1) && j + 4 * S + grp < n_here)
+      gstore(partial + (int)(S < 2 ? v.x : v.y), s);
+  };
+  for (int k = wave; k <= last; k += WAVES) {
+    const uint4v cur = next;
+    next = gload(base + min(k + WAVES, last) * 64 + lane);
+    const int j = k * kGroup;
+    step(std::integral_constant<int, 0>{}, cur, j);
+    if (j + 4 >= n_here) break;
+    step(std::integral_constant<int, 1>{}, cur, j);
+    if (j + 8 >= n_here) break;
+    step(std::integral_constant<int, 2>{}, cur, j);
+    if (j + 12 >= n_here) break;
+    step(std::integral_constant<int, 3>{}, cur, j);
+  }
+}
+
+// D_e = sum of the record's partials; inv_e = 1 / D_e (guarded or not)
+__global__ __launch_bounds__(256) void moment_inverse_kernel(
+    const int* __restrict__ counts, int64_t n, int max_bands,
+    const float* __restrict__ partial, int guard, float* __restrict__ inv,
+    float* __restrict__ denominators) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  float s = 0.0f;
+  const int c = counts[e];
+  for (int k = 0; k < c; ++k) s += partial[e * max_bands + k];
+  if (denominators) denominators[e] = s;
+  if (inv) inv[e] = guard ? ((s > 0.0f) ? 1.0f / s : 0.0f) : 1.0f / s;
+}
+
+// Back-projection of one task by one wavefront that owns the cells of its
+// bin's line in LDS.  A step takes four pairs, 16 lanes each.  A row's 16
+// additions (8 terms at the end cell of either side) go in four rounds of one
+// 16-byte read-modify-write per lane; in each round the four lane groups work on
+// different (side, half) quarters of the cells, so two pairs never meet in a word
+// and no atomics are needed.  Bound by VALU issue (79 instructions per step of 64
+// rows) and the chain of LDS round trips at the six wavefronts per CU that the
+// cells leave room for.  2e7 events, 1000 x 400 at 1 mm: 9.9 ms, against
+// 22.0 ms for the kernel that adds pixel by pixel (an LDS read and write each).
+template <int NM>
+__global__ __launch_bounds__(64) void moment_backward_kernel(
+    const MomentInstance* __restrict__ desc, const int4* __restrict__ tasks) {
+  using Half = HalfCell<NM>;
+  constexpr int W = Half::W, HALF = Half::half_words(),
+                CELL = Half::cell_words();
+  extern __shared__ float4v cells4[];
+  const int4 task = tasks[blockIdx.x];
+  const MomentInstance& d = desc[task.w];
+  const int lane = threadIdx.x;
+  const int row = lane & (R - 1);
+  const int grp = lane >> 4;
+  const int bin = task.x;
+  const int P = d.positions;
+  const int n_y = d.g.n_y, n_z = d.g.n_z;
+  const float w_px = d.g.pixel_width;
+  const int y_base = bin_band(d, bin) * R;
+  const int iy = y_base + row;
+  const LineRow l = line_row(d, bin, row);
+  const float qc = d.g.C * kExp2Scale;
+  const float cs = d.cs;
+  const float y = pixel_center_y(d.g, iy);
+  const float y2 = y * y;
+  const float* __restrict__ inv = d.inv;
+  float* __restrict__ bpT = d.bpT;
+  const int side_words = (P + 1) * CELL;
+  for (int i = lane; i < side_words / 2; i += 64)
+    cells4[i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+  const int n_here = task.z;
+  const uint4v* __restrict__ base =
+      reinterpret_cast<const uint4v*>(d.blocks) + (int64_t)task.y * 64;
+  const int last = (n_here - 1) / kGroup;
+  float* const mine = reinterpret_cast<float*>(cells4) + row * W;
+  const bool odd = grp & 1, high = grp & 2;
+  const int h0 = high ? HALF : 0;
+  const int h1 = HALF - h0;
+  // the weights of a group's pairs: the lanes that hold a record's index
+  // fetch its weight (word 0: steps 0 and 1, word 1: steps 2 and 3)
+  struct Weights {
+    float w01, w23;
+  };
+  auto weights = [&](const uint4v& v) {
+    const bool index = (row & 7) == 6;
+    Weights w;
+    w.w01 = gload(inv + (index ? (int)v.x : 0));
+    w.w23 = gload(inv + (index ? (int)v.y : 0));
+    return w;
+  };
+  struct Terms {
+    RowTerms r;
+    Half v0, v1;  // the moments of this lane's first and second half
+    float weight;
+    int a, b;
+  };
+  auto terms = [&](auto tag, const uint4v& v, const Weights& wt, int j) {
+    constexpr int S = decltype(tag)::value;
+    Terms t;
+    t.r = row_terms<S>(v, y, y2, l.x, qc);
+    const float eta = cs * t.r.delta;
+    t.weight = row_lane<6 + 8 * (S & 1)>(S < 2 ? wt.w01 : wt.w23);
+    if (j + 4 * S + grp >= n_here) t.weight = 0.0f;
+    const float f = t.r.run >= 0x8000u ? 0.0f : t.r.w * t.weight;
+    float m[NM];
+    m[0] = f;
+#pragma unroll
+    for (int i = 1; i < NM; ++i) m[i] = m[i - 1] * eta;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      t.v0.w[i] = high ? m[W + i] : m[i];
+      t.v1.w[i] = high ? m[i] : m[W + i];
+    }
+    t.a = (int)(t.r.run & 0xff) * CELL;
+    t.b = (int)((t.r.run >> 8) & 0x7f) * CELL + side_words;
+    return t;
+  };
+  auto add = [&](const Terms& t) {
+    float* const p0 = mine + (odd ? t.b : t.a);
+    float* const p1 = mine + (odd ? t.a : t.b);
+    auto round = [](float* p, const Half& v) {
+      Half x = Half::load(p);
+#pragma unroll
+      for (int i = 0; i < W; ++i) x.w[i] += v.w[i];
+      x.store(p);
+      lds_order();
+    };
+    round(p0 + h0, t.v0);
+    round(p1 + h0, t.v0);
+    round(p0 + h1, t.v1);
+    round(p1 + h1, t.v1);
+    if (t.r.run >= 0x8000u && t.weight != 0.0f) {
+      const int n = (int)((t.r.run >> 8) & 0x7f);
+      const int col = l.column + (int)(t.r.run & 0xff) - P / 2;
+      float dz = (__builtin_fmaf((float)col, w_px, d.g.tl_z_half_w) - l.x) -
+                 t.r.delta;
+      float* dst = bpT + (int64_t)col * n_y + iy;
+      const float f = t.r.pre * t.weight;
+      for (int k = 0; k < n; ++k) {
+        gatomic_add(dst, f * __builtin_amdgcn_exp2f(
+                                 __builtin_fmaf(qc * dz, dz, t.r.qa)));
+        dst += n_y;
+        dz += w_px;
+      }
+    }
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  using S2 = std::integral_constant<int, 2>;
+  using S3 = std::integral_constant<int, 3>;
+  // groups two ahead, weights one ahead, a step's terms while the step
+  // before it is added
+  uint4v cur = gload(base + lane);
+  uint4v next = gload(base + min(1, last) * 64 + lane);
+  Weights wt = weights(cur);
+  lds_order();
+  Terms t = terms(S0{}, cur, wt, 0);
+  for (int k = 0; k <= last; ++k) {
+    const uint4v next2 = gload(base + min(k + 2, last) * 64 + lane);
+    const Weights wt_next = weights(next);
+    const int j = k * kGroup;
+    Terms u = terms(S1{}, cur, wt, j);
+    add(t);
+    t = terms(S2{}, cur, wt, j);
+    if (j + 4 < n_here) add(u);
+    u = terms(S3{}, cur, wt, j);
+    if (j + 8 < n_here) add(t);
+    t = terms(S0{}, next, wt_next, j + kGroup);
+    if (j + 12 < n_here) add(u);
+    cur = next;
+    next = next2;
+    wt = wt_next;
+  }
+  lds_order();
+  // inward sums, cell by cell: lane = (row, side, half); the pixel's value
+  // replaces word 0 of its cell
+  {
+    const int side = grp & 1, half = grp >> 1;
+    float* cell = mine + side * side_words + half * HALF;
+    float s[W] = {}, c[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+      c[i] = half ? ExpPoly<NM>::c[W + i] : ExpPoly<NM>::c[i];
+    const float inv_s = d.inv_s;
+    for (int k = P; k >= 1; --k) {
+      float* at = cell + k * CELL;
+      const Half x = Half::load(at);
+#pragma unroll
+      for (int i = 0; i < W; ++i) s[i] += x.w[i];
+      const int col = side ? l.column + k - 1 : l.column - k;
+      const float u =
+          __builtin_fmaf((float)col, w_px, d.g.tl_z_half_w) - l.x;
+      const float v = u * inv_s;
+      float t = s[W - 1] * c[W - 1];
+#pragma unroll
+      for (int i = W - 2; i >= 0; --i) t = __builtin_fmaf(t, v, s[i] * c[i]);
+      if (half) {
+        t *= v * v;
+        t *= W == 4 ? v * v : v;
+      }
+      t += __shfl_xor(t, 32);
+      if (!half) *at = t * __builtin_amdgcn_exp2f(qc * u * u);
+    }
+  }
+  lds_order();
+  // column by column into the image: lane = (row, column of four)
+  int x_lo = l.column - P, x_hi = l.column + P;
+  for (int o = 1; o < R; o <<= 1) {
+    x_lo = min(x_lo, __shfl_xor(x_lo, o));
+    x_hi = max(x_hi, __shfl_xor(x_hi, o));
+  }
+  x_lo = max(__builtin_amdgcn_readfirstlane(x_lo), 0);
+  x_hi = min(__builtin_amdgcn_readfirstlane(x_hi), n_z);
+  for (int x = x_lo + grp; x < x_hi; x += 4) {
+    const int k = x - l.column;
+    const int cell = k >= 0 ? k + 1 : -k;
+    if (cell <= P && iy < n_y) {
+      const float val = mine[(k >= 0 ? side_words : 0) + cell * CELL];
+      if (val != 0.0f) gatomic_add(bpT + (int64_t)x * n_y + iy, val);
+    }
+  }
+}
+
+// total += columns of every stored run
+__global__ __launch_bounds__(256) void moment_count_kernel(
+    const uint32_t* __restrict__ blocks, int64_t n_lanes,
+    unsigned long long* __restrict__ total) {
+  unsigned long long mine = 0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+       i < 2 * n_lanes; i += (int64_t)gridDim.x * blockDim.x) {
+    const uint32_t w = blocks[(i >> 1) * 4 + 2 + (i & 1)];
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t run = (w >> (16 * k)) & 0xffff;
+      const uint32_t b = (run >> 8) & 0x7f;
+      mine += (run & 0x8000u) ? b : (run & 0xff) + b;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o);
+  if ((threadIdx.x & 63) == 0 && mine) atomicAdd(total, mine);
+}
+
+// ---------------------------------------------------------------------------
+// host
+// ---------------------------------------------------------------------------
+
+constexpr size_t kLds = 160 * 1024;
+// Runs of a smaller sigma_z (in pixels) are a few columns long, and how their
+// offsets round decides their kernel values.
+constexpr double kMinSigmaPixels = 1.4;
+constexpr int kFwdChunk = 2048;  // pairs of a forward workgroup's task
+constexpr int kBwdChunk = 1024;  // pairs of a back-projection wavefront's task
+
+unsigned grid_of(int64_t n) { return (unsigned)((n + 255) / 256); }
+
+// Cells per row and side: a run reaches at most its half length plus the
+// vertex's distance from the line plus half a column (the line's distance from
+// its column) to either side, and its columns from the line's on count that
+// column too.
+int positions_for(const DeviceGeometry& g, double reach) {
+  const double sigma_px = 1.0 / std::sqrt((double)g.inv_pow_sigma_z) /
+                          g.pixel_width;
+  const double p = (kRunHalf + reach) * sigma_px + 1.55;
+  return p < 1e6 ? (int)std::floor(p) : 1000000;
+}
+
+size_t table_bytes(int positions, int terms) {
+  return sizeof(float) * 2 * (size_t)(positions + 1) * R * terms;
+}
+
+// Device memory handed out from one allocation, in 256-byte steps.
+struct Arena {
+  size_t used = 0;
+  template <typename T>
+  size_t take(int64_t n) {
+    const size_t at = used;
+    used += (sizeof(T) * (size_t)std::max<int64_t>(n, 1) + 255) & ~(size_t)255;
+    return at;
+  }
+};
+
+}  // namespace
+
+bool moment_supported(const DeviceGeometry& g) {
+  const double sigma_px = 1.0 / std::sqrt((double)g.inv_pow_sigma_z) /
+                          g.pixel_width;
+  const int p = positions_for(g, ExpPoly<8>::reach);
+  return sigma_px >= kMinSigmaPixels && p <= 120 && table_bytes(p, 8) <= kLds &&
+         g.n_z >= 4 && g.n_y >= 1;
+}
+
+void moment_release(MomentPlan& plan) {
+  if (plan.arena) (void)hipFree(plan.arena);
+  if (plan.lists) (void)hipFree(plan.lists);
+  plan = MomentPlan{};
+}
+
+int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
+                   const EventSoA& ev, int64_t n, float* const rhoT[2],
+                   float* bpT, hipStream_t stream, bool* built,
+                   std::string* err) {
+  *built = false;
+  moment_release(plan);
+  if (n <= 0 || n > 0x3fffffff || !moment_supported(g)) return 0;
+  struct Scratch {
+    void* p = nullptr;
+    ~Scratch() {
+      if (p) (void)hipFree(p);
+    }
+  } stats_mem, temp;
+  // what the sizes of the plan depend on
+  BAND_TRY(hipMalloc(&stats_mem.p, sizeof(PlanStats) + 64));
+  PlanStats* d_stats = static_cast<PlanStats*>(stats_mem.p);
+  hipLaunchKernelGGL(fill_words_kernel, dim3(1), dim3(256), 0, stream,
+                     (uint32_t*)d_stats, (int64_t)((sizeof(PlanStats) + 64) / 4),
+                     0u);
+  hipLaunchKernelGGL(moment_stats_kernel,
+                     dim3(std::min<unsigned>(grid_of(n), 1024)), dim3(256), 0,
+                     stream, ev.box, ev.a, n, d_stats);
+  BAND_TRY(hipGetLastError());
+  PlanStats st{};
+  BAND_TRY(hipMemcpyAsync(&st, d_stats, sizeof(st), hipMemcpyDeviceToHost,
+                          stream));
+  BAND_TRY(hipStreamSynchronize(stream));
+  const int64_t n_pairs = (int64_t)st.pairs;
+  const double max_tan = (double)__builtin_bit_cast(float, st.max_tan);
+  if (n_pairs <= 0 || n_pairs > 0x3fffffff || !(max_tan < 1e3) ||
+      (double)n * st.max_bands > 2e9)
+    return 0;
+
+  // bins: half the reach for the vertex, half for the shear over a band
+  const double sigma = 1.0 / std::sqrt((double)g.inv_pow_sigma_z);
+  const double reach = ExpPoly<8>::reach * sigma * 0.995;
+  MomentInstance d{};
+  d.g = g;
+  const double dx = reach;
+  const double dt = reach / (0.5 * (R - 1) * (double)g.pixel_height);
+  const double iz = g.inv_pow_sigma_z, id = g.inv_pow_sigma_dl;
+  const double k = 8.0 * iz * id / (4.0 * id + 2.0 * iz);
+  const double half_width = 3.0 / std::sqrt(k);
+  const double margin = 2.0 * half_width + 4.0 * g.pixel_width +
+                        0.5 * R * g.pixel_height * max_tan + dx;
+  const double z_span = (double)g.n_z * g.pixel_width + 2.0 * margin;
+  const double nt = std::ceil(2.0 * max_tan / dt) + 1.0;
+  const double nx = std::ceil(z_span / dx) + 1.0;
+  const int n_bands = (g.n_y + R - 1) / R;
+  if (!(nt <= 4096.0) || !(nx * nt * n_bands <= (double)(1 << 24))) return 0;
+  d.nx = (int)nx;
+  d.nt = (int)nt;
+  d.x_lo = (float)((double)g.tl_z - margin);
+  d.dx = (float)dx;
+  d.t_lo = (float)(-0.5 * nt * dt);
+  d.dt = (float)dt;
+  d.positions = positions_for(g, ExpPoly<8>::reach);
+  d.max_bands = std::max(st.max_bands, 1);
+  const double s = (kRunHalf + ExpPoly<8>::reach) * sigma;
+  d.inv_s = (float)(1.0 / s);
+  d.cs = (float)((double)g.C * s);
+  d.n_events = n;
+  const int n_bins = d.nx * d.nt * n_bands;
+
+  // what building the plan needs
+  Arena work;
+  const int64_t sort_n = std::max<int64_t>(n, n_pairs);
+  const int64_t bins1 = (int64_t)n_bins + 1;
+  const size_t w_keys = work.take<uint32_t>(sort_n);
+  const size_t w_keys2 = work.take<uint32_t>(sort_n);
+  const size_t w_vals = work.take<int>(sort_n);
+  const size_t w_vals2 = work.take<int>(sort_n);
+  const size_t w_rec = work.take<BandRecord>(n);
+  const size_t w_offsets = work.take<int>(n);
+  const size_t w_first = work.take<int>(bins1);
+  const size_t w_end = work.take<int>(bins1);
+  const size_t w_count = work.take<int>(bins1);
+  const size_t w_pieces = work.take<int>(3 * bins1);
+  size_t cub = 0;
+  {
+    size_t b = 0;
+    hipcub::DoubleBuffer<uint32_t> kb(nullptr, nullptr);
+    hipcub::DoubleBuffer<int> vb(nullptr, nullptr);
+    BAND_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, b, kb, vb,
+                                                (int)sort_n, 0, 32, stream));
+    cub = std::max(cub, b);
+    BAND_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, b, (int*)nullptr,
+                                              (int*)nullptr, (int)n, stream));
+    cub = std::max(cub, b);
+    BAND_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, b, (int*)nullptr,
+                                              (int*)nullptr, (int)bins1,
+                                              stream));
+    cub = std::max(cub, b);
+  }
+  const size_t w_cub = work.take<char>((int64_t)cub);
+  // the plan's per-event memory; its groups and tasks are sized below
+  Arena own;
+  const size_t o_partial = own.take<float>(n * d.max_bands);
+  const size_t o_inv = own.take<float>(n);
+  const size_t o_counts = own.take<int>(n);
+  const size_t o_order = own.take<int>(n);
+  const size_t o_desc = own.take<MomentInstance>(2);
+  size_t free_bytes = 0, total_bytes = 0;
+  BAND_TRY(hipMemGetInfo(&free_bytes, &total_bytes));
+  if (64 * (size_t)n_pairs + own.used > free_bytes / 2 ||
+      80 * (size_t)n_pairs + own.used + work.used > free_bytes)
+    return 0;
+  // out of memory or unsuited events: the row-band lists take over
+  auto give_up = [&]() {
+    (void)hipGetLastError();
+    moment_release(plan);
+    return 0;
+  };
+  if (hipMalloc(&plan.arena, own.used) != hipSuccess) {
+    plan.arena = nullptr;
+    return give_up();
+  }
+  if (hipMalloc(&temp.p, work.used) != hipSuccess) {
+    temp.p = nullptr;
+    return give_up();
+  }
+  char* A = static_cast<char*>(plan.arena);
+  char* W = static_cast<char*>(temp.p);
+  plan.partial = reinterpret_cast<float*>(A + o_partial);
+  plan.inv = reinterpret_cast<float*>(A + o_inv);
+  plan.counts = reinterpret_cast<int*>(A + o_counts);
+  plan.order = reinterpret_cast<int*>(A + o_order);
+  plan.desc = reinterpret_cast<MomentInstance*>(A + o_desc);
+  uint32_t* keys = reinterpret_cast<uint32_t*>(W + w_keys);
+  uint32_t* keys2 = reinterpret_cast<uint32_t*>(W + w_keys2);
+  int* vals = reinterpret_cast<int*>(W + w_vals);
+  int* vals2 = reinterpret_cast<int*>(W + w_vals2);
+  BandRecord* rec = reinterpret_cast<BandRecord*>(W + w_rec);
+  int* offsets = reinterpret_cast<int*>(W + w_offsets);
+  int* first = reinterpret_cast<int*>(W + w_first);
+  int* end = reinterpret_cast<int*>(W + w_end);
+  int* piece_count = reinterpret_cast<int*>(W + w_count);
+  int* pieces[3];  // first group, forward and back-projection task of each bin
+  for (int i = 0; i < 3; ++i)
+    pieces[i] = reinterpret_cast<int*>(W + w_pieces) + i * bins1;
+  void* cub_mem = W + w_cub;
+
+  // events in bin-friendly order, their records, their pairs by bin
+  hipLaunchKernelGGL(moment_order_kernel, dim3(grid_of(n)), dim3(256), 0,
+                     stream, d, ev.box, ev.a, n, keys, vals);
+  BAND_TRY(hipGetLastError());
+  {
+    hipcub::DoubleBuffer<uint32_t> kb(keys, keys2);
+    hipcub::DoubleBuffer<int> vb(vals, vals2);
+    size_t b = cub;
+    BAND_TRY(hipcub::DeviceRadixSort::SortPairs(cub_mem, b, kb, vb, (int)n, 0,
+                                                32, stream));
+    BAND_TRY(hipMemcpyAsync(plan.order, vb.Current(), sizeof(int) * n,
+                            hipMemcpyDeviceToDevice, stream));
+  }
+  hipLaunchKernelGGL(moment_records_kernel, dim3(grid_of(n)), dim3(256), 0,
+                     stream, ev, plan.order, n, rec, plan.counts);
+  BAND_TRY(hipGetLastError());
+  {
+    size_t b = cub;
+    BAND_TRY(hipcub::DeviceScan::ExclusiveSum(cub_mem, b, plan.counts, offsets,
+                                              (int)n, stream));
+  }
+  hipLaunchKernelGGL(moment_emit_kernel, dim3(grid_of(n)), dim3(256), 0,
+                     stream, d, rec, plan.counts, offsets, n, keys, vals);
+  BAND_TRY(hipGetLastError());
+  int end_bit = 1;
+  while (end_bit < 32 && (1 << end_bit) < n_bins) ++end_bit;
+  hipcub::DoubleBuffer<uint32_t> kb(keys, keys2);
+  hipcub::DoubleBuffer<int> vb(vals, vals2);
+  {
+    size_t b = cub;
+    BAND_TRY(hipcub::DeviceRadixSort::SortPairs(cub_mem, b, kb, vb,
+                                                (int)n_pairs, 0, end_bit,
+                                                stream));
+  }
+  // the bins' groups and tasks
+  hipLaunchKernelGGL(fill_words_kernel, dim3(1024), dim3(256), 0, stream,
+                     (uint32_t*)first, (int64_t)(w_count - w_first) / 4, 0u);
+  hipLaunchKernelGGL(moment_bins_kernel, dim3(grid_of(n_pairs)), dim3(256), 0,
+                     stream, kb.Current(), n_pairs, first, end);
+  BAND_TRY(hipGetLastError());
+  const int chunks[3] = {kGroup, kFwdChunk, kBwdChunk};
+  int totals[3] = {0, 0, 0};
+  for (int i = 0; i < 3; ++i) {
+    hipLaunchKernelGGL(moment_piece_count_kernel, dim3(grid_of(bins1)),
+                       dim3(256), 0, stream, first, end, n_bins, chunks[i],
+                       piece_count);
+    size_t b = cub;
+    BAND_TRY(hipcub::DeviceScan::ExclusiveSum(cub_mem, b, piece_count,
+                                              pieces[i], (int)bins1, stream));
+    BAND_TRY(hipMemcpyAsync(&totals[i], pieces[i] + n_bins, sizeof(int),
+                            hipMemcpyDeviceToHost, stream));
+  }
+  BAND_TRY(hipStreamSynchronize(stream));
+  // Where the bins hold few pairs, tabulating and expanding their lines costs
+  // more than walking the runs' pixels, and more so the more cells a line has.
+  // Measured per iteration, lists against moments: 24 cells, 2.4 pairs per bin
+  // 0.14 and 0.31 ms, 25 pairs 0.48 and 0.38 ms; 48 cells, 33 pairs 0.95 and
+  // 1.52 ms, 369 pairs 5.6 and 3.6 ms; 13 cells, 1.1 pairs 0.036 and 0.031 ms.
+  if ((double)n_pairs < 1.6 * (d.positions - 16) * (double)totals[1])
+    return give_up();
+  const int n_groups = totals[0];
+  Arena lists;
+  const size_t o_blocks = lists.take<uint4>((int64_t)n_groups * 64);
+  const size_t o_groups = lists.take<int2>(n_groups);
+  const size_t o_fwd = lists.take<int4>(totals[1]);
+  const size_t o_bwd = lists.take<int4>(totals[2]);
+  if (hipMalloc(&plan.lists, lists.used) != hipSuccess) {
+    plan.lists = nullptr;
+    return give_up();
+  }
+  char* L = static_cast<char*>(plan.lists);
+  plan.blocks = reinterpret_cast<uint32_t*>(L + o_blocks);
+  plan.fwd_tasks = reinterpret_cast<int4*>(L + o_fwd);
+  plan.bwd_tasks = reinterpret_cast<int4*>(L + o_bwd);
+  int2* groups = reinterpret_cast<int2*>(L + o_groups);
+  hipLaunchKernelGGL(moment_group_emit_kernel, dim3(grid_of(n_bins)),
+                     dim3(256), 0, stream, first, end, n_bins, pieces[0],
+                     groups);
+  for (int pass = 0; pass < 2; ++pass)
+    hipLaunchKernelGGL(moment_task_emit_kernel, dim3(grid_of(n_bins)),
+                       dim3(256), 0, stream, first, end, n_bins,
+                       chunks[1 + pass], pieces[0], pieces[1 + pass],
+                       pass ? plan.bwd_tasks : plan.fwd_tasks);
+  int* d_status = reinterpret_cast<int*>(d_stats + 1);
+  hipLaunchKernelGGL(moment_pack_kernel,
+                     dim3((unsigned)std::min(n_groups, 1 << 20)), dim3(256), 0,
+                     stream, d, rec, groups, end, vb.Current(), n_groups,
+                     reinterpret_cast<uint4*>(plan.blocks), d_status);
+  BAND_TRY(hipGetLastError());
+  int status = 0;
+  BAND_TRY(hipMemcpyAsync(&status, d_status, sizeof(int),
+                          hipMemcpyDeviceToHost, stream));
+  d.blocks = plan.blocks;
+  d.partial = plan.partial;
+  d.counts = plan.counts;
+  d.inv = plan.inv;
+  d.bpT = bpT;
+  MomentInstance both[2] = {d, d};
+  for (int c = 0; c < 2; ++c) {
+    both[c].rhoT = rhoT[c];
+    both[c].rho_next = rhoT[c ^ 1];
+  }
+  BAND_TRY(hipMemcpyAsync(plan.desc, both, sizeof(both), hipMemcpyHostToDevice,
+                          stream));
+  BAND_TRY(hipStreamSynchronize(stream));
+  if (status) {
+    moment_release(plan);
+    return 0;
+  }
+  plan.inst = both[0];
+  plan.n_events = n;
+  plan.n_pairs = n_pairs;
+  plan.n_groups = n_groups;
+  plan.n_bins = n_bins;
+  plan.n_fwd = totals[1];
+  plan.n_bwd = totals[2];
+  plan.fwd_lds = plan.bwd_lds = table_bytes(d.positions, 8);
+  plan.fwd_waves = n_pairs / std::max(plan.n_fwd, 1) >= 200 ? 4 : 1;
+  for (const void* kern :
+       {reinterpret_cast<const void*>(moment_forward_kernel<8, 1>),
+        reinterpret_cast<const void*>(moment_forward_kernel<8, 4>),
+        reinterpret_cast<const void*>(moment_backward_kernel<8>)})
+    BAND_TRY(hipFuncSetAttribute(
+        kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds));
+  plan.ready = true;
+  *built = true;
+  return 0;
+}
+
+int moment_forward(MomentPlan& plan, int cur, hipStream_t stream,
+                   std::string* err) {
+  if (plan.n_fwd == 0) return 0;
+  auto kern = plan.fwd_waves == 4 ? moment_forward_kernel<8, 4>
+                                  : moment_forward_kernel<8, 1>;
+  hipLaunchKernelGGL(kern, dim3(plan.n_fwd), dim3(64 * plan.fwd_waves),
+                     plan.fwd_lds, stream, plan.desc + cur, plan.fwd_tasks);
+  BAND_TRY(hipGetLastError());
+  return 0;
+}
+
+int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
+                   hipStream_t stream, std::string* err) {
+  hipLaunchKernelGGL(moment_inverse_kernel, dim3(grid_of(plan.n_events)),
+                     dim3(256), 0, stream, plan.counts, plan.n_events,
+                     plan.inst.max_bands, plan.partial, guard, inv,
+                     denominators);
+  BAND_TRY(hipGetLastError());
+  return 0;
+}
+
+int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
+                    std::string* err) {
+  if (plan.n_bwd == 0) return 0;
+  hipLaunchKernelGGL(moment_backward_kernel<8>, dim3(plan.n_bwd), dim3(64),
+                     plan.bwd_lds, stream, plan.desc + cur, plan.bwd_tasks);
+  BAND_TRY(hipGetLastError());
+  return 0;
+}
+
+int moment_count(MomentPlan& plan, unsigned long long* total,
+                 hipStream_t stream, std::string* err) {
+  hipLaunchKernelGGL(moment_count_kernel, dim3(2048), dim3(256), 0, stream,
+                     plan.blocks, (int64_t)plan.n_groups * 64, total);
+  BAND_TRY(hipGetLastError());
+  return 0;
+}
+
+}  // namespace strip

@@ -1,0 +1,104 @@
+// Moment-table form of the strip MLEM iteration (host interface).
+//
+// Along an image row an event's kernel is a Gaussian of one fixed width (sigma_z
+// alone sets it) around the row's vertex c = cz + tan dy, cut to the row's
+// in-ellipse run [lo, hi].  About a nearby line X that many events share,
+// with u = x - X and delta = c - X,
+//   exp(-(C/2)(x - c)^2) = exp(-(C/2) u^2) exp(C u delta) exp(-(C/2) delta^2),
+// and where |C u delta| <= 1 the middle factor is a degree-7 polynomial in
+// (C s delta)(u / s) to 1.9e-7.  Events are therefore split into (event, band)
+// pairs (a band = 16 image rows) and the pairs binned by band, by the vertex at
+// the band's middle and by tan: all pairs of a bin share one sheared line X(row)
+// from which no vertex strays further than 0.214 sigma_z.  Then
+//   forward          a workgroup tabulates, per row and side of the line, the
+//                    running sums over columns outward from the line of
+//                    rho exp(-(C/2) u^2) (u / s)^m, m = 0..7; a row's sum over
+//                    its run is 2 x 8 table words and a Horner evaluation,
+//                    whatever the run's length;
+//   back-projection  the transpose: a row adds weight x eta^m at the two cells
+//                    its run ends in; per task the cells are summed inward
+//                    and expanded back to pixels.
+// Sums run outward from the line, so no difference of large numbers is
+// formed and a pixel outside an event's run never enters its sums (an infinity
+// or NaN there stays away from it, as in the pixel-by-pixel kernels).  A run
+// that misses the line's column (a short run at an ellipse's tip) is walked
+// pixel by pixel.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <string>
+
+#include "strip_device.hpp"
+
+namespace strip {
+
+constexpr int kMomentRows = 16;  // image rows of a band
+
+// What the kernels need of one reconstruction (device array; a task names its
+// entry).
+struct MomentInstance {
+  DeviceGeometry g;
+  // bins: band-major, then the vertex at the band's middle row, then tan
+  int nx, nt;
+  float x_lo, dx;  // lower edge of bin 0 and bin width, z coordinate
+  float t_lo, dt;  // the same of tan
+  int positions;   // table cells per row and side, besides the empty one
+  int max_bands;
+  float inv_s;     // 1 / s
+  float cs;        // C s
+  const uint32_t* blocks;  // 1 KiB per 16 pairs (moment_pack_kernel)
+  const float* rhoT;       // image the forward pass reads (column-major)
+  float* rho_next;
+  float* partial;          // per (record, band of the record)
+  const int* counts;       // bands of each record
+  float* inv;
+  float* bpT;
+  int64_t n_events;
+};
+
+struct MomentPlan {
+  bool ready = false;
+  int64_t n_events = 0, n_pairs = 0;
+  int n_bins = 0, n_groups = 0;
+  int n_fwd = 0, n_bwd = 0;
+  int fwd_waves = 4;  // wavefronts per forward workgroup
+  size_t fwd_lds = 0, bwd_lds = 0;
+  MomentInstance inst;  // host copy (image 0)
+  void* arena = nullptr;  // per-event arrays and descriptors
+  void* lists = nullptr;  // pair groups and tasks
+  // pieces of them
+  uint32_t* blocks = nullptr;
+  float* partial = nullptr;
+  float* inv = nullptr;
+  int* counts = nullptr;
+  int* order = nullptr;     // record -> caller's event
+  int4* fwd_tasks = nullptr;  // (bin, first group, pairs, instance)
+  int4* bwd_tasks = nullptr;
+  MomentInstance* desc = nullptr;  // images 0 / 1
+};
+
+// Whether the geometry suits the moment form at all.
+bool moment_supported(const DeviceGeometry& g);
+
+// Builds the plan for the events.  *built = false (and 0) where the row-band
+// lists are the better choice or the plan does not fit.
+int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
+                   const EventSoA& ev, int64_t n_events, float* const rhoT[2],
+                   float* bpT, hipStream_t stream, bool* built,
+                   std::string* err);
+void moment_release(MomentPlan& plan);
+
+// The passes of an iteration reading image `cur`.
+int moment_forward(MomentPlan& plan, int cur, hipStream_t stream,
+                   std::string* err);
+// D_e = sum of the record's partials; inv (guarded or not) and / or D
+int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
+                   hipStream_t stream, std::string* err);
+int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
+                    std::string* err);
+// *total += kernel evaluations of the stored runs
+int moment_count(MomentPlan& plan, unsigned long long* total,
+                 hipStream_t stream, std::string* err);
+
+}  // namespace strip

@@ -1,0 +1,129 @@
+"""The moment form of the row-band iteration (csrc/strip_moment.hip) against
+the CPU oracle, at the edges of what it takes: band and grid remainders, runs
+clipped by the image, lines whose column is clamped, steep events, anisotropic
+pixels, the smallest lists and the smallest sigma.
+
+Tolerances, derived: a kernel value's polynomial factor is within 1.9e-7 and
+its 8-term FP32 evaluation within 8 x 6e-8 x e^2 = 3.5e-6 of exact (the terms'
+magnitudes sum to at most e^2 times the value); with the row terms' own FP32
+rounding (under 5e-6 between the row-band kernels and the oracle) a forward
+projection is within 1e-5.  Support counts are integers: exact.  Images: the
+graded bar, rel-L2 1e-4.
+"""
+import numpy as np
+import pytest
+
+from conftest import print_case
+
+pytestmark = pytest.mark.gpu
+
+# n_z, n_y, pixel width, height, sigma_z, sigma_dl, R, L, phantom half sizes,
+# events.  Lines of at most 16 cells (sigma_z up to 6 pixels) always take the
+# moment form; wider ones need dense bins.
+CASES = {
+    "command line defaults, sigma 1.5 px": (
+        100, 100, 0.01, 0.01, 0.015, 0.06, 0.5, 1.0, 0.3, 0.3, 20_011),
+    "object beyond every edge": (
+        61, 37, 5.0, 5.0, 10.0, 42.0, 250.0, 700.0, 220.0, 150.0, 6_000),
+    "one row past a band, flat pixels": (
+        128, 33, 2.0, 1.5, 10.0, 42.0, 120.0, 500.0, 100.0, 20.0, 5_000),
+    "fifteen rows, tall pixels": (
+        90, 15, 2.0, 4.0, 10.0, 42.0, 120.0, 500.0, 70.0, 25.0, 3_000),
+    "narrower than a run": (
+        12, 200, 2.0, 2.0, 12.0, 42.0, 300.0, 500.0, 20.0, 150.0, 4_000),
+    "steep events": (
+        200, 64, 2.0, 2.0, 10.0, 30.0, 70.0, 1200.0, 150.0, 40.0, 5_000),
+    "one event": (256, 160, 2.0, 2.0, 10.0, 42.0, 350.0, 500.0, 80.0, 60.0, 1),
+    "seventeen events": (
+        256, 160, 2.0, 2.0, 10.0, 42.0, 350.0, 500.0, 80.0, 60.0, 17),
+    "wide line, dense bins": (
+        300, 200, 1.0, 1.0, 10.0, 42.0, 250.0, 500.0, 40.0, 30.0, 30_000),
+}
+
+
+def _case(pystrip_mod, phantom_mod, oracle_mod, name, seed=5):
+    n_z, n_y, w, h, sz, sdl, R, L, a, b, n = CASES[name]
+    ev = phantom_mod.generate_events(
+        [phantom_mod.Ellipse(0.3 * a, -0.2 * b, 0.2 * a, 0.3 * b, 20, 3),
+         phantom_mod.Ellipse(0, 0, a, b, 0, 1)], R, L, sz, sdl, n, seed=seed,
+        batch=1 << 16)
+    g = pystrip_mod.Geometry.make(R, L, n_z, n_y, w, sz, sdl, pixel_height=h)
+    og = oracle_mod.geometry(R, L, n_z, n_y, w, h, sz, sdl, 0.0, 0.0)
+    return ev, g, og
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_moment_form_against_oracle(pystrip_mod, phantom_mod, oracle_mod,
+                                    name):
+    print_case("moment form:", name)
+    ev, g, og = _case(pystrip_mod, phantom_mod, oracle_mod, name)
+    rec = pystrip_mod.Reconstruction(g)
+    rec.set_events(ev)
+    _, ne = oracle_mod.support_counts(og, ev)
+    assert rec.kernel_evaluations() == int(ne.sum())
+    rho = np.random.default_rng(3).uniform(0.5, 2.0, rec.shape).astype(
+        np.float32)
+    rec.rho = rho
+    d = rec.forward().astype(np.float64)
+    ref = oracle_mod.forward(og, ev, rho).astype(np.float64)
+    assert np.array_equal(d > 0, ref > 0)
+    nz = ref > 0
+    err = np.max(np.abs(d[nz] - ref[nz]) / ref[nz]) if nz.any() else 0.0
+    print("events with support", int(nz.sum()), "of", len(ev), "max rel D",
+          err)
+    assert err < 1e-5
+    rec.iterate(3)
+    e = oracle_mod.rel_l2(rec.rho, oracle_mod.mlem(og, ev, rho0=rho,
+                                                   iterations=3))
+    print("rel-L2", e)
+    assert e <= 1e-4
+
+
+def test_moment_form_non_finite_pixels(pystrip_mod, phantom_mod, oracle_mod):
+    # a pixel that is not finite reaches the events whose support holds it
+    # and no others: as the pixel-by-pixel kernels give it
+    ev, g, og = _case(pystrip_mod, phantom_mod, oracle_mod,
+                      "object beyond every edge")
+    for value in (np.inf, np.nan):
+        print_case("moment form, pixel =", value)
+        rho = np.ones((g.n_y_pixels, g.n_z_pixels), np.float32)
+        rho[20, 30] = value
+        rho[5, 1] = value
+        out = []
+        for algorithm in (1, 0):
+            rec = pystrip_mod.Reconstruction(g)
+            rec.set_algorithm(algorithm)
+            rec.set_events(ev)
+            rec.rho = rho
+            out.append(rec.forward())
+        fine = np.isfinite(out[0])
+        assert 0 < fine.sum() < len(ev)
+        assert np.array_equal(fine, np.isfinite(out[1]))
+        assert np.array_equal(np.isnan(out[0]), np.isnan(out[1]))
+        nz = fine & (out[0] > 0)
+        assert np.max(np.abs(out[1][nz] - out[0][nz]) / out[0][nz]) < 1e-5
+
+
+def test_moment_form_knobs(pystrip_mod, phantom_mod, oracle_mod):
+    # leaving a knob's default takes the lists, returning to it the moment
+    # form again: the same reconstruction within rounding
+    print_case("moment form and tiling knobs")
+    ev, g, og = _case(pystrip_mod, phantom_mod, oracle_mod,
+                      "command line defaults, sigma 1.5 px")
+    ref = oracle_mod.mlem(og, ev, iterations=2)
+    rec = pystrip_mod.Reconstruction(g)
+    rec.set_events(ev)
+    tiling = rec.band_tiling()
+    assert tiling[:2] == (32, 16) and rec.band_groups() == (2, 4)
+    assert rec.span_table()
+    for change in (lambda: None, lambda: rec.set_exp_mode(0),
+                   lambda: rec.set_exp_mode(1),
+                   lambda: rec.set_span_table(False),
+                   lambda: rec.set_span_table(True),
+                   lambda: rec.set_algorithm(2),
+                   lambda: rec.set_algorithm(0)):
+        change()
+        rec.rho = np.ones(rec.shape, np.float32)
+        rec.iterate(2)
+        assert oracle_mod.rel_l2(rec.rho, ref) <= 1e-4
+        assert rec.band_tiling()[:2] == tiling[:2]
