@@ -199,19 +199,26 @@ __global__ __launch_bounds__(64 * kFwdWaves) void band_moments_kernel(
 //     w1 = 1/D, w2 = G/D^2 with D = sum K x0, G = sum K x1,
 //     gz = (Z1 - Z0 G/D) / D, gd = (Y1 - Y0 G/D) / D
 //     (the -2 terms of d ln K / d ln sigma_z cancel here).
-// Events with D <= 0 contribute nothing (the reference's guard).
+// Events with D <= 0 contribute nothing (the reference's guard).  counts: the
+// records' bands, or null for those of a forward list of height H.
 template <int NIMG>
 __global__ __launch_bounds__(256) void adjoint_event_kernel(
-    const BandRecord* __restrict__ rec, int64_t n, int H, int max_bands,
-    const float* __restrict__ moments, float* __restrict__ w1,
+    const BandRecord* __restrict__ rec, const int* __restrict__ counts,
+    int64_t n, int H, int max_bands, const float* __restrict__ moments,
+    float* __restrict__ w1,
     float* __restrict__ w2, float* __restrict__ value, float* __restrict__ gz,
     float* __restrict__ gd) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n) return;
-  int x0, x1, y0, y1;
-  record_box(rec[e], x0, x1, y0, y1);
+  int nb;
+  if (counts) {
+    nb = counts[e];
+  } else {
+    int x0, x1, y0, y1;
+    record_box(rec[e], x0, x1, y0, y1);
+    nb = band_count(y0, y1, x1 > x0, H, true);
+  }
   float m[kMoments * 2] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  const int nb = band_count(y0, y1, x1 > x0, H, true);
   for (int k = 0; k < nb; ++k) {
     const float* src = moments + (e * max_bands + k) * (kMoments * NIMG);
 #pragma unroll
@@ -333,10 +340,15 @@ void free_dev(T*& p) {
   p = nullptr;
 }
 
+// most bands of one event in the plan's forward pairs
+int plan_bands(const BandPlan& plan) {
+  return plan.moment.ready ? plan.moment.inst.max_bands : plan.fwd.max_bands;
+}
+
 int ensure_work(AdjointWork& wk, const BandPlan& plan, int64_t n_pixels,
                 std::string* err) {
   const int64_t n = std::max<int64_t>(plan.n_events, 1);
-  const int64_t m = n * plan.fwd.max_bands * kMoments * 2;
+  const int64_t m = n * plan_bands(plan) * kMoments * 2;
   if (m > wk.moments_cap) {
     free_dev(wk.moments);
     BAND_TRY(hipMalloc(&wk.moments, sizeof(float) * m));
@@ -377,6 +389,14 @@ template <int NIMG>
 int launch_moments(BandPlan& plan, const DeviceGeometry& g, AdjointWork& wk,
                    const float* x0T, const float* x1T, hipStream_t stream,
                    std::string* err) {
+  if (plan.moment.ready) {
+    const float* x[2] = {x0T, x1T};
+    for (int i = 0; i < NIMG; ++i)
+      if (moment_gradient(plan.moment, x[i], kMoments * NIMG,
+                          wk.moments + kMoments * i, stream, err))
+        return -1;
+    return 0;
+  }
   const PairList& L = plan.fwd;
   if (L.n_tasks == 0) return 0;
   const size_t lds = (size_t)L.Wt * 2 * L.H * sizeof(float) * NIMG;
@@ -433,8 +453,8 @@ int band_loglik_terms(BandPlan& plan, const DeviceGeometry& g,
   if (launch_moments<1>(plan, g, wk, rhoT, nullptr, stream, err)) return -1;
   const unsigned blocks = (unsigned)((n + 255) / 256);
   hipLaunchKernelGGL(adjoint_event_kernel<1>, dim3(blocks), dim3(256), 0,
-                     stream, plan.records, n, plan.fwd.H, plan.fwd.max_bands,
-                     wk.moments, w1, nullptr, val, gz, gd);
+                     stream, plan.records, plan.moment.counts, n, plan.fwd.H,
+                     plan_bands(plan), wk.moments, w1, nullptr, val, gz, gd);
   BAND_TRY(hipGetLastError());
   if (reduce_sum(wk, val, n, 0, stream, err) ||
       reduce_sum(wk, gz, n, 1, stream, err) ||
@@ -554,8 +574,8 @@ int band_mlem_adjoint_step(BandPlan& plan, const DeviceGeometry& g,
     if (launch_moments<2>(plan, g, wk, rhoT_k, hT, stream, err)) return -1;
     const unsigned blocks = (unsigned)((n + 255) / 256);
     hipLaunchKernelGGL(adjoint_event_kernel<2>, dim3(blocks), dim3(256), 0,
-                       stream, plan.records, n, plan.fwd.H,
-                       plan.fwd.max_bands, wk.moments, w1, w2, nullptr, gz,
+                       stream, plan.records, plan.moment.counts, n, plan.fwd.H,
+                       plan_bands(plan), wk.moments, w1, w2, nullptr, gz,
                        gd);
     BAND_TRY(hipGetLastError());
     if (reduce_sum(wk, gz, n, 0, stream, err) ||

@@ -1633,6 +1633,8 @@ int band_backproject(BandPlan& plan, const DeviceGeometry& g,
     if (err) *err = "band plan not prepared";
     return -1;
   }
+  if (plan.moment.ready)
+    return moment_backward(plan.moment, 0, stream, err, weights, outT);
   return dispatch_backward(plan, g, weights, outT, stream, err);
 }
 

@@ -676,10 +676,6 @@ int adjoint_ready(strip_mlem_ctx* ctx, bool full_plan = true) {
   if (effective_algorithm(ctx) != 2)
     return strip::fail(STRIP_MLEM_ERR_UNSUPPORTED,
                        "gradients need the row-band algorithm");
-  if (ctx->band.tuning.moments) {
-    ctx->band.tuning.moments = 0;
-    ctx->band_dirty = ctx->subsets_dirty = true;
-  }
   if (!full_plan) return STRIP_MLEM_OK;
   int rc = ensure_band(ctx);
   if (rc) return rc;

@@ -95,8 +95,15 @@ int moment_forward(MomentPlan& plan, int cur, hipStream_t stream,
 // D_e = sum of the record's partials; inv (guarded or not) and / or D
 int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
                    hipStream_t stream, std::string* err);
+// (weights in record order and a column-major image of the caller's, or null
+// for the plan's own)
 int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
-                    std::string* err);
+                    std::string* err, const float* weights = nullptr,
+                    float* into = nullptr);
+// out[stride * (record * max_bands + band of the record) + {0, 1, 2}] = sum K x,
+// sum K x Q, sum K x (w - Qd) of the column-major image xT (strip_adjoint.hip)
+int moment_gradient(MomentPlan& plan, const float* xT, int stride, float* out,
+                    hipStream_t stream, std::string* err);
 // *total += kernel evaluations of the stored runs
 int moment_count(MomentPlan& plan, unsigned long long* total,
                  hipStream_t stream, std::string* err);
