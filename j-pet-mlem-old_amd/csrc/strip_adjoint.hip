@@ -200,11 +200,13 @@ __global__ __launch_bounds__(64 * kFwdWaves) void band_moments_kernel(
 //     gz = (Z1 - Z0 G/D) / D, gd = (Y1 - Y0 G/D) / D
 //     (the -2 terms of d ln K / d ln sigma_z cancel here).
 // Events with D <= 0 contribute nothing (the reference's guard).  counts: the
-// records' bands, or null for those of a forward list of height H.
+// records' bands, or null for those of a forward list of height H; band k of
+// record e lies at e e_stride + k k_stride.
 template <int NIMG>
 __global__ __launch_bounds__(256) void adjoint_event_kernel(
     const BandRecord* __restrict__ rec, const int* __restrict__ counts,
-    int64_t n, int H, int max_bands, const float* __restrict__ moments,
+    int64_t n, int H, int64_t e_stride, int64_t k_stride,
+    const float* __restrict__ moments,
     float* __restrict__ w1,
     float* __restrict__ w2, float* __restrict__ value, float* __restrict__ gz,
     float* __restrict__ gd) {
@@ -220,7 +222,7 @@ __global__ __launch_bounds__(256) void adjoint_event_kernel(
   }
   float m[kMoments * 2] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   for (int k = 0; k < nb; ++k) {
-    const float* src = moments + (e * max_bands + k) * (kMoments * NIMG);
+    const float* src = moments + (e * e_stride + k * k_stride) * (kMoments * NIMG);
 #pragma unroll
     for (int i = 0; i < kMoments * NIMG; ++i) m[i] += src[i];
   }
@@ -348,7 +350,8 @@ int plan_bands(const BandPlan& plan) {
 int ensure_work(AdjointWork& wk, const BandPlan& plan, int64_t n_pixels,
                 std::string* err) {
   const int64_t n = std::max<int64_t>(plan.n_events, 1);
-  const int64_t m = n * plan_bands(plan) * kMoments * 2;
+  // (one more than the pairs: the moment form's spare)
+  const int64_t m = (n * plan_bands(plan) + 1) * kMoments * 2;
   if (m > wk.moments_cap) {
     free_dev(wk.moments);
     BAND_TRY(hipMalloc(&wk.moments, sizeof(float) * m));
@@ -452,9 +455,12 @@ int band_loglik_terms(BandPlan& plan, const DeviceGeometry& g,
   float* gd = wk.ev_buf + 4 * wk.ev_cap;
   if (launch_moments<1>(plan, g, wk, rhoT, nullptr, stream, err)) return -1;
   const unsigned blocks = (unsigned)((n + 255) / 256);
+  const bool by_band = plan.moment.ready;  // layout of the band moments
+  const int64_t e_stride = by_band ? 1 : plan.fwd.max_bands;
+  const int64_t k_stride = by_band ? n : 1;
   hipLaunchKernelGGL(adjoint_event_kernel<1>, dim3(blocks), dim3(256), 0,
                      stream, plan.records, plan.moment.counts, n, plan.fwd.H,
-                     plan_bands(plan), wk.moments, w1, nullptr, val, gz, gd);
+                     e_stride, k_stride, wk.moments, w1, nullptr, val, gz, gd);
   BAND_TRY(hipGetLastError());
   if (reduce_sum(wk, val, n, 0, stream, err) ||
       reduce_sum(wk, gz, n, 1, stream, err) ||
@@ -573,9 +579,12 @@ int band_mlem_adjoint_step(BandPlan& plan, const DeviceGeometry& g,
   if (n > 0) {
     if (launch_moments<2>(plan, g, wk, rhoT_k, hT, stream, err)) return -1;
     const unsigned blocks = (unsigned)((n + 255) / 256);
+    const bool by_band = plan.moment.ready;  // layout of the band moments
+    const int64_t e_stride = by_band ? 1 : plan.fwd.max_bands;
+    const int64_t k_stride = by_band ? n : 1;
     hipLaunchKernelGGL(adjoint_event_kernel<2>, dim3(blocks), dim3(256), 0,
                        stream, plan.records, plan.moment.counts, n, plan.fwd.H,
-                       plan_bands(plan), wk.moments, w1, w2, nullptr, gz,
+                       e_stride, k_stride, wk.moments, w1, w2, nullptr, gz,
                        gd);
     BAND_TRY(hipGetLastError());
     if (reduce_sum(wk, gz, n, 0, stream, err) ||

@@ -69,29 +69,38 @@ struct HalfCell {
   __device__ static constexpr int cell_words() { return 2 * R * W; }
 };
 
-// The line of a bin on one row of its band and its column, evaluated alike in
-// every kernel (contraction off): runs are stored relative to `column`.
+// A bin's line: z = xc at the band's middle row, slope tc.  Bins count
+// band-major, then the vertex, then tan.
+struct BinLine {
+  float xc, tc;
+  int band;
+};
+
+__device__ inline BinLine bin_line(const MomentInstance& d, int bin) {
+#pragma clang fp contract(off)
+  const int jt = bin % d.nt, rest = bin / d.nt;
+  BinLine l;
+  l.xc = d.x_lo + ((float)(rest % d.nx) + 0.5f) * d.dx;
+  l.tc = d.t_lo + ((float)jt + 0.5f) * d.dt;
+  l.band = rest / d.nx;
+  return l;
+}
+
+// The line on one row of its band and its column, evaluated alike in every
+// kernel (contraction off): runs are stored relative to `column`.
 struct LineRow {
   float x;     // z coordinate
   int column;  // nearest column, inside the columns a clamped bbox can hold
 };
 
-__device__ inline LineRow line_row(const MomentInstance& d, int bin, int row) {
+__device__ inline LineRow line_row(const DeviceGeometry& g, float xc, float tc,
+                                   int row) {
 #pragma clang fp contract(off)
-  const int jt = bin % d.nt, rest = bin / d.nt;
-  const int ix = rest % d.nx, band = rest / d.nx;
-  const float xc = d.x_lo + ((float)ix + 0.5f) * d.dx;
-  const float tc = d.t_lo + ((float)jt + 0.5f) * d.dt;
   LineRow l;
-  l.x = xc - tc * (((float)row - 0.5f * (R - 1)) * d.g.pixel_height);
-  const float col = rintf((l.x - d.g.tl_z_half_w) * d.g.inv_pixel_width);
-  l.column = (int)fminf(fmaxf(col, 0.0f), (float)max(d.g.n_z - 2, 0));
-  (void)band;
+  l.x = xc - tc * (((float)row - 0.5f * (R - 1)) * g.pixel_height);
+  const float col = rintf((l.x - g.tl_z_half_w) * g.inv_pixel_width);
+  l.column = (int)fminf(fmaxf(col, 0.0f), (float)max(g.n_z - 2, 0));
   return l;
-}
-
-__device__ inline int bin_band(const MomentInstance& d, int bin) {
-  return bin / (d.nt * d.nx);
 }
 
 // lane i of each row of 16 lanes, in all of them (a DPP operand)
@@ -104,6 +113,13 @@ __device__ inline float row_lane(float v) {
 template <int I>
 __device__ inline int row_lane(uint32_t v) {
   return __builtin_amdgcn_mov_dpp((int)v, 0x150 + I, 0xF, 0xF, true);
+}
+
+// Has a value computed before what follows in program order (an empty
+// statement that claims to change it).
+template <typename T>
+__device__ inline void computed(T& v) {
+  asm volatile("" : "+v"(v));
 }
 
 // Keeps LDS accesses of one wavefront in program order across lanes: the
@@ -181,17 +197,24 @@ __device__ inline int tan_bin(const MomentInstance& d, float t) {
   return (int)fminf(fmaxf(j, 0.0f), (float)(d.nt - 1));
 }
 
-// event order: tan bin, then the band of the bbox top, then the bbox's
-// column, so the pairs of a bin come from a few runs of neighbouring records
+// event order: eighths of a tan bin, then the band of the bbox top, then the
+// vertex line's crossing of the axis y = 0: the pairs of a bin then come from
+// short runs of nearly consecutive records, so that the wavefronts' accesses to
+// the per-record arrays (partial sums, weights) share cache lines.  (With
+// whole tan bins and the bbox column instead, neighbouring pairs of a bin lay
+// 17 records apart, and their partial sums cost half the forward pass.)
 __global__ __launch_bounds__(256) void moment_order_kernel(
     MomentInstance d, const uint2* __restrict__ box,
     const float4* __restrict__ a, int64_t n, uint32_t* __restrict__ keys,
     int* __restrict__ values) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n) return;
-  const uint2 b = box[e];
-  keys[e] = ((uint32_t)min(tan_bin(d, a[e].z), 63) << 26) |
-            (((b.y & 0xffff) / R) << 15) | (b.x & 0x7fff);
+  const float4 ev = a[e];  // z, y, tan
+  const float t = floorf((ev.z - d.t_lo) * (8.0f / d.dt));
+  const float x = (ev.x - ev.z * ev.y - d.x_lo) / ((float)d.nx * d.dx);
+  keys[e] = ((uint32_t)fminf(fmaxf(t, 0.0f), 511.0f) << 23) |
+            (((box[e].y & 0xffff) / R) << 12) |
+            (uint32_t)(fminf(fmaxf(x, 0.0f), 1.0f) * 4095.0f);
   values[e] = (int)e;
 }
 
@@ -275,19 +298,27 @@ __global__ __launch_bounds__(256) void moment_group_emit_kernel(
 
 // tasks of a bin: its groups in nearly equal parts of at most `chunk` pairs
 __global__ __launch_bounds__(256) void moment_task_emit_kernel(
-    const int* __restrict__ first, const int* __restrict__ end, int n_bins,
+    MomentInstance d, const int* __restrict__ first, const int* __restrict__ end, int n_bins,
     int chunk, const int* __restrict__ group_of,
-    const int* __restrict__ offsets, int4* __restrict__ tasks) {
+    const int* __restrict__ offsets, MomentTask* __restrict__ tasks) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_bins) return;
   const int total = end[i] - first[i];
   const int groups = (total + kGroup - 1) / kGroup;
   const int parts = (total + chunk - 1) / chunk;
+  const BinLine line = bin_line(d, i);
   for (int k = 0; k < parts; ++k) {
     const int lo = (int)((int64_t)groups * k / parts);
     const int hi = (int)((int64_t)groups * (k + 1) / parts);
-    tasks[offsets[i] + k] = make_int4(
-        i, group_of[i] + lo, min(total, hi * kGroup) - lo * kGroup, 0);
+    MomentTask t;
+    t.xc = line.xc;
+    t.tc = line.tc;
+    t.band = line.band;
+    t.instance = 0;
+    t.group = group_of[i] + lo;
+    t.pairs = min(total, hi * kGroup) - lo * kGroup;
+    t.pad[0] = t.pad[1] = 0;
+    tasks[offsets[i] + k] = t;
   }
 }
 
@@ -303,50 +334,55 @@ __global__ __launch_bounds__(256) void moment_task_emit_kernel(
 //     the line's column, 0x8000 | n << 8 | (offset + positions / 2), n
 //     columns, the first at the line's column + offset (both parts at most
 //     `positions`, so that either form addresses cells that exist).
-// Missing pairs of a last group are zero.
+// Missing pairs of a last group repeat the bin's last pair with empty runs and
+// the index of a spare partial sum, so a wavefront need not tell them apart.
 __global__ __launch_bounds__(256) void moment_pack_kernel(
     MomentInstance d, const BandRecord* __restrict__ rec,
     const int2* __restrict__ groups, const int* __restrict__ end,
-    const int* __restrict__ values, int n_groups,
+    const int* __restrict__ values, int n_groups, int n_records, int spare,
     uint4* __restrict__ blocks, int* __restrict__ status) {
   __shared__ uint32_t words[kGroup * 16];
   const int pair = threadIdx.x >> 4, row = threadIdx.x & 15;
   const int step = pair >> 2, grp = pair & 3;
   for (int k = blockIdx.x; k < n_groups; k += gridDim.x) {
-    const int bin = groups[k].x, p = groups[k].y + pair;
+    const int bin = groups[k].x;
+    const int p = min(groups[k].y + pair, end[bin] - 1);
+    const bool missing = p != groups[k].y + pair;
     uint32_t word = 0, field = 0;
-    if (p < end[bin]) {
-      const int e = values[p];
-      const BandRecord r = rec[e];
-      int x0, x1, y0, y1;
-      record_box(r, x0, x1, y0, y1);
-      const int band = bin_band(d, bin);
-      const LineRow l = line_row(d, bin, row);
-      const RowSpan s = row_span(d.g, r.cz, r.cy, r.A, r.B, r.P, r.Q0, x0, x1,
-                                 y0, y1, band * R + row);
-      if (s.n > 0) {
-        const int a = l.column - s.lo, b = s.lo + s.n - l.column;
-        const int off = s.lo - l.column + d.positions / 2;
-        if (a >= 0 && b >= 0 && a <= d.positions && b <= d.positions)
-          word = (uint32_t)(a | (b << 8));
-        else if (s.n <= d.positions && off >= 0 && off <= d.positions)
-          word = 0x8000u | ((uint32_t)s.n << 8) | (uint32_t)off;
-        else
-          *status = 1;  // does not fit: the host falls back
-      }
-      const float t = -r.B * d.g.inv_2c;
-      const float ad = 4.0f * d.g.inv_pow_sigma_dl * __builtin_fmaf(t, t, 1.0f);
-      switch (row) {
-        case 0: field = __builtin_bit_cast(uint32_t, r.cz); break;
-        case 1: field = __builtin_bit_cast(uint32_t, r.cy); break;
-        case 2: field = __builtin_bit_cast(uint32_t, t); break;
-        case 3: field = __builtin_bit_cast(uint32_t, ad * kExp2Scale); break;
-        case 4: field = __builtin_bit_cast(uint32_t, r.P); break;
-        case 5: field = __builtin_bit_cast(uint32_t, r.Q0); break;
-        case 6: field = (uint32_t)e; break;
-        case 7: field = (uint32_t)(e * d.max_bands + (band - y0 / R)); break;
-        default: break;
-      }
+    const int e = values[p];
+    const BandRecord r = rec[e];
+    int x0, x1, y0, y1;
+    record_box(r, x0, x1, y0, y1);
+    const BinLine line = bin_line(d, bin);
+    const int band = line.band;
+    const LineRow l = line_row(d.g, line.xc, line.tc, row);
+    const RowSpan s = row_span(d.g, r.cz, r.cy, r.A, r.B, r.P, r.Q0, x0, x1,
+                               y0, y1, band * R + row);
+    if (s.n > 0 && !missing) {
+      const int a = l.column - s.lo, b = s.lo + s.n - l.column;
+      const int off = s.lo - l.column + d.positions / 2;
+      if (a >= 0 && b >= 0 && a <= d.positions && b <= d.positions)
+        word = (uint32_t)(a | (b << 8));
+      else if (s.n <= d.positions && off >= 0 && off <= d.positions)
+        word = 0x8000u | ((uint32_t)s.n << 8) | (uint32_t)off;
+      else
+        *status = 1;  // does not fit: the host falls back
+    }
+    const float t = -r.B * d.g.inv_2c;
+    const float ad = 4.0f * d.g.inv_pow_sigma_dl * __builtin_fmaf(t, t, 1.0f);
+    switch (row) {
+      case 0: field = __builtin_bit_cast(uint32_t, r.cz); break;
+      case 1: field = __builtin_bit_cast(uint32_t, r.cy); break;
+      case 2: field = __builtin_bit_cast(uint32_t, t); break;
+      case 3: field = __builtin_bit_cast(uint32_t, ad * kExp2Scale); break;
+      case 4: field = __builtin_bit_cast(uint32_t, r.P); break;
+      case 5: field = __builtin_bit_cast(uint32_t, r.Q0); break;
+      case 6: field = (uint32_t)e; break;
+      case 7:
+        field = (uint32_t)(missing ? spare
+                                   : (band - y0 / R) * n_records + e);
+        break;
+      default: break;
     }
     __syncthreads();  // the previous group has been written out
     if (row < 8)
@@ -392,37 +428,48 @@ __device__ inline RowTerms row_terms(const uint4v& v, float y, float y2,
   return r;
 }
 
+// Whether a lane's row of the group's four pairs has a run that misses the
+// line's column.
+__device__ inline bool any_direct(const uint4v& v) {
+  return ((v.z | v.w) & 0x80008000u) != 0;
+}
+
+// Whether any lane of the wavefront has it: the row terms read their fields
+// from other lanes, so branches around them are taken by whole wavefronts.
+__device__ inline bool wave_any(bool v) {
+  return __builtin_amdgcn_ballot_w64(v) != 0;
+}
+
 // Forward projection of one task: the workgroup tabulates the image around
 // the bin's line, then every wavefront step takes four pairs, 16 lanes each.
 // Bound by VALU issue (58 instructions per step of 64 rows, whatever the runs'
-// lengths; 0.64 per CU-cycle) and the waits around it.  2e7 events, 1000 x 400
-// at 1 mm: 6.4 ms, against 12.4 ms for the kernel that walks the runs' pixels
-// (33 columns per row, 6.9 lane operations each).
+// lengths).  2e7 events, 1000 x 400 at 1 mm: 3.6 ms (6.4 ms while neighbouring
+// pairs' partial sums shared no cache lines), against 12.4 ms for the kernel that
+// walks the runs' pixels (33 columns per row, 6.9 lane operations each).
 template <int NM, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void moment_forward_kernel(
-    const MomentInstance* __restrict__ desc, const int4* __restrict__ tasks) {
+    const MomentInstance* __restrict__ desc, const MomentTask* __restrict__ tasks) {
   using Half = HalfCell<NM>;
   constexpr int W = Half::W, HALF = Half::half_words(),
                 CELL = Half::cell_words();
   extern __shared__ float4v table4[];
   float* const table = reinterpret_cast<float*>(table4);
-  const int4 task = tasks[blockIdx.x];
-  const MomentInstance& d = desc[task.w];
+  const MomentTask task = tasks[blockIdx.x];
+  const MomentInstance& d = desc[task.instance];
   const int lane = threadIdx.x & 63;
   const int row = lane & (R - 1);
   const int grp = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int bin = task.x;
   const int P = d.positions;
   const int n_y = d.g.n_y, n_z = d.g.n_z;
   const float w_px = d.g.pixel_width;
-  const int iy = bin_band(d, bin) * R + row;
-  const LineRow l = line_row(d, bin, row);
+  const int iy = task.band * R + row;
+  const LineRow l = line_row(d.g, task.xc, task.tc, row);
   const float qc = d.g.C * kExp2Scale;
   const float* __restrict__ rhoT = d.rhoT;
-  const int n_here = task.z;
+  const int n_here = task.pairs;
   const uint4v* __restrict__ base =
-      reinterpret_cast<const uint4v*>(d.blocks) + (int64_t)task.y * 64;
+      reinterpret_cast<const uint4v*>(d.blocks) + (int64_t)task.group * 64;
   const int last = (n_here - 1) / kGroup;
   uint4v next = gload(base + min(wave, last) * 64 + lane);
   {
@@ -490,7 +537,7 @@ __global__ __launch_bounds__(64 * WAVES) void moment_forward_kernel(
   float* __restrict__ partial = d.partial;
   const float* const left = table + row * W;
   const float* const right = left + (P + 1) * CELL;
-  auto step = [&](auto tag, const uint4v& v, int j) {
+  auto row_sum = [&](auto tag, const uint4v& v) {
     constexpr int S = decltype(tag)::value;
     const RowTerms r = row_terms<S>(v, y, y2, l.x, qc);
     const float eta = cs * r.delta;
@@ -506,42 +553,70 @@ __global__ __launch_bounds__(64 * WAVES) void moment_forward_kernel(
 #pragma unroll
     for (int i = W - 1; i >= 0; --i)
       t = __builtin_fmaf(t, eta, l0.w[i] + r0.w[i]);
-    float s = t * r.w;
-    // runs that miss the line's column, and rows whose sum is not finite (an
-    // infinite pixel times powers of both signs), pixel by pixel
-    const bool direct = r.run >= 0x8000u;
-    if (direct || !(__builtin_fabsf(s) < __builtin_inff())) {
-      const int n = direct ? b : a + b;
-      const int col = l.column + (direct ? a - P / 2 : -a);
-      float dz = (__builtin_fmaf((float)col, w_px, d.g.tl_z_half_w) - l.x) -
-                 r.delta;
-      float acc = 0.0f;
-      const float* src = rhoT + (int64_t)col * n_y + iy;
-      for (int k = 0; k < n; ++k) {
-        acc = __builtin_fmaf(
-            __builtin_amdgcn_exp2f(__builtin_fmaf(qc * dz, dz, r.qa)),
-            gload(src), acc);
-        src += n_y;
-        dz += w_px;
-      }
-      s = n > 0 ? r.pre * acc : 0.0f;
-    }
-    s = group_total<R>(s);
-    // the lane that holds the partial's index stores it
-    if (row == 7 + 8 * (S & 1) && j + 4 * S + grp < n_here)
-      gstore(partial + (int)(S < 2 ? v.x : v.y), s);
+    return t * r.w;
   };
+  // a run pixel by pixel
+  auto walk = [&](auto tag, const uint4v& v, float s) {
+    constexpr int S = decltype(tag)::value;
+    const RowTerms r = row_terms<S>(v, y, y2, l.x, qc);
+    const bool direct = r.run >= 0x8000u;
+    if (!direct && __builtin_fabsf(s) < __builtin_inff()) return s;
+    const int a = (int)(r.run & 0xff), b = (int)((r.run >> 8) & 0x7f);
+    const int n = direct ? b : a + b;
+    const int col = l.column + (direct ? a - P / 2 : -a);
+    float dz = (__builtin_fmaf((float)col, w_px, d.g.tl_z_half_w) - l.x) -
+               r.delta;
+    float acc = 0.0f;
+    const float* src = rhoT + (int64_t)col * n_y + iy;
+    for (int k = 0; k < n; ++k) {
+      acc = __builtin_fmaf(
+          __builtin_amdgcn_exp2f(__builtin_fmaf(qc * dz, dz, r.qa)),
+          gload(src), acc);
+      src += n_y;
+      dz += w_px;
+    }
+    return n > 0 ? r.pre * acc : 0.0f;
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  using S2 = std::integral_constant<int, 2>;
+  using S3 = std::integral_constant<int, 3>;
   for (int k = wave; k <= last; k += WAVES) {
     const uint4v cur = next;
     next = gload(base + min(k + WAVES, last) * 64 + lane);
-    const int j = k * kGroup;
-    step(std::integral_constant<int, 0>{}, cur, j);
-    if (j + 4 >= n_here) break;
-    step(std::integral_constant<int, 1>{}, cur, j);
-    if (j + 8 >= n_here) break;
-    step(std::integral_constant<int, 2>{}, cur, j);
-    if (j + 12 >= n_here) break;
-    step(std::integral_constant<int, 3>{}, cur, j);
+    // a group's four steps at once; a last group's empty steps are left out
+    const int steps = min((n_here - k * kGroup + 3) / 4, 4);
+    float s0 = row_sum(S0{}, cur), s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+    if (steps == 4) {
+      s1 = row_sum(S1{}, cur);
+      s2 = row_sum(S2{}, cur);
+      s3 = row_sum(S3{}, cur);
+    } else {
+      if (steps > 1) s1 = row_sum(S1{}, cur);
+      if (steps > 2) s2 = row_sum(S2{}, cur);
+    }
+    // runs that miss the line's column, and rows whose sum is not finite (an
+    // infinite pixel times powers of both signs)
+    if (wave_any(any_direct(cur) ||
+                 !(__builtin_fabsf(s0) + __builtin_fabsf(s1) +
+                       __builtin_fabsf(s2) + __builtin_fabsf(s3) <
+                   __builtin_inff()))) {
+      s0 = walk(S0{}, cur, s0);
+      s1 = walk(S1{}, cur, s1);
+      s2 = walk(S2{}, cur, s2);
+      s3 = walk(S3{}, cur, s3);
+    }
+    s0 = group_total<R>(s0);
+    s1 = group_total<R>(s1);
+    s2 = group_total<R>(s2);
+    s3 = group_total<R>(s3);
+    // the next group is waited for here, not behind this group's stores
+    computed(next);
+    // lanes 7 and 15 of a row hold the partials' indices
+    if ((row & 7) == 7) {
+      gstore(partial + (int)cur.x, row == 7 ? s0 : s1);
+      gstore(partial + (int)cur.y, row == 7 ? s2 : s3);
+    }
   }
 }
 
@@ -565,28 +640,27 @@ __device__ inline int grad_word(int m, int row) {
 
 template <int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void moment_gradient_kernel(
-    const MomentInstance* __restrict__ desc, const int4* __restrict__ tasks,
+    const MomentInstance* __restrict__ desc, const MomentTask* __restrict__ tasks,
     const float* __restrict__ xT, int stride, float* __restrict__ out) {
   extern __shared__ float4v table4[];
   float* const table = reinterpret_cast<float*>(table4);
-  const int4 task = tasks[blockIdx.x];
-  const MomentInstance& d = desc[task.w];
+  const MomentTask task = tasks[blockIdx.x];
+  const MomentInstance& d = desc[task.instance];
   const int lane = threadIdx.x & 63;
   const int row = lane & (R - 1);
   const int grp = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int bin = task.x;
   const int P = d.positions;
   const int n_y = d.g.n_y, n_z = d.g.n_z;
   const float w_px = d.g.pixel_width;
-  const int iy = bin_band(d, bin) * R + row;
-  const LineRow l = line_row(d, bin, row);
+  const int iy = task.band * R + row;
+  const LineRow l = line_row(d.g, task.xc, task.tc, row);
   const float C = d.g.C;
   const float qc = C * kExp2Scale;
   const float inv_s = d.inv_s;
-  const int n_here = task.z;
+  const int n_here = task.pairs;
   const uint4v* __restrict__ base =
-      reinterpret_cast<const uint4v*>(d.blocks) + (int64_t)task.y * 64;
+      reinterpret_cast<const uint4v*>(d.blocks) + (int64_t)task.group * 64;
   const int last = (n_here - 1) / kGroup;
   uint4v next = gload(base + min(wave, last) * 64 + lane);
   {
@@ -639,7 +713,10 @@ __global__ __launch_bounds__(64 * WAVES) void moment_gradient_kernel(
       __builtin_fmaf(y2, 1.0f / (d.g.radius * d.g.radius), 1.0f);
   const float* const left = table + grad_word(0, row);
   const int right_words = (P + 1) * kGradCell;
-  auto step = [&](auto tag, const uint4v& v, int j) {
+  struct Sums {
+    float m[3];
+  };
+  auto step = [&](auto tag, const uint4v& v) {
     constexpr int S = decltype(tag)::value;
     const RowTerms r = row_terms<S>(v, y, y2, l.x, qc);
     const float eta = cs * r.delta;
@@ -695,40 +772,51 @@ __global__ __launch_bounds__(64 * WAVES) void moment_gradient_kernel(
     // w = Q0' (1 + y^2 / R^2) pre^2
     const float f = __builtin_bit_cast(float, S < 2 ? v.x : v.y);
     const float w = row_lane<8 * (S & 1) + 5>(f) * w_row * r.pre * r.pre;
-    const float m0 = group_total<R>(k0);
-    const float m1 = group_total<R>(__builtin_fmaf(k0, qd, kq));
-    const float m2 = group_total<R>(k0 * (w - qd));
-    if (row == 7 + 8 * (S & 1) && j + 4 * S + grp < n_here) {
-      float* o = out + (int64_t)(int)(S < 2 ? v.x : v.y) * stride;
-      gstore(o, m0);
-      gstore(o + 1, m1);
-      gstore(o + 2, m2);
-    }
+    Sums o;
+    o.m[0] = group_total<R>(k0);
+    o.m[1] = group_total<R>(__builtin_fmaf(k0, qd, kq));
+    o.m[2] = group_total<R>(k0 * (w - qd));
+    return o;
   };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  using S2 = std::integral_constant<int, 2>;
+  using S3 = std::integral_constant<int, 3>;
   for (int k = wave; k <= last; k += WAVES) {
     const uint4v cur = next;
     next = gload(base + min(k + WAVES, last) * 64 + lane);
-    const int j = k * kGroup;
-    step(std::integral_constant<int, 0>{}, cur, j);
-    if (j + 4 >= n_here) break;
-    step(std::integral_constant<int, 1>{}, cur, j);
-    if (j + 8 >= n_here) break;
-    step(std::integral_constant<int, 2>{}, cur, j);
-    if (j + 12 >= n_here) break;
-    step(std::integral_constant<int, 3>{}, cur, j);
+    // (a last group's empty steps are left out)
+    const int steps = min((n_here - k * kGroup + 3) / 4, 4);
+    Sums s[4] = {};
+    s[0] = step(S0{}, cur);
+    if (steps > 1) s[1] = step(S1{}, cur);
+    if (steps > 2) s[2] = step(S2{}, cur);
+    if (steps > 3) s[3] = step(S3{}, cur);
+    // the next group is waited for here, not behind this group's stores
+    computed(next);
+    // lanes 7 and 15 of a row hold the partials' indices
+    if ((row & 7) == 7) {
+      float* const o01 = out + (int64_t)(int)cur.x * stride;
+      float* const o23 = out + (int64_t)(int)cur.y * stride;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        gstore(o01 + i, row == 7 ? s[0].m[i] : s[1].m[i]);
+        gstore(o23 + i, row == 7 ? s[2].m[i] : s[3].m[i]);
+      }
+    }
   }
 }
 
 // D_e = sum of the record's partials; inv_e = 1 / D_e (guarded or not)
 __global__ __launch_bounds__(256) void moment_inverse_kernel(
-    const int* __restrict__ counts, int64_t n, int max_bands,
+    const int* __restrict__ counts, int64_t n,
     const float* __restrict__ partial, int guard, float* __restrict__ inv,
     float* __restrict__ denominators) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n) return;
   float s = 0.0f;
   const int c = counts[e];
-  for (int k = 0; k < c; ++k) s += partial[e * max_bands + k];
+  for (int k = 0; k < c; ++k) s += partial[k * n + e];
   if (denominators) denominators[e] = s;
   if (inv) inv[e] = guard ? ((s > 0.0f) ? 1.0f / s : 0.0f) : 1.0f / s;
 }
@@ -745,24 +833,23 @@ __global__ __launch_bounds__(256) void moment_inverse_kernel(
 // 22.0 ms for the kernel that adds pixel by pixel (an LDS read and write each).
 template <int NM>
 __global__ __launch_bounds__(64) void moment_backward_kernel(
-    const MomentInstance* __restrict__ desc, const int4* __restrict__ tasks,
+    const MomentInstance* __restrict__ desc, const MomentTask* __restrict__ tasks,
     const float* __restrict__ weights_of, float* __restrict__ into) {
   using Half = HalfCell<NM>;
   constexpr int W = Half::W, HALF = Half::half_words(),
                 CELL = Half::cell_words();
   extern __shared__ float4v cells4[];
-  const int4 task = tasks[blockIdx.x];
-  const MomentInstance& d = desc[task.w];
+  const MomentTask task = tasks[blockIdx.x];
+  const MomentInstance& d = desc[task.instance];
   const int lane = threadIdx.x;
   const int row = lane & (R - 1);
   const int grp = lane >> 4;
-  const int bin = task.x;
   const int P = d.positions;
   const int n_y = d.g.n_y, n_z = d.g.n_z;
   const float w_px = d.g.pixel_width;
-  const int y_base = bin_band(d, bin) * R;
+  const int y_base = task.band * R;
   const int iy = y_base + row;
-  const LineRow l = line_row(d, bin, row);
+  const LineRow l = line_row(d.g, task.xc, task.tc, row);
   const float qc = d.g.C * kExp2Scale;
   const float cs = d.cs;
   const float y = pixel_center_y(d.g, iy);
@@ -772,9 +859,9 @@ __global__ __launch_bounds__(64) void moment_backward_kernel(
   const int side_words = (P + 1) * CELL;
   for (int i = lane; i < side_words / 2; i += 64)
     cells4[i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
-  const int n_here = task.z;
+  const int n_here = task.pairs;
   const uint4v* __restrict__ base =
-      reinterpret_cast<const uint4v*>(d.blocks) + (int64_t)task.y * 64;
+      reinterpret_cast<const uint4v*>(d.blocks) + (int64_t)task.group * 64;
   const int last = (n_here - 1) / kGroup;
   float* const mine = reinterpret_cast<float*>(cells4) + row * W;
   const bool odd = grp & 1, high = grp & 2;
@@ -793,91 +880,153 @@ __global__ __launch_bounds__(64) void moment_backward_kernel(
     return w;
   };
   struct Terms {
-    RowTerms r;
     Half v0, v1;  // the moments of this lane's first and second half
-    float weight;
-    int a, b;
+    float* p0;    // the cells its run ends in, this lane's first side first
+    float* p1;
   };
-  auto terms = [&](auto tag, const uint4v& v, const Weights& wt, int j) {
+  auto terms = [&](auto tag, const uint4v& v, const Weights& wt) {
     constexpr int S = decltype(tag)::value;
-    Terms t;
-    t.r = row_terms<S>(v, y, y2, l.x, qc);
-    const float eta = cs * t.r.delta;
-    t.weight = row_lane<6 + 8 * (S & 1)>(S < 2 ? wt.w01 : wt.w23);
-    if (j + 4 * S + grp >= n_here) t.weight = 0.0f;
-    const float f = t.r.run >= 0x8000u ? 0.0f : t.r.w * t.weight;
+    const RowTerms r = row_terms<S>(v, y, y2, l.x, qc);
+    const float eta = cs * r.delta;
     float m[NM];
-    m[0] = f;
+    m[0] = r.w * row_lane<6 + 8 * (S & 1)>(S < 2 ? wt.w01 : wt.w23);
+    // (a run that misses the line's column adds nothing here)
+    if (r.run >= 0x8000u) m[0] = 0.0f;
 #pragma unroll
     for (int i = 1; i < NM; ++i) m[i] = m[i - 1] * eta;
+    Terms t;
 #pragma unroll
     for (int i = 0; i < W; ++i) {
       t.v0.w[i] = high ? m[W + i] : m[i];
       t.v1.w[i] = high ? m[i] : m[W + i];
     }
-    t.a = (int)(t.r.run & 0xff) * CELL;
-    t.b = (int)((t.r.run >> 8) & 0x7f) * CELL + side_words;
+    const int a = (int)(r.run & 0xff) * CELL;
+    const int b = (int)((r.run >> 8) & 0x7f) * CELL + side_words;
+    t.p0 = mine + (odd ? b : a);
+    t.p1 = mine + (odd ? a : b);
     return t;
   };
-  auto add = [&](const Terms& t) {
-    float* const p0 = mine + (odd ? t.b : t.a);
-    float* const p1 = mine + (odd ? t.a : t.b);
-    auto round = [](float* p, const Half& v) {
-      Half x = Half::load(p);
+  auto add_to = [](float* p, Half x, const Half& v) {
 #pragma unroll
-      for (int i = 0; i < W; ++i) x.w[i] += v.w[i];
-      x.store(p);
-      lds_order();
-    };
-    round(p0 + h0, t.v0);
-    round(p1 + h0, t.v0);
-    round(p0 + h1, t.v1);
-    round(p1 + h1, t.v1);
-    if (t.r.run >= 0x8000u && t.weight != 0.0f) {
-      const int n = (int)((t.r.run >> 8) & 0x7f);
-      const int col = l.column + (int)(t.r.run & 0xff) - P / 2;
-      float dz = (__builtin_fmaf((float)col, w_px, d.g.tl_z_half_w) - l.x) -
-                 t.r.delta;
-      float* dst = bpT + (int64_t)col * n_y + iy;
-      const float f = t.r.pre * t.weight;
-      for (int k = 0; k < n; ++k) {
-        gatomic_add(dst, f * __builtin_amdgcn_exp2f(
-                                 __builtin_fmaf(qc * dz, dz, t.r.qa)));
-        dst += n_y;
-        dz += w_px;
-      }
+    for (int i = 0; i < W; ++i) x.w[i] += v.w[i];
+    x.store(p);
+    lds_order();
+  };
+  auto add = [&](const Terms& t) {
+    add_to(t.p0 + h0, Half::load(t.p0 + h0), t.v0);
+    add_to(t.p1 + h0, Half::load(t.p1 + h0), t.v0);
+    add_to(t.p0 + h1, Half::load(t.p0 + h1), t.v1);
+    add_to(t.p1 + h1, Half::load(t.p1 + h1), t.v1);
+  };
+  // add(t), and the terms of step S of v a quarter at a time between each LDS
+  // read and its write: the arithmetic hides the reads' latency (the scheduler
+  // barriers keep it there)
+  auto add_and_form = [&](auto tag, const Terms& t, const uint4v& v,
+                          const Weights& wt) {
+    constexpr int S = decltype(tag)::value;
+    constexpr int F = 8 * (S & 1);
+    Half x = Half::load(t.p0 + h0);
+    __builtin_amdgcn_sched_barrier(0);
+    RowTerms r = row_terms<S>(v, y, y2, l.x, qc);
+    computed(r.delta);
+    computed(r.w);
+    __builtin_amdgcn_sched_barrier(0);
+    add_to(t.p0 + h0, x, t.v0);
+    x = Half::load(t.p1 + h0);
+    __builtin_amdgcn_sched_barrier(0);
+    const float eta = cs * r.delta;
+    float m[NM];
+    m[0] = r.w * row_lane<6 + F>(S < 2 ? wt.w01 : wt.w23);
+    if (r.run >= 0x8000u) m[0] = 0.0f;
+#pragma unroll
+    for (int i = 1; i < NM; ++i) m[i] = m[i - 1] * eta;
+#pragma unroll
+    for (int i = 0; i < NM; ++i) computed(m[i]);
+    __builtin_amdgcn_sched_barrier(0);
+    add_to(t.p1 + h0, x, t.v0);
+    x = Half::load(t.p0 + h1);
+    __builtin_amdgcn_sched_barrier(0);
+    Terms u;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      u.v0.w[i] = high ? m[W + i] : m[i];
+      u.v1.w[i] = high ? m[i] : m[W + i];
+      computed(u.v0.w[i]);
+      computed(u.v1.w[i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    add_to(t.p0 + h1, x, t.v1);
+    x = Half::load(t.p1 + h1);
+    __builtin_amdgcn_sched_barrier(0);
+    const int a = (int)(r.run & 0xff) * CELL;
+    const int b = (int)((r.run >> 8) & 0x7f) * CELL + side_words;
+    int first = odd ? b : a, second = odd ? a : b;
+    computed(first);
+    computed(second);
+    u.p0 = mine + first;
+    u.p1 = mine + second;
+    __builtin_amdgcn_sched_barrier(0);
+    add_to(t.p1 + h1, x, t.v1);
+    return u;
+  };
+  // a run that misses the line's column, pixel by pixel
+  auto walk = [&](auto tag, const uint4v& v, const Weights& wt) {
+    constexpr int S = decltype(tag)::value;
+    const RowTerms r = row_terms<S>(v, y, y2, l.x, qc);
+    const float weight = row_lane<6 + 8 * (S & 1)>(S < 2 ? wt.w01 : wt.w23);
+    if (r.run < 0x8000u || weight == 0.0f) return;
+    const int n = (int)((r.run >> 8) & 0x7f);
+    const int col = l.column + (int)(r.run & 0xff) - P / 2;
+    float dz = (__builtin_fmaf((float)col, w_px, d.g.tl_z_half_w) - l.x) -
+               r.delta;
+    float* dst = bpT + (int64_t)col * n_y + iy;
+    const float f = r.pre * weight;
+    for (int k = 0; k < n; ++k) {
+      gatomic_add(dst, f * __builtin_amdgcn_exp2f(
+                               __builtin_fmaf(qc * dz, dz, r.qa)));
+      dst += n_y;
+      dz += w_px;
     }
   };
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
   using S2 = std::integral_constant<int, 2>;
   using S3 = std::integral_constant<int, 3>;
-  // groups two ahead, weights one ahead, a step's terms while the step
-  // before it is added
+  // groups two ahead, weights one ahead, and a step's terms formed between the
+  // LDS accesses of the step before it
   uint4v cur = gload(base + lane);
   uint4v next = gload(base + min(1, last) * 64 + lane);
   Weights wt = weights(cur);
   lds_order();
-  Terms t = terms(S0{}, cur, wt, 0);
+  Terms t = terms(S0{}, cur, wt);
   for (int k = 0; k <= last; ++k) {
     const uint4v next2 = gload(base + min(k + 2, last) * 64 + lane);
     const Weights wt_next = weights(next);
-    const int j = k * kGroup;
-    Terms u = terms(S1{}, cur, wt, j);
-    add(t);
-    t = terms(S2{}, cur, wt, j);
-    if (j + 4 < n_here) add(u);
-    u = terms(S3{}, cur, wt, j);
-    if (j + 8 < n_here) add(t);
-    t = terms(S0{}, next, wt_next, j + kGroup);
-    if (j + 12 < n_here) add(u);
+    const int here = n_here - k * kGroup;
+    if (here > 12) {
+      t = add_and_form(S1{}, t, cur, wt);
+      t = add_and_form(S2{}, t, cur, wt);
+      t = add_and_form(S3{}, t, cur, wt);
+      t = add_and_form(S0{}, t, next, wt_next);
+    } else {
+      // a last group's empty steps are left out
+      add(t);
+      if (here > 4) add(terms(S1{}, cur, wt));
+      if (here > 8) add(terms(S2{}, cur, wt));
+    }
+    if (wave_any(any_direct(cur))) {
+      walk(S0{}, cur, wt);
+      walk(S1{}, cur, wt);
+      walk(S2{}, cur, wt);
+      walk(S3{}, cur, wt);
+    }
     cur = next;
     next = next2;
     wt = wt_next;
   }
   lds_order();
-  // inward sums, cell by cell: lane = (row, side, half); the pixel's value
-  // replaces word 0 of its cell
+  // inward sums, cell by cell: lane = (row, side, half).  The half's part of
+  // the pixel's value replaces word 0 of its half cell.
   {
     const int side = grp & 1, half = grp >> 1;
     float* cell = mine + side * side_words + half * HALF;
@@ -886,24 +1035,31 @@ __global__ __launch_bounds__(64) void moment_backward_kernel(
     for (int i = 0; i < W; ++i)
       c[i] = half ? ExpPoly<NM>::c[W + i] : ExpPoly<NM>::c[i];
     const float inv_s = d.inv_s;
-    for (int k = P; k >= 1; --k) {
-      float* at = cell + k * CELL;
-      const Half x = Half::load(at);
+    const int dir = side ? 1 : -1;
+    const int col0 = side ? l.column - 1 : l.column;  // + dir k: cell k
+    // four cells' words are in flight together
+    constexpr int B = 4;
+    for (int k0 = P; k0 >= 1; k0 -= B) {
+      Half x[B];
 #pragma unroll
-      for (int i = 0; i < W; ++i) s[i] += x.w[i];
-      const int col = side ? l.column + k - 1 : l.column - k;
-      const float u =
-          __builtin_fmaf((float)col, w_px, d.g.tl_z_half_w) - l.x;
-      const float v = u * inv_s;
-      float t = s[W - 1] * c[W - 1];
+      for (int i = 0; i < B; ++i)
+        x[i] = Half::load(cell + max(k0 - i, 0) * CELL);
 #pragma unroll
-      for (int i = W - 2; i >= 0; --i) t = __builtin_fmaf(t, v, s[i] * c[i]);
-      if (half) {
-        t *= v * v;
-        t *= W == 4 ? v * v : v;
+      for (int i = 0; i < B; ++i) {
+        const int k = k0 - i;
+#pragma unroll
+        for (int w = 0; w < W; ++w) s[w] += x[i].w[w];
+        const float u = __builtin_fmaf((float)(col0 + dir * k), w_px,
+                                       d.g.tl_z_half_w) - l.x;
+        const float v = u * inv_s;
+        float t = s[W - 1] * c[W - 1];
+#pragma unroll
+        for (int w = W - 2; w >= 0; --w) t = __builtin_fmaf(t, v, s[w] * c[w]);
+        const float v2 = v * v;
+        if (half) t *= v2 * (W == 4 ? v2 : v);
+        // (past the last cell the value lands in the unused cell 0)
+        cell[max(k, 0) * CELL] = t * __builtin_amdgcn_exp2f(qc * u * u);
       }
-      t += __shfl_xor(t, 32);
-      if (!half) *at = t * __builtin_amdgcn_exp2f(qc * u * u);
     }
   }
   lds_order();
@@ -915,13 +1071,23 @@ __global__ __launch_bounds__(64) void moment_backward_kernel(
   }
   x_lo = max(__builtin_amdgcn_readfirstlane(x_lo), 0);
   x_hi = min(__builtin_amdgcn_readfirstlane(x_hi), n_z);
-  for (int x = x_lo + grp; x < x_hi; x += 4) {
-    const int k = x - l.column;
-    const int cell = k >= 0 ? k + 1 : -k;
-    if (cell <= P && iy < n_y) {
-      const float val = mine[(k >= 0 ? side_words : 0) + cell * CELL];
-      if (val != 0.0f) gatomic_add(bpT + (int64_t)x * n_y + iy, val);
+  constexpr int B = 4;
+  for (int x0 = x_lo + grp; x0 < x_hi; x0 += 4 * B) {
+    float val[B];
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+      const int k = x0 + 4 * i - l.column;
+      const int cell = k >= 0 ? k + 1 : -k;
+      const bool in = cell <= P && x0 + 4 * i < x_hi && iy < n_y;
+      const float* at = mine + (k >= 0 ? side_words : 0) +
+                        (in ? cell : 0) * CELL;
+      const float sum = at[0] + at[HALF];
+      val[i] = in ? sum : 0.0f;
     }
+#pragma unroll
+    for (int i = 0; i < B; ++i)
+      if (val[i] != 0.0f)
+        gatomic_add(bpT + (int64_t)(x0 + 4 * i) * n_y + iy, val[i]);
   }
 }
 
@@ -1096,7 +1262,7 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   const size_t w_cub = work.take<char>((int64_t)cub);
   // the plan's per-event memory; its groups and tasks are sized below
   Arena own;
-  const size_t o_partial = own.take<float>(n * d.max_bands);
+  const size_t o_partial = own.take<float>(n * d.max_bands + 1);
   const size_t o_inv = own.take<float>(n);
   const size_t o_counts = own.take<int>(n);
   const size_t o_order = own.take<int>(n);
@@ -1205,29 +1371,30 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   Arena lists;
   const size_t o_blocks = lists.take<uint4>((int64_t)n_groups * 64);
   const size_t o_groups = lists.take<int2>(n_groups);
-  const size_t o_fwd = lists.take<int4>(totals[1]);
-  const size_t o_bwd = lists.take<int4>(totals[2]);
+  const size_t o_fwd = lists.take<MomentTask>(totals[1]);
+  const size_t o_bwd = lists.take<MomentTask>(totals[2]);
   if (hipMalloc(&plan.lists, lists.used) != hipSuccess) {
     plan.lists = nullptr;
     return give_up();
   }
   char* L = static_cast<char*>(plan.lists);
   plan.blocks = reinterpret_cast<uint32_t*>(L + o_blocks);
-  plan.fwd_tasks = reinterpret_cast<int4*>(L + o_fwd);
-  plan.bwd_tasks = reinterpret_cast<int4*>(L + o_bwd);
+  plan.fwd_tasks = reinterpret_cast<MomentTask*>(L + o_fwd);
+  plan.bwd_tasks = reinterpret_cast<MomentTask*>(L + o_bwd);
   int2* groups = reinterpret_cast<int2*>(L + o_groups);
   hipLaunchKernelGGL(moment_group_emit_kernel, dim3(grid_of(n_bins)),
                      dim3(256), 0, stream, first, end, n_bins, pieces[0],
                      groups);
   for (int pass = 0; pass < 2; ++pass)
     hipLaunchKernelGGL(moment_task_emit_kernel, dim3(grid_of(n_bins)),
-                       dim3(256), 0, stream, first, end, n_bins,
+                       dim3(256), 0, stream, d, first, end, n_bins,
                        chunks[1 + pass], pieces[0], pieces[1 + pass],
                        pass ? plan.bwd_tasks : plan.fwd_tasks);
   int* d_status = reinterpret_cast<int*>(d_stats + 1);
   hipLaunchKernelGGL(moment_pack_kernel,
                      dim3((unsigned)std::min(n_groups, 1 << 20)), dim3(256), 0,
                      stream, d, rec, groups, end, vb.Current(), n_groups,
+                     (int)n, (int)(n * d.max_bands),
                      reinterpret_cast<uint4*>(plan.blocks), d_status);
   BAND_TRY(hipGetLastError());
   int status = 0;
@@ -1258,7 +1425,7 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   plan.n_fwd = totals[1];
   plan.n_bwd = totals[2];
   plan.fwd_lds = plan.bwd_lds = table_bytes(d.positions, 8);
-  plan.fwd_waves = n_pairs / std::max(plan.n_fwd, 1) >= 200 ? 4 : 1;
+  plan.fwd_waves = n_pairs / std::max(plan.n_fwd, 1) >= 100 ? 4 : 1;
   for (const void* kern :
        {reinterpret_cast<const void*>(moment_forward_kernel<8, 1>),
         reinterpret_cast<const void*>(moment_forward_kernel<8, 4>),
@@ -1287,7 +1454,7 @@ int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
                    hipStream_t stream, std::string* err) {
   hipLaunchKernelGGL(moment_inverse_kernel, dim3(grid_of(plan.n_events)),
                      dim3(256), 0, stream, plan.counts, plan.n_events,
-                     plan.inst.max_bands, plan.partial, guard, inv,
+                     plan.partial, guard, inv,
                      denominators);
   BAND_TRY(hipGetLastError());
   return 0;

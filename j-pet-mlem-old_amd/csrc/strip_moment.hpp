@@ -50,11 +50,21 @@ struct MomentInstance {
   const uint32_t* blocks;  // 1 KiB per 16 pairs (moment_pack_kernel)
   const float* rhoT;       // image the forward pass reads (column-major)
   float* rho_next;
-  float* partial;          // per (record, band of the record)
+  float* partial;          // per (band of the record, record)
   const int* counts;       // bands of each record
   float* inv;
   float* bpT;
   int64_t n_events;
+};
+
+// One workgroup's (forward) or wavefront's (back-projection) share of a bin.
+struct MomentTask {
+  float xc, tc;  // the bin's line: z at the band's middle row, slope
+  int band;
+  int instance;  // index of its MomentInstance
+  int group;     // first 16-pair group
+  int pairs;
+  int pad[2];
 };
 
 struct MomentPlan {
@@ -73,8 +83,8 @@ struct MomentPlan {
   float* inv = nullptr;
   int* counts = nullptr;
   int* order = nullptr;     // record -> caller's event
-  int4* fwd_tasks = nullptr;  // (bin, first group, pairs, instance)
-  int4* bwd_tasks = nullptr;
+  MomentTask* fwd_tasks = nullptr;
+  MomentTask* bwd_tasks = nullptr;
   MomentInstance* desc = nullptr;  // images 0 / 1
 };
 
@@ -100,7 +110,7 @@ int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
 int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
                     std::string* err, const float* weights = nullptr,
                     float* into = nullptr);
-// out[stride * (record * max_bands + band of the record) + {0, 1, 2}] = sum K x,
+// out[stride * (band of the record * n_events + record) + {0, 1, 2}] = sum K x,
 // sum K x Q, sum K x (w - Qd) of the column-major image xT (strip_adjoint.hip)
 int moment_gradient(MomentPlan& plan, const float* xT, int stride, float* out,
                     hipStream_t stream, std::string* err);
