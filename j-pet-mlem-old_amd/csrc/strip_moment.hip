@@ -20,19 +20,29 @@ namespace {
 constexpr int R = kMomentRows;
 constexpr int kGroup = 16;  // pairs of one 1 KiB group
 
-// exp(v) ~ sum c_m v^m, m < NM, on [-1, 1] with the least largest relative
-// error, 1.9e-7 (a linear program over 2001 Chebyshev points).  The vertex may
-// then lie reach * sigma_z from the line, 2 (3 / sqrt 2 + reach) reach = 1, for
-// |C u delta| <= 1 on every u of a 3-sigma run.
+// exp(v) ~ sum c_m v^m, m < NM, on |v| <= V: 8 terms on V = 1, 6 terms on
+// V = 0.42.  The vertex may then lie reach * sigma_z from the line,
+// 2 (3 / sqrt 2 + reach) reach = V, for |C u delta| <= V on every u of a
+// 3-sigma run.  The relative error is a minimax one (linear programs over 4001
+// Chebyshev points) weighted by the kernel value that v goes with, but by no
+// less than 0.2, with its mean over a run's kernel values and over their
+// products with u^2 held at zero (2e-10 with the rounded coefficients): the
+// sigma derivatives are small differences of such sums.  At most 4.9e-7
+// (6 terms 7.8e-7) at a run's far ends, 1e-7 (2.2e-7) for |v| < 0.3 V.
 template <int NM>
 struct ExpPoly;
 template <>
 struct ExpPoly<8> {
-  static constexpr double reach = 0.2140;
-  static constexpr float c[8] = {
-      0.9999998808238608f,    1.000001053962846f,   0.5000048572256811f,
-      0.16665825143600693f,   0.04163906763089733f, 0.008348694726996652f,
-      0.0014365374436724502f, 0.00019297136769021376f};
+  static constexpr double reach = 0.2141;
+  static constexpr float c[8] = {1.0f,           0.999999762f,   0.500000596f,
+                                 0.166664779f,   0.0416531637f,  0.008342674f,
+                                 0.00142612169f, 0.000193406566f};
+};
+template <>
+struct ExpPoly<6> {
+  static constexpr double reach = 0.0948;
+  static constexpr float c[6] = {1.0f,         1.00000179f,  0.499997377f,
+                                 0.166656896f, 0.0419010967f, 0.00834288821f};
 };
 constexpr double kRunHalf = 2.1213203435596424;  // 3 / sqrt 2, in sigma_z
 
@@ -67,6 +77,12 @@ struct HalfCell {
   }
   __device__ static constexpr int half_words() { return R * W; }
   __device__ static constexpr int cell_words() { return 2 * R * W; }
+  // Words of one side.  Rows of three words (6 terms) touch 16 of the 32
+  // banks; 16 words more put the other side's rows on the other 16, so lane
+  // groups working on opposite sides do not conflict.
+  __device__ static int side_words(int positions) {
+    return (positions + 1) * cell_words() + (W == 3 ? 16 : 0);
+  }
 };
 
 // A bin's line: z = xc at the band's middle row, slope tc.  Bins count
@@ -480,7 +496,7 @@ __global__ __launch_bounds__(64 * WAVES) void moment_forward_kernel(
     const int side = grp & 1;
     const int m0 = (int)(threadIdx.x >> 5) * MG;
     if (m0 < NM) {
-      float* cell = table + (side * (P + 1)) * CELL + (m0 / W) * HALF +
+      float* cell = table + side * Half::side_words(P) + (m0 / W) * HALF +
                     row * W + m0 % W;
       float acc[MG], cm[MG];
 #pragma unroll
@@ -536,14 +552,20 @@ __global__ __launch_bounds__(64 * WAVES) void moment_forward_kernel(
   const float cs = d.cs;
   float* __restrict__ partial = d.partial;
   const float* const left = table + row * W;
-  const float* const right = left + (P + 1) * CELL;
+  const int side_words = Half::side_words(P);
+  const bool odd = grp & 1;
   auto row_sum = [&](auto tag, const uint4v& v) {
     constexpr int S = decltype(tag)::value;
     const RowTerms r = row_terms<S>(v, y, y2, l.x, qc);
     const float eta = cs * r.delta;
     const int a = (int)(r.run & 0xff), b = (int)((r.run >> 8) & 0x7f);
     const float* pl = left + a * CELL;
-    const float* pr = right + b * CELL;
+    const float* pr = left + b * CELL + side_words;
+    if (W == 3) {  // opposite sides first in neighbouring lane groups
+      const float* first = odd ? pr : pl;
+      pr = odd ? pl : pr;
+      pl = first;
+    }
     const Half l0 = Half::load(pl), l1 = Half::load(pl + HALF);
     const Half r0 = Half::load(pr), r1 = Half::load(pr + HALF);
     float t = l1.w[W - 1] + r1.w[W - 1];
@@ -656,7 +678,11 @@ __global__ __launch_bounds__(64 * WAVES) void moment_gradient_kernel(
   const int iy = task.band * R + row;
   const LineRow l = line_row(d.g, task.xc, task.tc, row);
   const float C = d.g.C;
+  // (the part of C * scale that qc rounds off: with it left out every Q is off
+  // by the same factor, up to 6e-8, which the sums over all events show)
   const float qc = C * kExp2Scale;
+  const float qc_low =
+      (float)((double)C * (-0.5 * 1.4426950408889634) - (double)qc);
   const float inv_s = d.inv_s;
   const int n_here = task.pairs;
   const uint4v* __restrict__ base =
@@ -692,7 +718,9 @@ __global__ __launch_bounds__(64 * WAVES) void moment_gradient_kernel(
           cell += kGradCell;
           const float u = __builtin_fmaf((float)(k0 + k), du, u0);
           const float v = u * inv_s, v2 = v * v, v4 = v2 * v2;
-          float t = __builtin_amdgcn_exp2f(qc * u * u) * x[k];
+          const float u2 = u * u;
+          float t = __builtin_amdgcn_exp2f(
+                        __builtin_fmaf(qc, u2, qc_low * u2)) * x[k];
           if (m0 & 2) t *= v2;
           if (m0 & 4) t *= v4;
           if (m0 & 8) t *= v4 * v4;
@@ -760,7 +788,9 @@ __global__ __launch_bounds__(64 * WAVES) void moment_gradient_kernel(
       for (int k = 0; k < n; ++k) {
         const float z = dz * dz;
         const float t =
-            __builtin_amdgcn_exp2f(__builtin_fmaf(qc, z, r.qa)) * gload(src);
+            __builtin_amdgcn_exp2f(
+                __builtin_fmaf(qc, z, __builtin_fmaf(qc_low, z, r.qa))) *
+            gload(src);
         acc += t;
         accq = __builtin_fmaf(t, C * z, accq);
         src += n_y;
@@ -827,10 +857,12 @@ __global__ __launch_bounds__(256) void moment_inverse_kernel(
 // 16-byte read-modify-write per lane; in each round the four lane groups work on
 // different (side, half) quarters of the cells, so two pairs never meet in a word
 // and no atomics are needed.  weights_of / into replace the instance's weights and
-// image where they are not null.  Bound by VALU issue (79 instructions per step of 64
-// rows) and the chain of LDS round trips at the six wavefronts per CU that the
-// cells leave room for.  2e7 events, 1000 x 400 at 1 mm: 9.9 ms, against
-// 22.0 ms for the kernel that adds pixel by pixel (an LDS read and write each).
+// image where they are not null.  Bound by VALU issue (61 instructions per step of
+// 64 rows) and the chain of LDS round trips at the six wavefronts per CU (eight
+// with 6 terms) that the cells leave room for.  2e7 events, 1000 x 400 at 1 mm:
+// 6.9 ms (8 terms 8.5 ms; 9.9 ms with a step's arithmetic not between its LDS
+// reads and writes), against 22.0 ms for the kernel that adds pixel by pixel (an
+// LDS read and write each).
 template <int NM>
 __global__ __launch_bounds__(64) void moment_backward_kernel(
     const MomentInstance* __restrict__ desc, const MomentTask* __restrict__ tasks,
@@ -856,7 +888,7 @@ __global__ __launch_bounds__(64) void moment_backward_kernel(
   const float y2 = y * y;
   const float* __restrict__ inv = weights_of ? weights_of : d.inv;
   float* __restrict__ bpT = into ? into : d.bpT;
-  const int side_words = (P + 1) * CELL;
+  const int side_words = Half::side_words(P);
   for (int i = lane; i < side_words / 2; i += 64)
     cells4[i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
   const int n_here = task.pairs;
@@ -1134,7 +1166,8 @@ int positions_for(const DeviceGeometry& g, double reach) {
 }
 
 size_t table_bytes(int positions, int terms) {
-  return sizeof(float) * 2 * (size_t)(positions + 1) * R * terms;
+  return sizeof(float) *
+         (2 * (size_t)(positions + 1) * R * terms + (terms == 6 ? 32 : 0));
 }
 
 // Device memory handed out from one allocation, in 256-byte steps.
@@ -1200,33 +1233,56 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
 
   // bins: half the reach for the vertex, half for the shear over a band
   const double sigma = 1.0 / std::sqrt((double)g.inv_pow_sigma_z);
-  const double reach = ExpPoly<8>::reach * sigma * 0.995;
-  MomentInstance d{};
-  d.g = g;
-  const double dx = reach;
-  const double dt = reach / (0.5 * (R - 1) * (double)g.pixel_height);
   const double iz = g.inv_pow_sigma_z, id = g.inv_pow_sigma_dl;
   const double k = 8.0 * iz * id / (4.0 * id + 2.0 * iz);
   const double half_width = 3.0 / std::sqrt(k);
-  const double margin = 2.0 * half_width + 4.0 * g.pixel_width +
-                        0.5 * R * g.pixel_height * max_tan + dx;
-  const double z_span = (double)g.n_z * g.pixel_width + 2.0 * margin;
-  const double nt = std::ceil(2.0 * max_tan / dt) + 1.0;
-  const double nx = std::ceil(z_span / dx) + 1.0;
   const int n_bands = (g.n_y + R - 1) / R;
-  if (!(nt <= 4096.0) || !(nx * nt * n_bands <= (double)(1 << 24))) return 0;
-  d.nx = (int)nx;
-  d.nt = (int)nt;
-  d.x_lo = (float)((double)g.tl_z - margin);
-  d.dx = (float)dx;
-  d.t_lo = (float)(-0.5 * nt * dt);
-  d.dt = (float)dt;
-  d.positions = positions_for(g, ExpPoly<8>::reach);
+  MomentInstance d{};
+  d.g = g;
   d.max_bands = std::max(st.max_bands, 1);
-  const double s = (kRunHalf + ExpPoly<8>::reach) * sigma;
-  d.inv_s = (float)(1.0 / s);
-  d.cs = (float)((double)g.C * s);
   d.n_events = n;
+  int terms = 8;
+  double n_bins_f = 0.0;
+  auto set_bins = [&]() {
+    const double reach_of = terms == 8 ? ExpPoly<8>::reach : ExpPoly<6>::reach;
+    const double reach = reach_of * sigma * 0.995;
+    const double dx = reach;
+    const double dt = reach / (0.5 * (R - 1) * (double)g.pixel_height);
+    const double margin = 2.0 * half_width + 4.0 * g.pixel_width +
+                          0.5 * R * g.pixel_height * max_tan + dx;
+    const double z_span = (double)g.n_z * g.pixel_width + 2.0 * margin;
+    const double nt = std::ceil(2.0 * max_tan / dt) + 1.0;
+    const double nx = std::ceil(z_span / dx) + 1.0;
+    n_bins_f = nx * nt * n_bands;
+    if (!(nt <= 4096.0) || !(n_bins_f <= (double)(1 << 24))) return false;
+    d.nx = (int)nx;
+    d.nt = (int)nt;
+    d.x_lo = (float)((double)g.tl_z - margin);
+    d.dx = (float)dx;
+    d.t_lo = (float)(-0.5 * nt * dt);
+    d.dt = (float)dt;
+    d.positions = positions_for(g, reach_of);
+    // (a power of two near the largest |u|: no rounding in u / s and C s)
+    const double s =
+        std::exp2(std::round(std::log2((kRunHalf + reach_of) * sigma)));
+    d.inv_s = (float)(1.0 / s);
+    d.cs = (float)((double)g.C * s);
+    return true;
+  };
+  if (!set_bins()) return 0;
+  // Six terms about lines 2.3 times closer leave room for eight instead of six
+  // back-projection wavefronts per CU (24 cells) and save arithmetic, but make
+  // five times the bins, each with its table and its expansion: taken where
+  // the bins stay full.  Measured per iteration with 8 and 6 terms: 947 pairs
+  // per bin (occupied or not) 12.1 and 10.8 ms, 100 pairs 0.40 and 0.44 ms, 83
+  // pairs of 48 cells 2.8 and 4.5 ms.
+  if ((double)n_pairs >= 400.0 * n_bins_f) {
+    terms = 6;
+    if (!set_bins()) {
+      terms = 8;
+      if (!set_bins()) return 0;
+    }
+  }
   const int n_bins = d.nx * d.nt * n_bands;
 
   // what building the plan needs
@@ -1424,11 +1480,15 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   plan.n_bins = n_bins;
   plan.n_fwd = totals[1];
   plan.n_bwd = totals[2];
-  plan.fwd_lds = plan.bwd_lds = table_bytes(d.positions, 8);
+  plan.terms = terms;
+  plan.fwd_lds = plan.bwd_lds = table_bytes(d.positions, terms);
   plan.fwd_waves = n_pairs / std::max(plan.n_fwd, 1) >= 100 ? 4 : 1;
   for (const void* kern :
        {reinterpret_cast<const void*>(moment_forward_kernel<8, 1>),
         reinterpret_cast<const void*>(moment_forward_kernel<8, 4>),
+        reinterpret_cast<const void*>(moment_forward_kernel<6, 1>),
+        reinterpret_cast<const void*>(moment_forward_kernel<6, 4>),
+        reinterpret_cast<const void*>(moment_backward_kernel<6>),
         reinterpret_cast<const void*>(moment_gradient_kernel<1>),
         reinterpret_cast<const void*>(moment_gradient_kernel<4>),
         reinterpret_cast<const void*>(moment_backward_kernel<8>)})
@@ -1442,8 +1502,12 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
 int moment_forward(MomentPlan& plan, int cur, hipStream_t stream,
                    std::string* err) {
   if (plan.n_fwd == 0) return 0;
-  auto kern = plan.fwd_waves == 4 ? moment_forward_kernel<8, 4>
-                                  : moment_forward_kernel<8, 1>;
+  const bool many = plan.fwd_waves == 4;
+  auto kern = plan.terms == 8
+                  ? (many ? moment_forward_kernel<8, 4>
+                          : moment_forward_kernel<8, 1>)
+                  : (many ? moment_forward_kernel<6, 4>
+                          : moment_forward_kernel<6, 1>);
   hipLaunchKernelGGL(kern, dim3(plan.n_fwd), dim3(64 * plan.fwd_waves),
                      plan.fwd_lds, stream, plan.desc + cur, plan.fwd_tasks);
   BAND_TRY(hipGetLastError());
@@ -1463,7 +1527,9 @@ int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
 int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
                     std::string* err, const float* weights, float* into) {
   if (plan.n_bwd == 0) return 0;
-  hipLaunchKernelGGL(moment_backward_kernel<8>, dim3(plan.n_bwd), dim3(64),
+  auto kern = plan.terms == 8 ? moment_backward_kernel<8>
+                              : moment_backward_kernel<6>;
+  hipLaunchKernelGGL(kern, dim3(plan.n_bwd), dim3(64),
                      plan.bwd_lds, stream, plan.desc + cur, plan.bwd_tasks,
                      weights, into);
   BAND_TRY(hipGetLastError());

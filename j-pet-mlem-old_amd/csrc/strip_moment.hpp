@@ -6,10 +6,12 @@
 // with u = x - X and delta = c - X,
 //   exp(-(C/2)(x - c)^2) = exp(-(C/2) u^2) exp(C u delta) exp(-(C/2) delta^2),
 // and where |C u delta| <= 1 the middle factor is a degree-7 polynomial in
-// (C s delta)(u / s) to 1.9e-7.  Events are therefore split into (event, band)
-// pairs (a band = 16 image rows) and the pairs binned by band, by the vertex at
-// the band's middle and by tan: all pairs of a bin share one sheared line X(row)
-// from which no vertex strays further than 0.214 sigma_z.  Then
+// (C s delta)(u / s) to 5e-7 (where it is <= 0.42 a degree-5 one, to 8e-7), its
+// error averaging to nothing over a run.  Events are therefore split into
+// (event, band) pairs (a band = 16 image rows) and the pairs binned by band, by
+// the vertex at the band's middle and by tan: all pairs of a bin share one
+// sheared line X(row) from which no vertex strays further than 0.214 sigma_z.
+// Then
 //   forward          a workgroup tabulates, per row and side of the line, the
 //                    running sums over columns outward from the line of
 //                    rho exp(-(C/2) u^2) (u / s)^m, m = 0..7; a row's sum over
@@ -72,6 +74,7 @@ struct MomentPlan {
   int64_t n_events = 0, n_pairs = 0;
   int n_bins = 0, n_groups = 0;
   int n_fwd = 0, n_bwd = 0;
+  int terms = 8;      // of the polynomial: 8, or 6 about closer lines
   int fwd_waves = 4;  // wavefronts per forward workgroup
   size_t fwd_lds = 0, bwd_lds = 0;
   MomentInstance inst;  // host copy (image 0)

@@ -3,7 +3,7 @@ the CPU oracle, at the edges of what it takes: band and grid remainders, runs
 clipped by the image, lines whose column is clamped, steep events, anisotropic
 pixels, the smallest lists and the smallest sigma.
 
-Tolerances, derived: a kernel value's polynomial factor is within 1.9e-7 and
+Tolerances, derived: a kernel value's polynomial factor is within 7.8e-7 and
 its 8-term FP32 evaluation within 8 x 6e-8 x e^2 = 3.5e-6 of exact (the terms'
 magnitudes sum to at most e^2 times the value); with the row terms' own FP32
 rounding (under 5e-6 between the row-band kernels and the oracle) a forward
@@ -38,6 +38,9 @@ CASES = {
         256, 160, 2.0, 2.0, 10.0, 42.0, 350.0, 500.0, 80.0, 60.0, 17),
     "wide line, dense bins": (
         300, 200, 1.0, 1.0, 10.0, 42.0, 250.0, 500.0, 40.0, 30.0, 30_000),
+    # more than 400 pairs per bin: six terms
+    "full bins": (
+        60, 32, 2.0, 2.0, 30.0, 42.0, 200.0, 200.0, 50.0, 25.0, 300_000),
 }
 
 
