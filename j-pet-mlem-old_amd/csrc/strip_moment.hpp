@@ -37,6 +37,24 @@ namespace strip {
 
 constexpr int kMomentRows = 16;  // image rows of a band
 
+// One workgroup's (forward) or wavefront's (back-projection) share of a bin.
+struct MomentTask {
+  float xc, tc;  // the bin's line: z at the band's middle row, slope
+  int band;
+  int instance;  // index of its MomentInstance
+  int group;     // first 16-pair group
+  int pairs;
+  int first_column;  // merged tasks (`pairs` counts groups): see the kernel
+  int pad;
+};
+
+// 16 pairs (fewer at a bin's end) of one bin.
+struct MomentGroup {
+  float xc, tc;
+  int bin;
+  int pairs;
+};
+
 // What the kernels need of one reconstruction (device array; a task names its
 // entry).
 struct MomentInstance {
@@ -50,6 +68,7 @@ struct MomentInstance {
   float inv_s;     // 1 / s
   float cs;        // C s
   const uint32_t* blocks;  // 1 KiB per 16 pairs (moment_pack_kernel)
+  const MomentGroup* groups;
   const float* rhoT;       // image the forward pass reads (column-major)
   float* rho_next;
   float* partial;          // per (band of the record, record)
@@ -59,16 +78,6 @@ struct MomentInstance {
   int64_t n_events;
 };
 
-// One workgroup's (forward) or wavefront's (back-projection) share of a bin.
-struct MomentTask {
-  float xc, tc;  // the bin's line: z at the band's middle row, slope
-  int band;
-  int instance;  // index of its MomentInstance
-  int group;     // first 16-pair group
-  int pairs;
-  int pad[2];
-};
-
 struct MomentPlan {
   bool ready = false;
   int64_t n_events = 0, n_pairs = 0;
@@ -76,6 +85,7 @@ struct MomentPlan {
   int n_fwd = 0, n_bwd = 0;
   int terms = 8;      // of the polynomial: 8, or 6 about closer lines
   int fwd_waves = 4;  // wavefronts per forward workgroup
+  int merged_columns = 0;  // pixel columns of a merged back-projection task
   size_t fwd_lds = 0, bwd_lds = 0;
   MomentInstance inst;  // host copy (image 0)
   void* arena = nullptr;  // per-event arrays and descriptors

@@ -38,6 +38,10 @@ CASES = {
         256, 160, 2.0, 2.0, 10.0, 42.0, 350.0, 500.0, 80.0, 60.0, 17),
     "wide line, dense bins": (
         300, 200, 1.0, 1.0, 10.0, 42.0, 250.0, 500.0, 40.0, 30.0, 30_000),
+    # more than 12000 bins of few pairs on short lines: merged
+    # back-projection tasks, clipped by the image
+    "many small bins": (
+        150, 70, 4.0, 4.0, 10.0, 42.0, 200.0, 500.0, 330.0, 150.0, 40_000),
     # more than 400 pairs per bin: six terms
     "full bins": (
         60, 32, 2.0, 2.0, 30.0, 42.0, 200.0, 200.0, 50.0, 25.0, 300_000),
