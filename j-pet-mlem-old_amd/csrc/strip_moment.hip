@@ -1321,6 +1321,27 @@ size_t table_bytes(int positions, int terms) {
          (2 * (size_t)(positions + 1) * R * terms + (terms == 6 ? 32 : 0));
 }
 
+// Whether the row-band lists do an iteration in clearly less time (20 us) than
+// the moment form.  Where the bins hold few pairs, tabulating and expanding
+// their lines costs more than walking the runs' pixels, and more so the more
+// cells a line has (its LDS leaves fewer wavefronts to a CU).  Times in ns, fitted
+// to the ones below within a third; the lists' 0.2 ms is the chain of their
+// largest tasks, which events spread over a bin each do not have.  Measured
+// (cells, pairs, occupied bins: lists, moments):
+//   7, 1.8e6, 4.8e5: 0.40, 0.85 ms      13, 3.1e4, 2.6e4: 0.06, 0.12 ms
+//   14, 1.5e6, 5.8e4: 0.49, 0.36 ms     24, 2.2e5, 6.5e4: 0.25, 0.56 ms
+//   24, 8.2e6, 1.2e5: 2.17, 1.65 ms     34, 3.2e6, 5.8e4: 1.33, 1.14 ms
+//   48, 1.4e6, 5.2e4: 0.91, 1.37 ms     48, 1.4e7, 1.2e5: 5.27, 4.53 ms
+//   66, 6.4e5, 2.0e4: 0.77, 1.04 ms     66, 4.2e6, 2.2e4: 4.20, 1.70 ms
+bool lists_faster(int positions, double pairs, double bins) {
+  const double chain =
+      2e5 * std::min({1.0, pairs / 1e5, std::max(pairs / bins - 1.0, 0.0)});
+  const double lists = chain + pairs * (0.04 + 0.0075 * positions);
+  const double moments =
+      pairs * 0.07 + bins * 8.0 * std::pow(positions / 24.0, 1.6);
+  return moments > lists + 2e4;
+}
+
 // Device memory handed out from one allocation, in 256-byte steps.
 struct Arena {
   size_t used = 0;
@@ -1567,12 +1588,7 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
                             hipMemcpyDeviceToHost, stream));
   }
   BAND_TRY(hipStreamSynchronize(stream));
-  // Where the bins hold few pairs, tabulating and expanding their lines costs
-  // more than walking the runs' pixels, and more so the more cells a line has.
-  // Measured per iteration, lists against moments: 24 cells, 2.4 pairs per bin
-  // 0.14 and 0.31 ms, 25 pairs 0.48 and 0.38 ms; 48 cells, 33 pairs 0.95 and
-  // 1.52 ms, 369 pairs 5.6 and 3.6 ms; 13 cells, 1.1 pairs 0.036 and 0.031 ms.
-  if ((double)n_pairs < 1.6 * (d.positions - 16) * (double)totals[1])
+  if (lists_faster(d.positions, (double)n_pairs, (double)totals[1]))
     return give_up();
   const int n_groups = totals[0];
   int merged_chunk = 0;

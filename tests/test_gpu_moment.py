@@ -18,8 +18,8 @@ from conftest import print_case
 pytestmark = pytest.mark.gpu
 
 # n_z, n_y, pixel width, height, sigma_z, sigma_dl, R, L, phantom half sizes,
-# events.  Lines of at most 16 cells (sigma_z up to 6 pixels) always take the
-# moment form; wider ones need dense bins.
+# events.  All of them take the moment form: where bins hold few pairs, wide lines
+# and many bins stay on the lists.
 CASES = {
     "command line defaults, sigma 1.5 px": (
         100, 100, 0.01, 0.01, 0.015, 0.06, 0.5, 1.0, 0.3, 0.3, 20_011),
