@@ -255,6 +255,44 @@ __global__ __launch_bounds__(256) void moment_records_kernel(
   counts[i] = box_bands(box);
 }
 
+// The bin of a pair: the line z = cz + t (y - cy) at the middle of band b.
+__device__ inline int pair_bin(const MomentInstance& d, float cz, float cy,
+                               float t, int jt, int b) {
+  const float yc = d.g.tl_y_half_h -
+                   ((float)(b * R) + 0.5f * (R - 1)) * d.g.pixel_height;
+  const float x = cz + t * (yc - cy);
+  const float f = floorf((x - d.x_lo) / d.dx);
+  const int ix = (int)fminf(fmaxf(f, 0.0f), (float)(d.nx - 1));
+  return (b * d.nx + ix) * d.nt + jt;
+}
+
+// occupied[bin] = 1 for every bin that has pairs
+__global__ __launch_bounds__(256) void moment_mark_kernel(
+    MomentInstance d, const uint2* __restrict__ box,
+    const float4* __restrict__ a, int64_t n, uint8_t* __restrict__ occupied) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int c = box_bands(box[i]);
+  if (!c) return;
+  const float4 ev = a[i];  // z, y, tan
+  const int jt = tan_bin(d, ev.z);
+  const int b0 = (int)(box[i].y & 0xffff) / R;
+  for (int k = 0; k < c; ++k)
+    occupied[pair_bin(d, ev.x, ev.y, ev.z, jt, b0 + k)] = 1;
+}
+
+// *total += occupied bins (four to a word)
+__global__ __launch_bounds__(256) void moment_marked_kernel(
+    const uint32_t* __restrict__ occupied, int n_words,
+    int* __restrict__ total) {
+  int c = 0;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n_words;
+       i += gridDim.x * blockDim.x)
+    c += __popc(occupied[i]);
+  c = wave_sum_int(c);
+  if ((threadIdx.x & 63) == 0 && c) atomicAdd(total, c);
+}
+
 // (bin, record) of every pair
 __global__ __launch_bounds__(256) void moment_emit_kernel(
     MomentInstance d, const BandRecord* __restrict__ rec,
@@ -270,13 +308,7 @@ __global__ __launch_bounds__(256) void moment_emit_kernel(
   const int b0 = (int)(r.by & 0xffff) / R;
   const int at = offsets[i];
   for (int k = 0; k < c; ++k) {
-    const float yc = d.g.tl_y_half_h -
-                     ((float)((b0 + k) * R) + 0.5f * (R - 1)) *
-                         d.g.pixel_height;
-    const float x = r.cz + t * (yc - r.cy);
-    const float f = floorf((x - d.x_lo) / d.dx);
-    const int ix = (int)fminf(fmaxf(f, 0.0f), (float)(d.nx - 1));
-    keys[at + k] = (uint32_t)(((b0 + k) * d.nx + ix) * d.nt + jt);
+    keys[at + k] = (uint32_t)pair_bin(d, r.cz, r.cy, t, jt, b0 + k);
     values[at + k] = (int)i;
   }
 }
@@ -1457,6 +1489,28 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   }
   const int n_bins = d.nx * d.nt * n_bands;
 
+  // Only where the occupied bins can make the lists the faster form are they
+  // counted, before anything is sorted.
+  if (lists_faster(d.positions, (double)n_pairs, (double)n_bins)) {
+    Scratch marks;
+    const int n_words = (n_bins + 3) / 4;
+    if (hipMalloc(&marks.p, sizeof(uint32_t) * (size_t)n_words) != hipSuccess)
+      return 0;
+    hipLaunchKernelGGL(fill_words_kernel, dim3(256), dim3(256), 0, stream,
+                       (uint32_t*)marks.p, (int64_t)n_words, 0u);
+    hipLaunchKernelGGL(moment_mark_kernel, dim3(grid_of(n)), dim3(256), 0,
+                       stream, d, ev.box, ev.a, n, (uint8_t*)marks.p);
+    int* d_total = reinterpret_cast<int*>(d_stats + 1) + 1;
+    hipLaunchKernelGGL(moment_marked_kernel, dim3(256), dim3(256), 0, stream,
+                       (const uint32_t*)marks.p, n_words, d_total);
+    BAND_TRY(hipGetLastError());
+    int occupied = 0;
+    BAND_TRY(hipMemcpyAsync(&occupied, d_total, sizeof(int),
+                            hipMemcpyDeviceToHost, stream));
+    BAND_TRY(hipStreamSynchronize(stream));
+    if (lists_faster(d.positions, (double)n_pairs, (double)occupied)) return 0;
+  }
+
   // what building the plan needs
   Arena work;
   const int64_t sort_n = std::max<int64_t>(n, n_pairs);
@@ -1588,8 +1642,6 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
                             hipMemcpyDeviceToHost, stream));
   }
   BAND_TRY(hipStreamSynchronize(stream));
-  if (lists_faster(d.positions, (double)n_pairs, (double)totals[1]))
-    return give_up();
   const int n_groups = totals[0];
   int merged_chunk = 0;
   // Bins of few pairs are back-projected several to a task, whose pixels are
