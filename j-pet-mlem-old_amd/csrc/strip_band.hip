@@ -768,11 +768,16 @@ __global__ __launch_bounds__(256) void batch_inverse_kernel(
   const BandInstance& d = desc[blockIdx.y];
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= d.n_events) return;
-  int x0, x1, y0, y1;
-  record_box(d.rec[e], x0, x1, y0, y1);
   float sum = 0.0f;
-  const int nb = band_count(y0, y1, x1 > x0, H, true);
-  for (int k = 0; k < nb; ++k) sum += d.partial[e * d.fwd_max_bands + k];
+  if (d.counts) {
+    const int nb = d.counts[e];
+    for (int k = 0; k < nb; ++k) sum += d.partial[k * d.n_events + e];
+  } else {
+    int x0, x1, y0, y1;
+    record_box(d.rec[e], x0, x1, y0, y1);
+    const int nb = band_count(y0, y1, x1 > x0, H, true);
+    for (int k = 0; k < nb; ++k) sum += d.partial[e * d.fwd_max_bands + k];
+  }
   d.inv[e] = (sum > 0.0f) ? 1.0f / sum : 0.0f;
 }
 
@@ -1214,7 +1219,7 @@ int band_prepare_once(BandPlan& plan, const DeviceGeometry& g,
   if (plan.tuning.moments && default_tuning(plan.tuning)) {
     bool built = false;
     if (moment_prepare(plan.moment, g, ev, n_events, plan.rhoT, plan.bpT,
-                       stream, &built, err))
+                       plan.tuning.moments == 2, stream, &built, err))
       return -1;
     if (built) {
       plan.ready = true;
@@ -1449,6 +1454,11 @@ BandInstance band_descriptor(const BandPlan& plan, const DeviceGeometry& g,
   d.span_stride = plan.span_stride;
   d.Wt = plan.Wt;
   d.fwd_max_bands = plan.fwd.max_bands;
+  if (plan.moment.ready) {
+    d.partial = plan.moment.partial;
+    d.inv = plan.moment.inv;
+    d.counts = plan.moment.counts;
+  }
   return d;
 }
 

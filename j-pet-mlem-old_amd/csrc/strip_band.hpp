@@ -63,7 +63,8 @@ struct BandTuning {
   // iteration kernels
   int spans = 1;
   // 1 = the moment form (strip_moment.hpp) where every other knob has its
-  // default value and the events suit it, 0 = always the row-band lists
+  // default value and the events suit it, 2 = the same among the members of a
+  // batch, 0 = always the row-band lists
   int moments = 1;
 };
 
@@ -114,6 +115,7 @@ struct BandInstance {
   float* inv;               // back-projection weight per record
   float* bpT;               // back-projection accumulator (column-major)
   const float* sensT;       // sensitivity (numerator mode) or null
+  const int* counts;        // moment form: bands per record, partials band-major
   int64_t n_events;
   int span_stride;
   int Wt;                   // task window width (columns)

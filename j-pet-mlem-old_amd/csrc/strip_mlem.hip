@@ -1887,7 +1887,7 @@ int strip_mlem_run(const strip_mlem_geometry* geometry,
 // ===========================================================================
 // Batched reconstructions: many independent event lists and grids iterated
 // together.  Each member keeps its own row-band plan (records, span table,
-// pair lists); the batch merges the members' task lists, tagging every task
+// pair lists, or the moment form); the batch merges the members' task lists, tagging every task
 // with its member's index, and runs each pass of an iteration as ONE launch
 // over all members (persistent workgroups walking the merged task list).
 // Iterations are recorded once into a HIP graph and replayed.
@@ -1913,6 +1913,7 @@ struct strip_mlem_batch {
   int bwd_wave_words = 0;  // LDS words per back-projection wavefront
   size_t fwd_lds = 0;
   bool spans = true;
+  strip::MomentBatch moment;  // the members in the moment form
   int64_t max_events = 0, max_pixels = 0;
   int cu_count = 0;
   int cur = 0;  // image parity of every member's plan
@@ -1938,6 +1939,7 @@ void batch_drop_merge(strip_mlem_batch* b) {
     if (d) (void)hipFree(d);
     d = nullptr;
   }
+  strip::moment_batch_release(b->moment);
   if (b->fwd_tasks) (void)hipFree(b->fwd_tasks);
   if (b->bwd_tasks) (void)hipFree(b->bwd_tasks);
   if (b->queue) (void)hipFree(b->queue);
@@ -1969,6 +1971,8 @@ int batch_merge(strip_mlem_batch* b) {
   b->bwd_wave_words = 0;
   b->spans = true;
   b->max_events = b->max_pixels = 0;
+  bool first_lists = true;
+  std::vector<const strip::MomentPlan*> moment_plans;
   for (int i = 0; i < n; ++i) {
     strip_mlem_ctx* c = b->items[i];
     if (c->band.tuning.fwd_rows != b->tuning.fwd_rows ||
@@ -1987,10 +1991,20 @@ int batch_merge(strip_mlem_batch* b) {
     int rc = ensure_band(c);
     if (rc) return rc;
     const strip::BandPlan& P = c->band;
+    b->max_events = std::max<int64_t>(b->max_events, P.n_events);
+    b->max_pixels = std::max<int64_t>(b->max_pixels, c->n_pixels);
+    d0[i] = strip::band_descriptor(P, c->g, 0);
+    d1[i] = strip::band_descriptor(P, c->g, 1);
+    b->generations.push_back(P.generation);
+    if (P.moment.ready) {
+      moment_plans.push_back(&P.moment);
+      continue;
+    }
     // the pairs per wavefront step only shape the launches: the batch takes
     // the smallest of its members' forward G and back-projection limit, and
     // the largest back-projection LDS budget (the widest member's windows)
-    if (i == 0) {
+    if (first_lists) {
+      first_lists = false;
       b->H_fwd = P.fwd.H;
       b->H_bwd = P.bwd.H;
       b->G_fwd = P.fwd_group;
@@ -2004,10 +2018,6 @@ int batch_merge(strip_mlem_batch* b) {
     b->fwd_Wt = std::max(b->fwd_Wt, P.fwd.Wt);
     b->bwd_wave_words = std::max(b->bwd_wave_words, P.bwd_wave_words);
     b->spans = b->spans && P.spans != nullptr;
-    b->max_events = std::max<int64_t>(b->max_events, P.n_events);
-    b->max_pixels = std::max<int64_t>(b->max_pixels, c->n_pixels);
-    d0[i] = strip::band_descriptor(P, c->g, 0);
-    d1[i] = strip::band_descriptor(P, c->g, 1);
     for (int4 t : P.fwd.tasks_host) {
       t.x |= i << 16;
       fwd.push_back(t);
@@ -2016,15 +2026,18 @@ int batch_merge(strip_mlem_batch* b) {
       t.x |= i << 16;
       bwd.push_back(t);
     }
-    b->generations.push_back(P.generation);
   }
+  std::string err;
+  if (strip::moment_batch_build(b->moment, moment_plans, b->stream, &err))
+    return strip::fail(STRIP_MLEM_ERR_HIP, err);
   // forward windows hold 2 H rows (bands aligned to their events)
   b->fwd_lds = sizeof(float) * (size_t)b->fwd_Wt * 2 * b->H_fwd;
   const size_t window = sizeof(float) * (size_t)b->bwd_wave_words;
   if (b->fwd_lds > 160 * 1024 || window > 160 * 1024)
     return strip::fail(STRIP_MLEM_ERR_UNSUPPORTED,
                        "a member's task window does not fit in LDS");
-  b->bwd_waves = (int)std::max<size_t>(1, std::min<size_t>(4, 160 * 1024 / window));
+  b->bwd_waves = (int)std::max<size_t>(
+      1, std::min<size_t>(4, 160 * 1024 / std::max<size_t>(window, 1)));
   for (int c = 0; c < 2; ++c) {
     HIP_TRY(hipMalloc(&b->desc[c], sizeof(strip::BandInstance) * std::max(n, 1)));
     HIP_TRY(hipMemcpy(b->desc[c], c ? d1.data() : d0.data(),
@@ -2085,7 +2098,8 @@ int batch_store_images(strip_mlem_batch* b) {
   return STRIP_MLEM_OK;
 }
 
-// One iteration of every member with image parity c (four launches).
+// One iteration of every member with image parity c: four passes, each one
+// launch over the members with lists and one per kind of moment task.
 int batch_launch_iteration(strip_mlem_batch* b, int c) {
   std::string err;
   const int n = (int)b->items.size();
@@ -2096,6 +2110,7 @@ int batch_launch_iteration(strip_mlem_batch* b, int c) {
                                  b->G_fwd, b->spans, rec, b->fwd_lds,
                                  std::min(b->n_fwd, persistent), b->queue,
                                  b->stream, &err) ||
+      strip::moment_batch_launch(b->moment, c, false, b->stream, &err) ||
       strip::band_launch_batch_update(b->desc[c], n, b->max_events,
                                       b->max_pixels, b->H_fwd, true,
                                       b->stream, &err) ||
@@ -2104,6 +2119,7 @@ int batch_launch_iteration(strip_mlem_batch* b, int c) {
           rec, b->bwd_wave_words, b->bwd_waves,
           std::min((b->n_bwd + b->bwd_waves - 1) / b->bwd_waves, persistent),
           b->queue + 1, b->stream, &err) ||
+      strip::moment_batch_launch(b->moment, c, true, b->stream, &err) ||
       strip::band_launch_batch_update(b->desc[c], n, b->max_events,
                                       b->max_pixels, b->H_fwd, false,
                                       b->stream, &err))
@@ -2191,7 +2207,7 @@ int strip_mlem_batch_create(int device, strip_mlem_batch** out) {
     return strip::fail(STRIP_MLEM_ERR_HIP, "cannot create batch stream");
   }
   b->cu_count = prop.multiProcessorCount;
-  b->tuning.moments = 0;
+  b->tuning.moments = 2;
   *out = b;
   return STRIP_MLEM_OK;
 }

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <tuple>
 #include <type_traits>
 
 #include "strip_band.hpp"
@@ -960,8 +961,7 @@ __global__ __launch_bounds__(256) void moment_inverse_kernel(
 template <int NM, bool MERGED>
 __global__ __launch_bounds__(64) void moment_backward_kernel(
     const MomentInstance* __restrict__ desc, const MomentTask* __restrict__ tasks,
-    const float* __restrict__ weights_of, float* __restrict__ into,
-    int merged_columns) {
+    const float* __restrict__ weights_of, float* __restrict__ into) {
   using Half = HalfCell<NM>;
   constexpr int W = Half::W, HALF = Half::half_words(),
                 CELL = Half::cell_words();
@@ -984,6 +984,7 @@ __global__ __launch_bounds__(64) void moment_backward_kernel(
   const float* __restrict__ inv = weights_of ? weights_of : d.inv;
   float* __restrict__ bpT = into ? into : d.bpT;
   const int side_words = Half::side_words(P);
+  const int merged_columns = MERGED ? d.merged_columns : 0;
   for (int i = lane; i < side_words / 2; i += 64)
     cells4[i] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
   const uint4v* __restrict__ base =
@@ -1365,13 +1366,59 @@ size_t table_bytes(int positions, int terms) {
 //   24, 8.2e6, 1.2e5: 2.17, 1.65 ms     34, 3.2e6, 5.8e4: 1.33, 1.14 ms
 //   48, 1.4e6, 5.2e4: 0.91, 1.37 ms     48, 1.4e7, 1.2e5: 5.27, 4.53 ms
 //   66, 6.4e5, 2.0e4: 0.77, 1.04 ms     66, 4.2e6, 2.2e4: 4.20, 1.70 ms
-bool lists_faster(int positions, double pairs, double bins) {
+// In a batch the members' tasks share the card, so nobody waits for that chain,
+// and the moment form has to be a seventh faster.  24 members of 1e4 to 3e5 events,
+// whose bins hold 2 to 186 pairs, ten iterations with all copies: 27.4 ms on the
+// lists, 43.1 ms with 22 members in the moment form, 26.0 ms with this rule.
+bool lists_faster(int positions, double pairs, double bins, bool batch) {
+  if (batch)
+    return 1.15 * (pairs * 0.07 + bins * 8.0 * std::pow(positions / 24.0, 1.6)) >
+           pairs * (0.04 + 0.0065 * positions);
   const double chain =
       2e5 * std::min({1.0, pairs / 1e5, std::max(pairs / bins - 1.0, 0.0)});
   const double lists = chain + pairs * (0.04 + 0.0075 * positions);
   const double moments =
       pairs * 0.07 + bins * 8.0 * std::pow(positions / 24.0, 1.6);
   return moments > lists + 2e4;
+}
+
+int launch_forward(int terms, int waves, size_t lds, const MomentInstance* desc,
+                   const MomentTask* tasks, int n_tasks, hipStream_t stream,
+                   std::string* err) {
+  if (n_tasks == 0) return 0;
+  auto kern = terms == 8 ? (waves == 4 ? moment_forward_kernel<8, 4>
+                                       : moment_forward_kernel<8, 1>)
+                         : (waves == 4 ? moment_forward_kernel<6, 4>
+                                       : moment_forward_kernel<6, 1>);
+  hipLaunchKernelGGL(kern, dim3(n_tasks), dim3(64 * waves), lds, stream, desc,
+                     tasks);
+  BAND_TRY(hipGetLastError());
+  return 0;
+}
+
+int launch_backward(int terms, bool merged, size_t lds,
+                    const MomentInstance* desc, const MomentTask* tasks,
+                    int n_tasks, const float* weights, float* into,
+                    hipStream_t stream, std::string* err) {
+  if (n_tasks == 0) return 0;
+  auto kern = terms == 6 ? moment_backward_kernel<6, false>
+              : merged   ? moment_backward_kernel<8, true>
+                         : moment_backward_kernel<8, false>;
+  hipLaunchKernelGGL(kern, dim3(n_tasks), dim3(64), lds, stream, desc, tasks,
+                     weights, into);
+  BAND_TRY(hipGetLastError());
+  return 0;
+}
+
+// dst = src as tasks of the batch's instance
+__global__ __launch_bounds__(256) void moment_tag_kernel(
+    const MomentTask* __restrict__ src, int n, int instance,
+    MomentTask* __restrict__ dst) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  MomentTask t = src[i];
+  t.instance = instance;
+  dst[i] = t;
 }
 
 // Device memory handed out from one allocation, in 256-byte steps.
@@ -1404,7 +1451,7 @@ void moment_release(MomentPlan& plan) {
 
 int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
                    const EventSoA& ev, int64_t n, float* const rhoT[2],
-                   float* bpT, hipStream_t stream, bool* built,
+                   float* bpT, bool batch, hipStream_t stream, bool* built,
                    std::string* err) {
   *built = false;
   moment_release(plan);
@@ -1491,7 +1538,7 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
 
   // Only where the occupied bins can make the lists the faster form are they
   // counted, before anything is sorted.
-  if (lists_faster(d.positions, (double)n_pairs, (double)n_bins)) {
+  if (lists_faster(d.positions, (double)n_pairs, (double)n_bins, batch)) {
     Scratch marks;
     const int n_words = (n_bins + 3) / 4;
     if (hipMalloc(&marks.p, sizeof(uint32_t) * (size_t)n_words) != hipSuccess)
@@ -1508,7 +1555,8 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
     BAND_TRY(hipMemcpyAsync(&occupied, d_total, sizeof(int),
                             hipMemcpyDeviceToHost, stream));
     BAND_TRY(hipStreamSynchronize(stream));
-    if (lists_faster(d.positions, (double)n_pairs, (double)occupied)) return 0;
+    if (lists_faster(d.positions, (double)n_pairs, (double)occupied, batch))
+      return 0;
   }
 
   // what building the plan needs
@@ -1731,6 +1779,7 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   d.partial = plan.partial;
   d.counts = plan.counts;
   d.groups = groups;
+  d.merged_columns = merged_columns;
   d.inv = plan.inv;
   d.bpT = bpT;
   MomentInstance both[2] = {d, d};
@@ -1753,7 +1802,7 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   plan.n_fwd = totals[1];
   plan.n_bwd = totals[2];
   plan.terms = terms;
-  plan.merged_columns = merged ? merged_columns : 0;
+  plan.merged = merged;
   plan.fwd_lds = table_bytes(d.positions, terms);
   plan.bwd_lds = plan.fwd_lds + (merged ? merged_bytes : 0);
   plan.fwd_waves = n_pairs / std::max(plan.n_fwd, 1) >= 100 ? 4 : 1;
@@ -1776,17 +1825,9 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
 
 int moment_forward(MomentPlan& plan, int cur, hipStream_t stream,
                    std::string* err) {
-  if (plan.n_fwd == 0) return 0;
-  const bool many = plan.fwd_waves == 4;
-  auto kern = plan.terms == 8
-                  ? (many ? moment_forward_kernel<8, 4>
-                          : moment_forward_kernel<8, 1>)
-                  : (many ? moment_forward_kernel<6, 4>
-                          : moment_forward_kernel<6, 1>);
-  hipLaunchKernelGGL(kern, dim3(plan.n_fwd), dim3(64 * plan.fwd_waves),
-                     plan.fwd_lds, stream, plan.desc + cur, plan.fwd_tasks);
-  BAND_TRY(hipGetLastError());
-  return 0;
+  return launch_forward(plan.terms, plan.fwd_waves, plan.fwd_lds,
+                        plan.desc + cur, plan.fwd_tasks, plan.n_fwd, stream,
+                        err);
 }
 
 int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
@@ -1801,15 +1842,9 @@ int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
 
 int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
                     std::string* err, const float* weights, float* into) {
-  if (plan.n_bwd == 0) return 0;
-  auto kern = plan.terms == 6        ? moment_backward_kernel<6, false>
-              : plan.merged_columns ? moment_backward_kernel<8, true>
-                                    : moment_backward_kernel<8, false>;
-  hipLaunchKernelGGL(kern, dim3(plan.n_bwd), dim3(64),
-                     plan.bwd_lds, stream, plan.desc + cur, plan.bwd_tasks,
-                     weights, into, plan.merged_columns);
-  BAND_TRY(hipGetLastError());
-  return 0;
+  return launch_backward(plan.terms, plan.merged, plan.bwd_lds,
+                         plan.desc + cur, plan.bwd_tasks, plan.n_bwd, weights,
+                         into, stream, err);
 }
 
 int moment_gradient(MomentPlan& plan, const float* xT, int stride, float* out,
@@ -1821,6 +1856,105 @@ int moment_gradient(MomentPlan& plan, const float* xT, int stride, float* out,
                      table_bytes(plan.inst.positions, kGradMoments), stream,
                      plan.desc, plan.fwd_tasks, xT, stride, out);
   BAND_TRY(hipGetLastError());
+  return 0;
+}
+
+void moment_batch_release(MomentBatch& batch) {
+  for (MomentInstance* d : batch.desc)
+    if (d) (void)hipFree(d);
+  if (batch.tasks) (void)hipFree(batch.tasks);
+  batch = MomentBatch{};
+}
+
+int moment_batch_build(MomentBatch& batch,
+                       const std::vector<const MomentPlan*>& plans,
+                       hipStream_t stream, std::string* err) {
+  moment_batch_release(batch);
+  if (plans.empty()) return 0;
+  const int n = (int)plans.size();
+  std::vector<MomentInstance> inst(n);
+  for (int c = 0; c < 2; ++c) {
+    for (int i = 0; i < n; ++i) {
+      inst[i] = plans[i]->inst;
+      if (c) {
+        float* next = const_cast<float*>(inst[i].rhoT);
+        inst[i].rhoT = inst[i].rho_next;
+        inst[i].rho_next = next;
+      }
+    }
+    BAND_TRY(hipMalloc(&batch.desc[c], sizeof(MomentInstance) * n));
+    BAND_TRY(hipMemcpy(batch.desc[c], inst.data(), sizeof(MomentInstance) * n,
+                       hipMemcpyHostToDevice));
+  }
+  // parts: a plan's forward or back-projection tasks; those of one launch are
+  // put next to each other, the plans with most pairs first
+  struct Part {
+    MomentBatch::Launch kind;
+    int plan;
+  };
+  std::vector<Part> parts;
+  int64_t total = 0;
+  for (int i = 0; i < n; ++i) {
+    const MomentPlan& p = *plans[i];
+    const Part fwd{{false, p.terms, p.fwd_waves, false, p.fwd_lds, 0, p.n_fwd},
+                   i};
+    const Part bwd{{true, p.terms, 1, p.merged, p.bwd_lds, 0, p.n_bwd}, i};
+    for (const Part& part : {fwd, bwd})
+      if (part.kind.n) {
+        parts.push_back(part);
+        total += part.kind.n;
+      }
+  }
+  if (total > 0x7fffffff) {
+    if (err) *err = "too many tasks in one batch";
+    return -1;
+  }
+  auto key = [](const MomentBatch::Launch& l) {
+    const int residents = (int)std::min<size_t>(kLds / std::max<size_t>(l.lds, 1), 16);
+    return std::make_tuple(l.backward, l.terms, l.waves, l.merged, residents);
+  };
+  std::stable_sort(parts.begin(), parts.end(),
+                   [&](const Part& a, const Part& b) {
+                     const auto ka = key(a.kind), kb = key(b.kind);
+                     if (ka != kb) return ka < kb;
+                     return plans[a.plan]->n_pairs > plans[b.plan]->n_pairs;
+                   });
+  BAND_TRY(hipMalloc(&batch.tasks,
+                     sizeof(MomentTask) * std::max<int64_t>(total, 1)));
+  int at = 0;
+  for (const Part& part : parts) {
+    const MomentPlan& p = *plans[part.plan];
+    hipLaunchKernelGGL(moment_tag_kernel, dim3(grid_of(part.kind.n)), dim3(256),
+                       0, stream,
+                       part.kind.backward ? p.bwd_tasks : p.fwd_tasks,
+                       part.kind.n, part.plan, batch.tasks + at);
+    BAND_TRY(hipGetLastError());
+    if (batch.launches.empty() ||
+        key(batch.launches.back()) != key(part.kind)) {
+      batch.launches.push_back(part.kind);
+      batch.launches.back().first = at;
+    } else {
+      batch.launches.back().n += part.kind.n;
+      batch.launches.back().lds =
+          std::max(batch.launches.back().lds, part.kind.lds);
+    }
+    at += part.kind.n;
+  }
+  BAND_TRY(hipStreamSynchronize(stream));
+  return 0;
+}
+
+int moment_batch_launch(const MomentBatch& batch, int c, bool backward,
+                        hipStream_t stream, std::string* err) {
+  for (const MomentBatch::Launch& l : batch.launches) {
+    if (l.backward != backward) continue;
+    const MomentTask* tasks = batch.tasks + l.first;
+    if (backward ? launch_backward(l.terms, l.merged, l.lds, batch.desc[c],
+                                   tasks, l.n, nullptr, nullptr, stream, err)
+                 : launch_forward(l.terms, l.waves, l.lds, batch.desc[c], tasks,
+                                  l.n, stream, err))
+      return -1;
+  }
   return 0;
 }
 

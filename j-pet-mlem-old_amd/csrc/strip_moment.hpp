@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <vector>
 
 #include "strip_device.hpp"
 
@@ -64,6 +65,7 @@ struct MomentInstance {
   float x_lo, dx;  // lower edge of bin 0 and bin width, z coordinate
   float t_lo, dt;  // the same of tan
   int positions;   // table cells per row and side, besides the empty one
+  int merged_columns;  // pixel columns of a merged back-projection task
   int max_bands;
   float inv_s;     // 1 / s
   float cs;        // C s
@@ -85,7 +87,7 @@ struct MomentPlan {
   int n_fwd = 0, n_bwd = 0;
   int terms = 8;      // of the polynomial: 8, or 6 about closer lines
   int fwd_waves = 4;  // wavefronts per forward workgroup
-  int merged_columns = 0;  // pixel columns of a merged back-projection task
+  bool merged = false;  // back-projection tasks of several bins
   size_t fwd_lds = 0, bwd_lds = 0;
   MomentInstance inst;  // host copy (image 0)
   void* arena = nullptr;  // per-event arrays and descriptors
@@ -105,10 +107,11 @@ struct MomentPlan {
 bool moment_supported(const DeviceGeometry& g);
 
 // Builds the plan for the events.  *built = false (and 0) where the row-band
-// lists are the better choice or the plan does not fit.
+// lists are the better choice (batch: among the members of a batch) or the plan
+// does not fit.
 int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
                    const EventSoA& ev, int64_t n_events, float* const rhoT[2],
-                   float* bpT, hipStream_t stream, bool* built,
+                   float* bpT, bool batch, hipStream_t stream, bool* built,
                    std::string* err);
 void moment_release(MomentPlan& plan);
 
@@ -127,6 +130,27 @@ int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
 // sum K x Q, sum K x (w - Qd) of the column-major image xT (strip_adjoint.hip)
 int moment_gradient(MomentPlan& plan, const float* xT, int stride, float* out,
                     hipStream_t stream, std::string* err);
+// The plans of many reconstructions, iterated together: one launch per pass and
+// kind of task (terms, wavefronts, merged, workgroups that share a CU).
+struct MomentBatch {
+  struct Launch {
+    bool backward;
+    int terms, waves;
+    bool merged;
+    size_t lds;
+    int first, n;  // tasks
+  };
+  std::vector<Launch> launches;
+  MomentInstance* desc[2] = {nullptr, nullptr};  // image parity 0 / 1
+  MomentTask* tasks = nullptr;
+};
+void moment_batch_release(MomentBatch& batch);
+int moment_batch_build(MomentBatch& batch,
+                       const std::vector<const MomentPlan*>& plans,
+                       hipStream_t stream, std::string* err);
+// the forward or back-projection launches, image parity c
+int moment_batch_launch(const MomentBatch& batch, int c, bool backward,
+                        hipStream_t stream, std::string* err);
 // *total += kernel evaluations of the stored runs
 int moment_count(MomentPlan& plan, unsigned long long* total,
                  hipStream_t stream, std::string* err);

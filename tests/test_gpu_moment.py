@@ -134,3 +134,27 @@ def test_moment_form_knobs(pystrip_mod, phantom_mod, oracle_mod):
         rec.iterate(2)
         assert oracle_mod.rel_l2(rec.rho, ref) <= 1e-4
         assert rec.band_tiling()[:2] == tiling[:2]
+
+
+def test_moment_form_in_a_batch(pystrip_mod, phantom_mod, oracle_mod):
+    # members of every kind of task (few and many terms, merged, one and four
+    # wavefronts) and one that stays on the lists, iterated together, eagerly
+    # and replayed
+    names = ["full bins", "many small bins", "wide line, dense bins",
+             "command line defaults, sigma 1.5 px", "one event"]
+    print_case("moment form in a batch:", names)
+    cases = [_case(pystrip_mod, phantom_mod, oracle_mod, n) for n in names]
+    ev, g, og = cases[2]
+    cases.append((ev[:300], g, og))  # wide lines, sparse: lists
+    for graph in (False, True):
+        b = pystrip_mod.Batch()
+        b.set_graph(graph)
+        for ev, g, _ in cases:
+            b.add(g, ev)
+        b.iterate(2)
+        b.iterate(5)
+        for i, (ev, g, og) in enumerate(cases):
+            ref = oracle_mod.mlem(og, ev, iterations=7)
+            e = oracle_mod.rel_l2(b.rho(i), ref)
+            print(i, e)
+            assert e <= 1e-4
