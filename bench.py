@@ -30,15 +30,17 @@ PEAK_FP32_TFLOPS = 157.3
 # algorithmic FP32 operations per kernel evaluation (forward + back-projection
 # of one in-ellipse pixel): Q = rowA + dz*(rowB + C*dz) (2 FMA = 4 flop),
 # exp2 (1), K = pre*e (1), D += K*rho (2); again Q (4), exp2 (1), K (1),
-# K*inv (1) and the image add (1)
+# K*inv (1) and the image add (1).  The moment form gets the same sums with
+# fewer operations (a row costs the same whatever its run's length), so the
+# rate this gives is one of the algorithm's work, not of instructions issued.
 FLOPS_PER_KERNEL_EVAL = 16
-# HBM bytes per launch (read + written) of the band kernels on the default
+# HBM bytes per launch (read + written) of the moment kernels on the default
 # workload, from two rocprofv3 --pmc runs (FETCH_SIZE, WRITE_SIZE) each scaled
 # by the counter's reading for a plain 256 MiB copy kernel (x2.0 and x1.0);
-# recorded in profiles/band_kernels_strip-1000x400-1mm-2e7_counters.md
+# recorded in profiles/moment_kernels_strip-1000x400-1mm-2e7.md
 MEASURED_TRAFFIC_BYTES = {
-    "back-projection": (41.51 + 0.90) * 1e9,
-    "forward projection": (22.49 + 2.24) * 1e9,
+    "back-projection": (12.19 + 0.78) * 1e9,
+    "forward projection": (10.36 + 1.32) * 1e9,
 }
 TRAFFIC_WORKLOAD = "strip-1000x400-1mm-2e7"
 
@@ -528,7 +530,7 @@ def main():
             "frac": achieved_tflops / PEAK_FP32_TFLOPS,
             "traffic": (MEASURED_TRAFFIC_BYTES.get(dom_name)
                         if w.name == TRAFFIC_WORKLOAD and
-                        n_events == w.n_events and args.algorithm in (0, 2)
+                        n_events == w.n_events and args.algorithm == 0
                         else None),
             "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE + "
                             "WRITE_SIZE, copy-calibrated)",

@@ -296,7 +296,8 @@ int strip_mlem_unrolled_gradient_device(strip_mlem_ctx* ctx, const float* rho0,
  * one reconstruction per process).  Many independent event lists, each with
  * its own geometry and grid, iterated together: every pass of an iteration is
  * one launch over all members (persistent workgroups over the merged task
- * list) and the iterations are recorded once into a HIP graph and replayed.
+ * list; one more per kind of task for members in the moment form) and the
+ * iterations are recorded once into a HIP graph and replayed.
  * Members use the reference CPU semantics and start at rho = 1. ---- */
 typedef struct strip_mlem_batch strip_mlem_batch;
 
