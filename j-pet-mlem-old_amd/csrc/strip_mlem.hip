@@ -1155,10 +1155,20 @@ int strip_mlem_create(const strip_mlem_geometry* geometry,
   if ((m.kernel != 0 || m.sensitivity == 1) &&
       ctx->n_pixels <= kBpCopiesPixels)
     ctx->bp_copies = kBpCopies;
+  if (hipMalloc(&ctx->bp, sizeof(float) * ctx->n_pixels * ctx->bp_copies) !=
+      hipSuccess) {
+    ctx->bp = nullptr;
+    // where the copies do not fit, one serves as well
+    if (ctx->bp_copies > 1) {
+      (void)hipGetLastError();
+      ctx->bp_copies = 1;
+      if (hipMalloc(&ctx->bp, sizeof(float) * ctx->n_pixels) != hipSuccess)
+        ctx->bp = nullptr;
+    }
+  }
   if (hipMalloc(&ctx->rho[0], sizeof(float) * ctx->n_pixels) != hipSuccess ||
       hipMalloc(&ctx->rho[1], sizeof(float) * ctx->n_pixels) != hipSuccess ||
-      hipMalloc(&ctx->bp, sizeof(float) * ctx->n_pixels * ctx->bp_copies) !=
-          hipSuccess ||
+      !ctx->bp ||
       hipMalloc(&ctx->counter, sizeof(unsigned long long)) != hipSuccess)
     return cleanup(strip::fail(STRIP_MLEM_ERR_ALLOC, "cannot allocate images"));
   if ((rc = fill(ctx, ctx->rho[0], ctx->n_pixels, 1.0f)) ||

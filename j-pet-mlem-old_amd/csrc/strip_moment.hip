@@ -448,7 +448,8 @@ __global__ __launch_bounds__(256) void moment_task_emit_kernel(
 __global__ __launch_bounds__(256) void moment_pack_kernel(
     MomentInstance d, const BandRecord* __restrict__ rec,
     const MomentGroup* __restrict__ groups,
-    const int* __restrict__ group_pair, const int* __restrict__ values, int n_groups, int n_records, int spare,
+    const int* __restrict__ group_pair, const int* __restrict__ values,
+    int n_groups, int n_records, int spare,
     uint4* __restrict__ blocks, int* __restrict__ status) {
   __shared__ uint32_t words[kGroup * 16];
   const int pair = threadIdx.x >> 4, row = threadIdx.x & 15;
@@ -1541,8 +1542,12 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   if (lists_faster(d.positions, (double)n_pairs, (double)n_bins, batch)) {
     Scratch marks;
     const int n_words = (n_bins + 3) / 4;
-    if (hipMalloc(&marks.p, sizeof(uint32_t) * (size_t)n_words) != hipSuccess)
+    if (hipMalloc(&marks.p, sizeof(uint32_t) * (size_t)n_words) !=
+        hipSuccess) {
+      marks.p = nullptr;
+      (void)hipGetLastError();
       return 0;
+    }
     hipLaunchKernelGGL(fill_words_kernel, dim3(256), dim3(256), 0, stream,
                        (uint32_t*)marks.p, (int64_t)n_words, 0u);
     hipLaunchKernelGGL(moment_mark_kernel, dim3(grid_of(n)), dim3(256), 0,
