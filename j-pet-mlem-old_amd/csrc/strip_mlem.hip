@@ -1983,6 +1983,9 @@ int batch_merge(strip_mlem_batch* b) {
   b->max_events = b->max_pixels = 0;
   bool first_lists = true;
   std::vector<const strip::MomentPlan*> moment_plans;
+  // (the batch takes them when the merge is whole: after an error it is not
+  // current, and the next call builds it anew)
+  std::vector<int64_t> generations;
   for (int i = 0; i < n; ++i) {
     strip_mlem_ctx* c = b->items[i];
     if (c->band.tuning.fwd_rows != b->tuning.fwd_rows ||
@@ -2005,7 +2008,7 @@ int batch_merge(strip_mlem_batch* b) {
     b->max_pixels = std::max<int64_t>(b->max_pixels, c->n_pixels);
     d0[i] = strip::band_descriptor(P, c->g, 0);
     d1[i] = strip::band_descriptor(P, c->g, 1);
-    b->generations.push_back(P.generation);
+    generations.push_back(P.generation);
     if (P.moment.ready) {
       moment_plans.push_back(&P.moment);
       continue;
@@ -2075,6 +2078,7 @@ int batch_merge(strip_mlem_batch* b) {
                       hipMemcpyHostToDevice));
   }
   b->images_loaded = false;
+  b->generations = std::move(generations);
   return STRIP_MLEM_OK;
 }
 
