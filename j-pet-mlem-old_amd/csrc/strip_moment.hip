@@ -1383,17 +1383,23 @@ bool lists_faster(int positions, double pairs, double bins, bool batch) {
   return moments > lists + 2e4;
 }
 
+// A dispatch counts its work-items in 32 bits: tasks of one launch.
+constexpr int64_t kLaunchItems = (int64_t)1 << 31;
+int64_t tasks_per_launch(int waves) { return kLaunchItems / (64 * waves); }
+
 int launch_forward(int terms, int waves, size_t lds, const MomentInstance* desc,
                    const MomentTask* tasks, int n_tasks, hipStream_t stream,
                    std::string* err) {
-  if (n_tasks == 0) return 0;
   auto kern = terms == 8 ? (waves == 4 ? moment_forward_kernel<8, 4>
                                        : moment_forward_kernel<8, 1>)
                          : (waves == 4 ? moment_forward_kernel<6, 4>
                                        : moment_forward_kernel<6, 1>);
-  hipLaunchKernelGGL(kern, dim3(n_tasks), dim3(64 * waves), lds, stream, desc,
-                     tasks);
-  BAND_TRY(hipGetLastError());
+  const int64_t most = tasks_per_launch(waves);
+  for (int64_t at = 0; at < n_tasks; at += most) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min(most, n_tasks - at)),
+                       dim3(64 * waves), lds, stream, desc, tasks + at);
+    BAND_TRY(hipGetLastError());
+  }
   return 0;
 }
 
@@ -1401,13 +1407,15 @@ int launch_backward(int terms, bool merged, size_t lds,
                     const MomentInstance* desc, const MomentTask* tasks,
                     int n_tasks, const float* weights, float* into,
                     hipStream_t stream, std::string* err) {
-  if (n_tasks == 0) return 0;
   auto kern = terms == 6 ? moment_backward_kernel<6, false>
               : merged   ? moment_backward_kernel<8, true>
                          : moment_backward_kernel<8, false>;
-  hipLaunchKernelGGL(kern, dim3(n_tasks), dim3(64), lds, stream, desc, tasks,
-                     weights, into);
-  BAND_TRY(hipGetLastError());
+  const int64_t most = tasks_per_launch(1);
+  for (int64_t at = 0; at < n_tasks; at += most) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min(most, n_tasks - at)),
+                       dim3(64), lds, stream, desc, tasks + at, weights, into);
+    BAND_TRY(hipGetLastError());
+  }
   return 0;
 }
 

@@ -1,7 +1,15 @@
-"""A batch whose merge runs out of memory, on a HIP runtime without a GPU: the
-error is returned and no half-built merge is left behind, so later calls build
-it anew instead of launching kernels on descriptors that do not exist."""
+"""A batch at its limits, on a HIP runtime without a GPU.
+
+Where its merge runs out of memory, the error is returned and no half-built
+merge is left behind: later calls build it anew instead of launching kernels on
+descriptors that do not exist.  Where its members have more tasks than one
+launch may have, there are several launches.
+"""
+import os
+import subprocess
+
 import hip_stub
+import pytest
 
 
 def test_merge_is_built_anew_after_a_failed_allocation(tmp_path):
@@ -46,3 +54,27 @@ def test_merge_is_built_anew_after_a_failed_allocation(tmp_path):
         assert last, f"allocation {k}: the batch does not recover"
         assert launches > 0 and without_descriptors == 0, \
             f"allocation {k}: launched on a half-built merge"
+
+
+@pytest.mark.parametrize("backward, waves, tasks", [
+    (0, 4, 1000), (0, 4, (1 << 24) + 3), (0, 1, (1 << 26) + 1),
+    (1, 1, (1 << 26) + 1), (1, 1, 0)])
+def test_no_launch_of_more_work_items_than_a_dispatch_counts(
+        tmp_path, backward, waves, tasks):
+    # a dispatch counts its work-items in 32 bits; the members' tasks together
+    # can be more, and every one of them has to run
+    lib = str(tmp_path / "launch.so")
+    subprocess.run(["/opt/rocm/bin/hipcc", "-O1", "-std=c++17", "-shared",
+                    "-fPIC", "-x", "hip", "--offload-host-only",
+                    *hip_stub.compiler()[3:], os.path.join(
+                        hip_stub.HERE, "moment_batch_launch.cpp"),
+                    "-o", lib], check=True, capture_output=True, text=True)
+    over, items = hip_stub.run(tmp_path, f"""
+        ctypes.CDLL(pystrip.LIB_PATH, mode=ctypes.RTLD_GLOBAL)
+        assert ctypes.CDLL({lib!r}).launch_tasks({backward}, {waves},
+                                                 {tasks}) == 0
+        result = [stub.stub_launches(b"moment_", 0, (1 << 32) - 1),
+                  stub.stub_work_items(b"moment_")]
+    """)
+    assert over == 0
+    assert items == tasks * waves * 64
