@@ -219,6 +219,14 @@ int strip_mlem_set_backprojection_occupancy(strip_mlem_ctx* ctx,
 int strip_mlem_set_span_table(strip_mlem_ctx* ctx, int enable);
 int strip_mlem_get_span_table(strip_mlem_ctx* ctx, int* in_use);
 
+/* How many of the plans of the resident events (one, or one per ordered subset
+ * or per split of a long list) run in the moment form and how many over
+ * row-band lists; 0 and 0 with the bbox kernel.  A batch member's context
+ * answers for the member.  Builds the plans where they are not built yet, as
+ * the next iteration would. */
+int strip_mlem_get_plan_forms(strip_mlem_ctx* ctx, int* moment_plans,
+                              int* list_plans);
+
 /* The row-band tiling: band rows of both kernels, the widest
  * back-projection task window (columns) and the number of (event, band) pairs
  * of both kernels (where the moment form is in use, those its events would

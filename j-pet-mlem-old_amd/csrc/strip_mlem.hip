@@ -1679,6 +1679,21 @@ int strip_mlem_get_span_table(strip_mlem_ctx* ctx, int* in_use) {
   return STRIP_MLEM_OK;
 }
 
+int strip_mlem_get_plan_forms(strip_mlem_ctx* ctx, int* moment_plans,
+                              int* list_plans) {
+  CTX_CHECK(ctx);
+  if (!moment_plans || !list_plans)
+    return strip::fail(STRIP_MLEM_ERR_ARGUMENT, "NULL output");
+  *moment_plans = *list_plans = 0;
+  if (effective_algorithm(ctx) != 2) return STRIP_MLEM_OK;
+  std::vector<const strip::BandPlan*> plans;
+  int rc = active_plans(ctx, plans);
+  if (rc) return rc;
+  for (const strip::BandPlan* p : plans)
+    ++*(p->moment.ready ? moment_plans : list_plans);
+  return STRIP_MLEM_OK;
+}
+
 int strip_mlem_get_band_tiling(strip_mlem_ctx* ctx, int* forward_rows,
                                int* backward_rows, int* window_columns,
                                int64_t* forward_pairs,

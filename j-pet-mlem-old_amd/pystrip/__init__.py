@@ -219,6 +219,8 @@ def load_library():
                                                                dptr, P, dptr]),
         "strip_mlem_get_span_table": (ctypes.c_int,
                                       [P, ctypes.POINTER(ctypes.c_int)]),
+        "strip_mlem_get_plan_forms": (ctypes.c_int, [
+            P, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]),
         "strip_mlem_get_band_tiling": (ctypes.c_int, [
             P, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int),
             ctypes.POINTER(ctypes.c_int), ctypes.POINTER(i64),
@@ -274,7 +276,8 @@ def exported_symbols():
         "strip_mlem_batch_get_backprojection_occupancy",
         "strip_mlem_set_band_groups", "strip_mlem_get_band_groups",
         "strip_mlem_batch_set_groups", "strip_mlem_batch_get_groups",
-        "strip_mlem_get_span_table", "strip_mlem_loglik_gradient",
+        "strip_mlem_get_span_table", "strip_mlem_get_plan_forms",
+        "strip_mlem_loglik_gradient",
         "strip_mlem_loglik_gradient_device", "strip_mlem_unrolled_gradient",
         "strip_mlem_unrolled_gradient_device", "strip_mlem_batch_create",
         "strip_mlem_batch_destroy", "strip_mlem_batch_add",
@@ -449,6 +452,13 @@ class Reconstruction:
         v = ctypes.c_int()
         _check(self._lib.strip_mlem_get_span_table(self._ctx, ctypes.byref(v)))
         return bool(v.value)
+
+    def plan_forms(self):
+        """(plans in the moment form, plans over row-band lists)."""
+        m, l = ctypes.c_int(), ctypes.c_int()
+        _check(self._lib.strip_mlem_get_plan_forms(
+            self._ctx, ctypes.byref(m), ctypes.byref(l)))
+        return m.value, l.value
 
     def band_tiling(self):
         """(forward rows, back-projection rows, window columns,
