@@ -288,21 +288,34 @@ __global__ __launch_bounds__(256) void to_row_major_kernel(
   }
 }
 
+// A pixel of the back-projection, the sum over `images` of them, n apart; the
+// images are cleared.
+__device__ inline float take_pixel(float* __restrict__ bp, int64_t n,
+                                   int images, int64_t i) {
+  float sum = bp[i];
+  bp[i] = 0.0f;
+  for (int k = 1; k < images; ++k) {
+    sum += bp[k * n + i];
+    bp[k * n + i] = 0.0f;
+  }
+  return sum;
+}
+
 // rhoT'(p) = rhoT(p) * bpT(p) [/ sT(p)]; bpT = 0
 // (scale != 1: the update is multiplied by scale in FP64, the count ratio of
 // an ordered-subset update)
 __global__ __launch_bounds__(256) void band_finalize_kernel(
     int64_t n, const float* __restrict__ rho, float* __restrict__ bp,
-    const float* __restrict__ sens, int divide, double scale,
+    int images, const float* __restrict__ sens, int divide, double scale,
     float* __restrict__ next, float* __restrict__ bp_out) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    if (bp_out) bp_out[i] = bp[i];
-    float v = rho[i] * bp[i];
+    const float b = take_pixel(bp, n, images, i);
+    if (bp_out) bp_out[i] = b;
+    float v = rho[i] * b;
     if (divide) v = v / sens[i];
     if (scale != 1.0) v = (float)((double)v * scale);
     next[i] = v;
-    bp[i] = 0.0f;
   }
 }
 
@@ -788,8 +801,7 @@ __global__ __launch_bounds__(256) void batch_finalize_kernel(
   const int64_t n = (int64_t)d.g.n_z * d.g.n_y;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    d.rho_next[i] = d.rhoT[i] * d.bpT[i];
-    d.bpT[i] = 0.0f;
+    d.rho_next[i] = d.rhoT[i] * take_pixel(d.bpT, n, d.bp_images, i);
   }
 }
 
@@ -1449,6 +1461,7 @@ BandInstance band_descriptor(const BandPlan& plan, const DeviceGeometry& g,
   d.partial = plan.partial;
   d.inv = plan.inv;
   d.bpT = plan.bpT;
+  d.bp_images = 1;
   d.sensT = plan.sensT;
   d.n_events = plan.n_events;
   d.span_stride = plan.span_stride;
@@ -1457,6 +1470,8 @@ BandInstance band_descriptor(const BandPlan& plan, const DeviceGeometry& g,
   if (plan.moment.ready) {
     d.partial = plan.moment.partial;
     d.inv = plan.moment.inv;
+    d.bpT = plan.moment.bpT;
+    d.bp_images = plan.moment.bp_images;
     d.counts = plan.moment.counts;
   }
   return d;
@@ -1530,18 +1545,29 @@ int band_store_image(BandPlan& plan, const DeviceGeometry& g, float* rho,
   return 0;
 }
 
-int band_finalize(BandPlan& plan, const DeviceGeometry& g,
-                  int sensitivity_mode, hipStream_t stream, std::string* err,
-                  double scale, float* bp_out) {
-  const int64_t n_pixels = (int64_t)g.n_z * g.n_y;
+namespace {
+
+int finalize_from(BandPlan& plan, float* bp, int images, int64_t n_pixels,
+                  int sensitivity_mode, double scale, float* bp_out,
+                  hipStream_t stream, std::string* err) {
   const int blocks = (int)std::min<int64_t>((n_pixels + 255) / 256, 4096);
   hipLaunchKernelGGL(band_finalize_kernel, dim3(blocks), dim3(256), 0, stream,
-                     n_pixels, plan.rhoT[plan.curT], plan.bpT, plan.sensT,
+                     n_pixels, plan.rhoT[plan.curT], bp, images, plan.sensT,
                      sensitivity_mode == 2 ? 1 : 0, scale,
                      plan.rhoT[plan.curT ^ 1], bp_out);
   BAND_TRY(hipGetLastError());
   plan.curT ^= 1;
   return 0;
+}
+
+}  // namespace
+
+int band_finalize(BandPlan& plan, const DeviceGeometry& g,
+                  int sensitivity_mode, hipStream_t stream, std::string* err,
+                  double scale, float* bp_out) {
+  const int64_t n_pixels = (int64_t)g.n_z * g.n_y;
+  return finalize_from(plan, plan.bpT, 1, n_pixels, sensitivity_mode, scale,
+                       bp_out, stream, err);
 }
 
 int band_iteration(BandPlan& plan, const DeviceGeometry& g,
@@ -1565,9 +1591,11 @@ int band_iteration(BandPlan& plan, const DeviceGeometry& g,
         moment_backward(plan.moment, plan.curT, stream, err))
       return -1;
     if (t_bwd) BAND_TRY(hipEventRecord(t_bwd, stream));
-    if (!finalize) return 0;
-    return band_finalize(plan, g, sensitivity_mode, stream, err, scale,
-                         bp_out);
+    // (several plans that add to one image update it together)
+    if (!finalize) return moment_fold(plan.moment, plan.bpT, stream, err);
+    return finalize_from(plan, plan.moment.bpT, plan.moment.bp_images,
+                         (int64_t)g.n_z * g.n_y, sensitivity_mode, scale,
+                         bp_out, stream, err);
   }
   if (dispatch_forward(plan, g, 0, nullptr, stream, err)) return -1;
   if (t_fwd) BAND_TRY(hipEventRecord(t_fwd, stream));
@@ -1644,7 +1672,7 @@ int band_backproject(BandPlan& plan, const DeviceGeometry& g,
     return -1;
   }
   if (plan.moment.ready)
-    return moment_backward(plan.moment, 0, stream, err, weights, outT);
+    return moment_backward_into(plan.moment, weights, outT, stream, err);
   return dispatch_backward(plan, g, weights, outT, stream, err);
 }
 

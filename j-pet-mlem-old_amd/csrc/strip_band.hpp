@@ -114,6 +114,7 @@ struct BandInstance {
   float* partial;           // partial D per (record, forward band)
   float* inv;               // back-projection weight per record
   float* bpT;               // back-projection accumulator (column-major)
+  int bp_images;            // moment form: images it is the sum of, else 1
   const float* sensT;       // sensitivity (numerator mode) or null
   const int* counts;        // moment form: bands per record, partials band-major
   int64_t n_events;

@@ -950,7 +950,7 @@ __global__ __launch_bounds__(256) void moment_inverse_kernel(
 // 16-byte read-modify-write per lane; in each round the four lane groups work on
 // different (side, half) quarters of the cells, so two pairs never meet in a word
 // and no atomics are needed.  weights_of / into replace the instance's weights and
-// image where they are not null.  Bound by VALU issue (61 instructions per step of
+// images where they are not null.  Bound by VALU issue (61 instructions per step of
 // 64 rows) and the chain of LDS round trips at the six wavefronts per CU (eight
 // with 6 terms) that the cells leave room for.  2e7 events, 1000 x 400 at 1 mm:
 // 6.9 ms (8 terms 8.5 ms; 9.9 ms with a step's arithmetic not between its LDS
@@ -983,7 +983,9 @@ __global__ __launch_bounds__(64) void moment_backward_kernel(
   const float y = pixel_center_y(d.g, iy);
   const float y2 = y * y;
   const float* __restrict__ inv = weights_of ? weights_of : d.inv;
-  float* __restrict__ bpT = into ? into : d.bpT;
+  float* __restrict__ bpT =
+      into ? into
+           : d.bpT + (int64_t)(blockIdx.x % (unsigned)d.bp_images) * n_z * n_y;
   const int side_words = Half::side_words(P);
   const int merged_columns = MERGED ? d.merged_columns : 0;
   for (int i = lane; i < side_words / 2; i += 64)
@@ -1302,6 +1304,20 @@ __global__ __launch_bounds__(64) void moment_backward_kernel(
   }
 }
 
+// out += the sum of the images, which are cleared
+__global__ __launch_bounds__(256) void moment_fold_kernel(
+    int64_t n, int images, float* __restrict__ bp, float* __restrict__ out) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    float sum = 0.0f;
+    for (int k = 0; k < images; ++k) {
+      sum += bp[k * n + i];
+      bp[k * n + i] = 0.0f;
+    }
+    out[i] += sum;
+  }
+}
+
 // total += columns of every stored run
 __global__ __launch_bounds__(256) void moment_count_kernel(
     const uint32_t* __restrict__ blocks, int64_t n_lanes,
@@ -1336,6 +1352,8 @@ constexpr double kMergedPairs = 100.0;
 constexpr double kMergedSpan = 6.0;  // columns of a merged task's vertices
 constexpr int kMergedTasks = 4096;   // tasks aimed at, of 8 to 64 groups
 constexpr int kBwdChunk = 1024;  // pairs of a back-projection wavefront's task
+// images that the back-projection adds to (images_for says when)
+constexpr int kMaxImages = 4;
 
 unsigned grid_of(int64_t n) { return (unsigned)((n + 255) / 256); }
 
@@ -1381,6 +1399,21 @@ bool lists_faster(int positions, double pairs, double bins, bool batch) {
   const double moments =
       pairs * 0.07 + bins * 8.0 * std::pow(positions / 24.0, 1.6);
   return moments > lists + 2e4;
+}
+
+// Images that a plan's back-projection adds to.  Every task adds its cells to
+// the image with FP32 atomics, and the running sum rounds at each addition: over
+// k images it does so at a k-th of the size and of the number.  The error of
+// the image derivative of a log-likelihood against 64 bits (both with the FP32
+// support), pixel-by-pixel lists and moments with 1, 2, 4, 8 images:
+//   203 x 56, 96151 events, 330 additions a pixel:
+//     1.9e-7 | 3.2e-7, 2.0e-7, 1.3e-7, 1.2e-7
+//   476 x 197, 329679 events, 180: 1.8e-7 | 2.3e-7, 1.4e-7, 1.0e-7, 1.0e-7
+//   335 x 185, unrolled, 52 (merged): 9.7e-7 | 1.7e-6, 0.9e-6, 0.6e-6, 0.5e-6
+// Few additions need no second image, whose sum and clearing would cost a short
+// list on a large grid more than its own work.
+int images_for(double additions) {
+  return additions < 8.0 ? 1 : additions < 64.0 ? 2 : kMaxImages;
 }
 
 // A dispatch counts its work-items in 32 bits: tasks of one launch.
@@ -1707,15 +1740,13 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   int merged_chunk = 0;
   // Bins of few pairs are back-projected several to a task, whose pixels are
   // summed in LDS first: the atomic additions to the image, 16 x 2 cells per
-  // bin, and their rounding would otherwise outweigh the pairs' own work.  It
+  // bin, would otherwise outweigh the pairs' own work.  It
   // takes enough bins for full tasks, and short lines, as the pixels' LDS comes
   // on top of the cells'.  Back-projection, one bin to a task and merged: 5
   // cells, 2.5 pairs per bin, 15700 bins 0.051 and 0.032 ms; 15 cells, 20 pairs,
   // 27500 bins 0.182 and 0.107 ms, 58 pairs 0.212 and 0.195 ms, 185 pairs 0.35
   // and 0.41 ms; 13 cells, 62 pairs, 7500 bins 0.050 and 0.063 ms; 24 cells, 25
-  // pairs, 31400 bins 0.185 and 0.211 ms.  (The error of the image derivative
-  // of an unrolled run of 67000 events falls from 3.4e-6 to 3.0e-6, of a
-  // log-likelihood over 1e6 events from 6.1e-7 to 3.7e-7.)
+  // pairs, 31400 bins 0.185 and 0.211 ms.
   const double row_step = 0.5 * (R - 1) * (double)g.pixel_height;
   const float max_shear =
       (float)(row_step * ((double)d.nt * 0.5) * (double)d.dt);
@@ -1748,7 +1779,13 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
     BAND_TRY(hipStreamSynchronize(stream));
     merged_chunk = chunk;
   }
+  const int64_t n_pixels = (int64_t)g.n_z * g.n_y;
+  plan.bp_images = images_for(
+      (double)totals[2] * R * (merged ? merged_columns : 2 * d.positions + 1) /
+      (double)n_pixels);
   Arena lists;
+  const size_t o_images =
+      lists.take<float>(plan.bp_images > 1 ? n_pixels * plan.bp_images : 0);
   const size_t o_blocks = lists.take<uint4>((int64_t)n_groups * 64);
   const size_t o_groups = lists.take<MomentGroup>(n_groups);
   const size_t o_fwd = lists.take<MomentTask>(totals[1]);
@@ -1758,6 +1795,12 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
     return give_up();
   }
   char* L = static_cast<char*>(plan.lists);
+  plan.bpT = bpT;
+  if (plan.bp_images > 1) {
+    plan.bpT = reinterpret_cast<float*>(L + o_images);
+    hipLaunchKernelGGL(fill_words_kernel, dim3(1024), dim3(256), 0, stream,
+                       (uint32_t*)plan.bpT, n_pixels * plan.bp_images, 0u);
+  }
   plan.blocks = reinterpret_cast<uint32_t*>(L + o_blocks);
   plan.fwd_tasks = reinterpret_cast<MomentTask*>(L + o_fwd);
   plan.bwd_tasks = reinterpret_cast<MomentTask*>(L + o_bwd);
@@ -1794,7 +1837,8 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   d.groups = groups;
   d.merged_columns = merged_columns;
   d.inv = plan.inv;
-  d.bpT = bpT;
+  d.bpT = plan.bpT;
+  d.bp_images = plan.bp_images;
   MomentInstance both[2] = {d, d};
   for (int c = 0; c < 2; ++c) {
     both[c].rhoT = rhoT[c];
@@ -1854,10 +1898,31 @@ int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
 }
 
 int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
-                    std::string* err, const float* weights, float* into) {
+                    std::string* err) {
   return launch_backward(plan.terms, plan.merged, plan.bwd_lds,
-                         plan.desc + cur, plan.bwd_tasks, plan.n_bwd, weights,
-                         into, stream, err);
+                         plan.desc + cur, plan.bwd_tasks, plan.n_bwd, nullptr,
+                         nullptr, stream, err);
+}
+
+int moment_fold(MomentPlan& plan, float* into, hipStream_t stream,
+                std::string* err) {
+  if (plan.bpT == into) return 0;
+  const int64_t n = (int64_t)plan.inst.g.n_z * plan.inst.g.n_y;
+  hipLaunchKernelGGL(moment_fold_kernel,
+                     dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)),
+                     dim3(256), 0, stream, n, plan.bp_images, plan.bpT, into);
+  BAND_TRY(hipGetLastError());
+  return 0;
+}
+
+int moment_backward_into(MomentPlan& plan, const float* weights, float* into,
+                         hipStream_t stream, std::string* err) {
+  const bool direct = plan.bp_images == 1;
+  if (launch_backward(plan.terms, plan.merged, plan.bwd_lds, plan.desc,
+                      plan.bwd_tasks, plan.n_bwd, weights,
+                      direct ? into : nullptr, stream, err))
+    return -1;
+  return direct ? 0 : moment_fold(plan, into, stream, err);
 }
 
 int moment_gradient(MomentPlan& plan, const float* xT, int stride, float* out,

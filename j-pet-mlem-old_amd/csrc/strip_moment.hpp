@@ -76,7 +76,8 @@ struct MomentInstance {
   float* partial;          // per (band of the record, record)
   const int* counts;       // bands of each record
   float* inv;
-  float* bpT;
+  float* bpT;              // bp_images images, n_pixels apart
+  int bp_images;
   int64_t n_events;
 };
 
@@ -96,6 +97,10 @@ struct MomentPlan {
   uint32_t* blocks = nullptr;
   float* partial = nullptr;
   float* inv = nullptr;
+  // where the back-projection adds: the caller's image, or several images of
+  // the plan's own, zero between uses, whose sum it is
+  float* bpT = nullptr;
+  int bp_images = 1;
   int* counts = nullptr;
   int* order = nullptr;     // record -> caller's event
   MomentTask* fwd_tasks = nullptr;
@@ -121,11 +126,17 @@ int moment_forward(MomentPlan& plan, int cur, hipStream_t stream,
 // D_e = sum of the record's partials; inv (guarded or not) and / or D
 int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
                    hipStream_t stream, std::string* err);
-// (weights in record order and a column-major image of the caller's, or null
-// for the plan's own)
+// Adds to the plan's bpT images, whose sum the caller takes and clears.
 int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
-                    std::string* err, const float* weights = nullptr,
-                    float* into = nullptr);
+                    std::string* err);
+// The same with the caller's weights (record order), added to the column-major
+// image `into`.
+int moment_backward_into(MomentPlan& plan, const float* weights, float* into,
+                         hipStream_t stream, std::string* err);
+// The sum of the plan's images added to `into`, the images cleared (nothing
+// where `into` is where the back-projection adds).
+int moment_fold(MomentPlan& plan, float* into, hipStream_t stream,
+                std::string* err);
 // out[stride * (band of the record * n_events + record) + {0, 1, 2}] = sum K x,
 // sum K x Q, sum K x (w - Qd) of the column-major image xT (strip_adjoint.hip)
 int moment_gradient(MomentPlan& plan, const float* xT, int stride, float* out,
