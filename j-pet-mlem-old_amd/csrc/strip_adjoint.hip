@@ -569,11 +569,14 @@ int band_mlem_adjoint_step(BandPlan& plan, const DeviceGeometry& g,
   hipLaunchKernelGGL(mul_kernel, dim3(pg), dim3(256), 0, stream, n_pixels,
                      gbarT, rhoT_k, hT);
   BAND_TRY(hipGetLastError());
-  if (!bpT_k)
+  // (the moment form puts its sum into an image that the lists add to)
+  const bool add = !plan.moment.ready;
+  if (!bpT_k && add)
     hipLaunchKernelGGL(zero_kernel, dim3(pg), dim3(256), 0, stream, n_pixels,
                        bp1);
-  hipLaunchKernelGGL(zero_kernel, dim3(pg), dim3(256), 0, stream, n_pixels,
-                     bp2);
+  if (add)
+    hipLaunchKernelGGL(zero_kernel, dim3(pg), dim3(256), 0, stream, n_pixels,
+                       bp2);
   BAND_TRY(hipGetLastError());
   double sums[2] = {0.0, 0.0};
   if (n > 0) {
@@ -590,8 +593,8 @@ int band_mlem_adjoint_step(BandPlan& plan, const DeviceGeometry& g,
     if (reduce_sum(wk, gz, n, 0, stream, err) ||
         reduce_sum(wk, gd, n, 1, stream, err))
       return -1;
-    if ((!bpT_k && band_backproject(plan, g, w1, bp1, stream, err)) ||
-        band_backproject(plan, g, w2, bp2, stream, err))
+    if ((!bpT_k && band_backproject(plan, g, w1, bp1, stream, err, add)) ||
+        band_backproject(plan, g, w2, bp2, stream, err, add))
       return -1;
     BAND_TRY(hipMemcpyAsync(sums, wk.sums, sizeof(double) * 2,
                             hipMemcpyDeviceToHost, stream));

@@ -125,14 +125,7 @@ __global__ __launch_bounds__(256) void box_extent_kernel(
     int* __restrict__ extent) {
   int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n) return;
-  const uint2 b = box[e];
-  const uint32_t v = rows ? b.y : b.x;
-  const int lo = (int)(v & 0xffff), hi = (int)(v >> 16);
-  if (!rows || hi <= lo)
-    extent[e] = max(hi - lo, 0);
-  else
-    extent[e] = ((hi + kSpanAlign - 1) & ~(kSpanAlign - 1)) -
-                (lo & ~(kSpanAlign - 1));
+  extent[e] = rows ? box_slot_rows(box[e].y) : box_width(box[e].x);
 }
 
 // spatial order of the events: key = (bbox y0, bbox x0)
@@ -1228,10 +1221,13 @@ int band_prepare_once(BandPlan& plan, const DeviceGeometry& g,
   }
   static std::atomic<int64_t> generations{0};
   plan.generation = ++generations;
+  // widest and tallest clamped bbox (0: not known yet)
+  int max_extent[2] = {0, 0};
   if (plan.tuning.moments && default_tuning(plan.tuning)) {
     bool built = false;
     if (moment_prepare(plan.moment, g, ev, n_events, plan.rhoT, plan.bpT,
-                       plan.tuning.moments == 2, stream, &built, err))
+                       plan.tuning.moments == 2, stream, &built, max_extent,
+                       err))
       return -1;
     if (built) {
       plan.ready = true;
@@ -1240,9 +1236,7 @@ int band_prepare_once(BandPlan& plan, const DeviceGeometry& g,
   }
   const int64_t n = n_events;
   const unsigned blocks = (unsigned)((n + 255) / 256);
-  // widest and tallest clamped bbox
-  int max_extent[2] = {1, 1};
-  if (n > 0) {
+  if (n > 0 && max_extent[0] == 0) {
     int* extent = nullptr;
     int* d_red = nullptr;
     void* tmp = nullptr;
@@ -1261,12 +1255,12 @@ int band_prepare_once(BandPlan& plan, const DeviceGeometry& g,
       BAND_TRY(hipMemcpyAsync(&max_extent[rows], d_red, sizeof(int),
                               hipMemcpyDeviceToHost, stream));
       BAND_TRY(hipStreamSynchronize(stream));
-      max_extent[rows] = std::max(max_extent[rows], 1);
     }
     BAND_TRY(hipFree(tmp));
     BAND_TRY(hipFree(d_red));
     BAND_TRY(hipFree(extent));
   }
+  for (int& extent : max_extent) extent = std::max(extent, 1);
   const int max_width = max_extent[0];
   plan.max_width = max_width;
   // spatial renumbering and packed records
@@ -1592,7 +1586,7 @@ int band_iteration(BandPlan& plan, const DeviceGeometry& g,
       return -1;
     if (t_bwd) BAND_TRY(hipEventRecord(t_bwd, stream));
     // (several plans that add to one image update it together)
-    if (!finalize) return moment_fold(plan.moment, plan.bpT, stream, err);
+    if (!finalize) return moment_fold(plan.moment, plan.bpT, true, stream, err);
     return finalize_from(plan, plan.moment.bpT, plan.moment.bp_images,
                          (int64_t)g.n_z * g.n_y, sensitivity_mode, scale,
                          bp_out, stream, err);
@@ -1666,13 +1660,17 @@ int band_to_row_major(const DeviceGeometry& g, const float* inT, float* out,
 
 int band_backproject(BandPlan& plan, const DeviceGeometry& g,
                      const float* weights, float* outT, hipStream_t stream,
-                     std::string* err) {
+                     std::string* err, bool add) {
   if (!plan.ready) {
     if (err) *err = "band plan not prepared";
     return -1;
   }
   if (plan.moment.ready)
-    return moment_backward_into(plan.moment, weights, outT, stream, err);
+    return moment_backward_into(plan.moment, weights, outT, add, stream, err);
+  if (!add) {
+    if (err) *err = "the row-band lists add to the image";
+    return -1;
+  }
   return dispatch_backward(plan, g, weights, outT, stream, err);
 }
 

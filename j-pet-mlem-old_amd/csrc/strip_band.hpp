@@ -261,10 +261,11 @@ int band_to_row_major(const DeviceGeometry& g, const float* inT, float* out,
                       hipStream_t stream, std::string* err);
 
 // outT (column-major, not cleared) += sum_e K_e * weights[e] over the
-// resident events (weights in record order).
+// resident events (weights in record order).  add = false puts the sum there
+// (moment form only).
 int band_backproject(BandPlan& plan, const DeviceGeometry& g,
                      const float* weights, float* outT, hipStream_t stream,
-                     std::string* err);
+                     std::string* err, bool add = true);
 
 // ---------------------------------------------------------------------------
 // differentiation (strip_adjoint.hip)

@@ -49,6 +49,18 @@ __device__ __forceinline__ void gatomic_add(float* p, float v) {
     }                                                               \
   } while (0)
 
+// A clamped bbox's width, or its rows rounded out to multiples of kSpanAlign
+// (the record's span-table slot); bounds: a box word of either direction.
+__device__ inline int box_width(uint32_t bounds) {
+  return max((int)(bounds >> 16) - (int)(bounds & 0xffff), 0);
+}
+__device__ inline int box_slot_rows(uint32_t bounds) {
+  const int lo = (int)(bounds & 0xffff), hi = (int)(bounds >> 16);
+  if (hi <= lo) return 0;
+  return ((hi + kSpanAlign - 1) & ~(kSpanAlign - 1)) -
+         (lo & ~(kSpanAlign - 1));
+}
+
 // Exact per-row terms of the 3-sigma test (gaussian_kernel.h:131-137):
 // Q(dz) = ((A dy) dy + (B dy) dz) + (C dz) dz, evaluated like the reference.
 __device__ inline void row_terms_exact(float A, float B, float dy,

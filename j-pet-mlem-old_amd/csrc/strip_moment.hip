@@ -152,7 +152,11 @@ __device__ inline void lds_order() {
 struct PlanStats {
   unsigned long long pairs;
   int max_bands;
-  int max_tan;  // bit pattern of a non-negative float
+  int max_tan;        // bit pattern of a non-negative float
+  int max_extent[2];  // widest box, most rows of a span-table slot
+  int max_group[2];   // moment_groups_kernel: two bands, one
+  int status;         // moment_pack_kernel
+  int occupied;       // moment_marked_kernel
 };
 
 __device__ inline int box_bands(const uint2 box) {
@@ -161,43 +165,100 @@ __device__ inline int box_bands(const uint2 box) {
   return (x1 > x0 && y1 > y0) ? (y1 - 1) / R - y0 / R + 1 : 0;
 }
 
+// What the choice between the forms and the sizes of either plan depend on.
 __global__ __launch_bounds__(256) void moment_stats_kernel(
     const uint2* __restrict__ box, const float4* __restrict__ a, int64_t n,
     PlanStats* __restrict__ stats) {
   unsigned long long pairs = 0;
-  int bands = 0;
-  float tan = 0.0f;
+  int most[4] = {0, 0, 0, 0};  // bands, |tan| as bits, box width, slot rows
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
        e += (int64_t)gridDim.x * blockDim.x) {
-    const int c = box_bands(box[e]);
+    const uint2 b = box[e];
+    const int c = box_bands(b);
     pairs += (unsigned long long)c;
-    bands = max(bands, c);
+    most[0] = max(most[0], c);
+    most[2] = max(most[2], box_width(b.x));
+    most[3] = max(most[3], box_slot_rows(b.y));
     // (a NaN stays out: such an event's box is empty or its bin is clamped)
-    if (c) tan = fmaxf(tan, fabsf(a[e].z));
+    if (c)
+      most[1] =
+          max(most[1], __builtin_bit_cast(int, fmaxf(0.0f, fabsf(a[e].z))));
   }
   for (int o = 32; o > 0; o >>= 1) {
     pairs += __shfl_xor(pairs, o);
-    bands = max(bands, __shfl_xor(bands, o));
-    tan = fmaxf(tan, __shfl_xor(tan, o));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) most[i] = max(most[i], __shfl_xor(most[i], o));
   }
   __shared__ unsigned long long sp[4];
-  __shared__ int sb[4], st[4];
+  __shared__ int sm[4][4];
   if ((threadIdx.x & 63) == 0) {
     const int w = threadIdx.x >> 6;
     sp[w] = pairs;
-    sb[w] = bands;
-    st[w] = __builtin_bit_cast(int, tan);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sm[w][i] = most[i];
   }
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 4; ++w) {
       pairs += sp[w];
-      bands = max(bands, sb[w]);
-      st[0] = max(st[0], st[w]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) most[i] = max(most[i], sm[w][i]);
     }
     atomicAdd(&stats->pairs, pairs);
-    atomicMax(&stats->max_bands, bands);
-    atomicMax(&stats->max_tan, st[0]);
+    atomicMax(&stats->max_bands, most[0]);
+    atomicMax(&stats->max_tan, most[1]);
+    atomicMax(&stats->max_extent[0], most[2]);
+    atomicMax(&stats->max_extent[1], most[3]);
+  }
+}
+
+// The most pairs, among every step-th event's, of a group that the row-band
+// lists cut their tasks from: a band (two for the forward lists) and the bucket
+// of columns in which a pair's runs begin, about half_run columns and the line's
+// shear over half a band left of the vertex.  One workgroup counts them in LDS
+// (in global memory the additions to the same few words, from all over the card,
+// take 0.1 to 0.5 ms); grids of more groups than kGroupWords share words.
+constexpr int kBucket = 8;
+constexpr int kGroupWords = 1 << 14;
+constexpr int kSampled = 1 << 12;
+
+__global__ __launch_bounds__(1024) void moment_groups_kernel(
+    DeviceGeometry g, const uint2* __restrict__ box,
+    const float4* __restrict__ a, int64_t n, int64_t step, int buckets,
+    int words, float half_run, PlanStats* __restrict__ stats) {
+  __shared__ int group[kGroupWords];
+  for (int i = threadIdx.x; i < words; i += 1024) group[i] = 0;
+  __syncthreads();
+  for (int64_t e = threadIdx.x * step; e < n; e += 1024 * step) {
+    const uint2 b = box[e];
+    const int c = box_bands(b);
+    if (!c) continue;
+    const float4 ev = a[e];  // z, y, tan
+    const float shear = 0.5f * R * g.pixel_height * ev.z;
+    const float lo = (float)(b.x & 0xffff), hi = (float)(b.x >> 16) - 1.0f;
+    for (int k = 0; k < c; ++k) {
+      const int band = (int)(b.y & 0xffff) / R + k;
+      const float y = g.tl_y_half_h - ((float)band + 0.5f) * R * g.pixel_height;
+      const float z = ev.x + ev.z * (y - ev.y) - fabsf(shear) - g.tl_z_half_w;
+      const float col = fminf(fmaxf(z * g.inv_pixel_width - half_run, lo), hi);
+      atomicAdd(&group[(band * buckets + (int)col / kBucket) % words], 1);
+    }
+  }
+  __syncthreads();
+  int two = 0, one = 0;
+  for (int i = threadIdx.x; i < words; i += 1024) {
+    const int c = group[i];
+    const int next = i + buckets < words ? group[i + buckets] : 0;
+    one = max(one, c);
+    if (!(i / buckets & 1)) two = max(two, c + next);
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    two = max(two, __shfl_xor(two, o));
+    one = max(one, __shfl_xor(one, o));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicMax(&stats->max_group[0], two);
+    atomicMax(&stats->max_group[1], one);
   }
 }
 
@@ -1304,9 +1365,10 @@ __global__ __launch_bounds__(64) void moment_backward_kernel(
   }
 }
 
-// out += the sum of the images, which are cleared
+// out = or += the sum of the images, which are cleared
 __global__ __launch_bounds__(256) void moment_fold_kernel(
-    int64_t n, int images, float* __restrict__ bp, float* __restrict__ out) {
+    int64_t n, int images, int add, float* __restrict__ bp,
+    float* __restrict__ out) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     float sum = 0.0f;
@@ -1314,7 +1376,7 @@ __global__ __launch_bounds__(256) void moment_fold_kernel(
       sum += bp[k * n + i];
       bp[k * n + i] = 0.0f;
     }
-    out[i] += sum;
+    out[i] = add ? out[i] + sum : sum;
   }
 }
 
@@ -1373,32 +1435,66 @@ size_t table_bytes(int positions, int terms) {
          (2 * (size_t)(positions + 1) * R * terms + (terms == 6 ? 32 : 0));
 }
 
-// Whether the row-band lists do an iteration in clearly less time (20 us) than
-// the moment form.  Where the bins hold few pairs, tabulating and expanding
-// their lines costs more than walking the runs' pixels, and more so the more
-// cells a line has (its LDS leaves fewer wavefronts to a CU).  Times in ns, fitted
-// to the ones below within a third; the lists' 0.2 ms is the chain of their
-// largest tasks, which events spread over a bin each do not have.  Measured
-// (cells, pairs, occupied bins: lists, moments):
-//   7, 1.8e6, 4.8e5: 0.40, 0.85 ms      13, 3.1e4, 2.6e4: 0.06, 0.12 ms
-//   14, 1.5e6, 5.8e4: 0.49, 0.36 ms     24, 2.2e5, 6.5e4: 0.25, 0.56 ms
-//   24, 8.2e6, 1.2e5: 2.17, 1.65 ms     34, 3.2e6, 5.8e4: 1.33, 1.14 ms
-//   48, 1.4e6, 5.2e4: 0.91, 1.37 ms     48, 1.4e7, 1.2e5: 5.27, 4.53 ms
-//   66, 6.4e5, 2.0e4: 0.77, 1.04 ms     66, 4.2e6, 2.2e4: 4.20, 1.70 ms
-// In a batch the members' tasks share the card, so nobody waits for that chain,
+// Whether back-projection tasks hold several bins (of 8 terms).
+bool merge_bins(int positions, double pairs, double bins) {
+  return positions <= kMergedPositions && bins >= kMergedBins &&
+         pairs < kMergedPairs * bins;
+}
+
+// What the time of an iteration in either form depends on.
+struct FormSizes {
+  int positions;
+  double pairs;
+  double fwd_group, bwd_group;  // most pairs of a list task
+  double slope;                 // largest |tan|, columns per row
+  bool wide;                    // no span table for the lists
+  double pixels;
+};
+
+// Whether the row-band lists do an iteration in less time than the moment form.
+// Where the bins hold few pairs, tabulating and expanding their lines costs more
+// than walking the runs' pixels, and more so the more cells a line has: it takes
+// longer, and its LDS leaves fewer wavefronts to a CU.  The lists take as long as
+// all their pairs at full throughput or as the chains of their largest tasks,
+// which are short where events are few to a band and bucket.  Times in us, fitted
+// to 1790 contexts (20 to 1600 by 24 to 800 pixels of 0.5 to 2.5 mm, sigma_z 5 to
+// 14 mm, 3 to 1e6 events); for 1690 others, at 5 and 95 %, the lists' lie at 0.87
+// and 1.19 of those measured and the moments' at 0.86 and 1.14.  There the moment
+// form is taken 1236 times, 17 times where it is more than 3 % slower (at most
+// 1.18 times), and the lists where they are more than 10 % slower 8 times (at
+// most 1.48 times).  Some of them (cells, pairs, occupied bins: lists, moments):
+//   24, 3997, 3335: 25, 60 us            57, 1022, 683: 26, 58 us
+//   32, 1.2e5, 1.8e4: 189, 311 us        17, 1.8e5, 4.2e4: 237, 338 us
+//   45, 9056, 589: 420, 29 us            24, 1.2e6, 3.4e4: 488, 375 us
+//   13, 9.5e5, 5.2e4: 323, 256 us        24, 2.9e6, 8.5e4: 3433, 1025 us (wide)
+// The moment form's plan is made in half to a third of the time of the lists':
+// it is taken where the two are alike, on the shortest lines too, where a few
+// events take either form the time of four launches.
+// In a batch the members' tasks share the card, so nobody waits for the chains,
 // and the moment form has to be a seventh faster.  24 members of 1e4 to 3e5 events,
 // whose bins hold 2 to 186 pairs, ten iterations with all copies: 27.4 ms on the
 // lists, 43.1 ms with 22 members in the moment form, 26.0 ms with this rule.
-bool lists_faster(int positions, double pairs, double bins, bool batch) {
+bool lists_faster(const FormSizes& s, double bins, bool batch) {
+  const double P = s.positions;
   if (batch)
-    return 1.15 * (pairs * 0.07 + bins * 8.0 * std::pow(positions / 24.0, 1.6)) >
-           pairs * (0.04 + 0.0065 * positions);
-  const double chain =
-      2e5 * std::min({1.0, pairs / 1e5, std::max(pairs / bins - 1.0, 0.0)});
-  const double lists = chain + pairs * (0.04 + 0.0075 * positions);
-  const double moments =
-      pairs * 0.07 + bins * 8.0 * std::pow(positions / 24.0, 1.6);
-  return moments > lists + 2e4;
+    return 1.15 * (s.pairs * 0.07 + bins * 8.0 * std::pow(P / 24.0, 1.6)) >
+           s.pairs * (0.04 + 0.0065 * P);
+  const double wide = s.wide ? 2.08 : 1.0;
+  const double line = std::max(P - 7.0, 0.0);
+  const double chain = (s.fwd_group * (0.0333 + 0.00343 * P) +
+                        s.bwd_group * 0.00623 * (P + 8.0 * s.slope)) * wide;
+  const double work = s.pairs * (1.015e-4 + 6.28e-6 * P) * wide;
+  const double lists = 12.4 + 0.0925 * line + 5.92e-6 * s.pixels +
+                       std::hypot(chain, work);
+  // a bin's line at the wavefronts that its cells leave room for; the chain of
+  // the fullest bin
+  const double room = std::max(std::floor(160.0 / (P + 1.0)), 1.0);
+  const double per_bin = (0.0378 + 8.67e-4 * P) / room *
+                         (merge_bins(s.positions, s.pairs, bins) ? 0.79 : 1.0);
+  const double one = 0.298 * line + 0.085 * std::min(4.0 * s.pairs / bins, 1024.0);
+  const double all = bins * per_bin + s.pairs * (5.35e-5 + 1.15e-6 * P);
+  const double moments = 12.4 + 7.73e-6 * s.pixels + std::hypot(one, all);
+  return moments > (lists > 60.0 || P <= 7.0 ? 1.05 : 0.95) * lists;
 }
 
 // Images that a plan's back-projection adds to.  Every task adds its cells to
@@ -1494,7 +1590,7 @@ void moment_release(MomentPlan& plan) {
 int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
                    const EventSoA& ev, int64_t n, float* const rhoT[2],
                    float* bpT, bool batch, hipStream_t stream, bool* built,
-                   std::string* err) {
+                   int max_extent[2], std::string* err) {
   *built = false;
   moment_release(plan);
   if (n <= 0 || n > 0x3fffffff || !moment_supported(g)) return 0;
@@ -1504,20 +1600,33 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
       if (p) (void)hipFree(p);
     }
   } stats_mem, temp;
-  // what the sizes of the plan depend on
-  BAND_TRY(hipMalloc(&stats_mem.p, sizeof(PlanStats) + 64));
+  // what the choice and the sizes of the plan depend on
+  const int n_bands = (g.n_y + R - 1) / R;
+  const int buckets = (g.n_z + kBucket - 1) / kBucket;
+  const int64_t step = (n + kSampled - 1) / kSampled;
+  const double sigma = 1.0 / std::sqrt((double)g.inv_pow_sigma_z);
+  if (hipMalloc(&stats_mem.p, sizeof(PlanStats)) != hipSuccess) {
+    stats_mem.p = nullptr;
+    (void)hipGetLastError();
+    return 0;
+  }
   PlanStats* d_stats = static_cast<PlanStats*>(stats_mem.p);
   hipLaunchKernelGGL(fill_words_kernel, dim3(1), dim3(256), 0, stream,
-                     (uint32_t*)d_stats, (int64_t)((sizeof(PlanStats) + 64) / 4),
-                     0u);
+                     (uint32_t*)d_stats, (int64_t)(sizeof(PlanStats) / 4), 0u);
   hipLaunchKernelGGL(moment_stats_kernel,
                      dim3(std::min<unsigned>(grid_of(n), 1024)), dim3(256), 0,
                      stream, ev.box, ev.a, n, d_stats);
+  if (!batch)
+    hipLaunchKernelGGL(moment_groups_kernel, dim3(1), dim3(1024), 0, stream, g,
+                       ev.box, ev.a, n, step, buckets,
+                       std::min(n_bands * buckets, kGroupWords),
+                       (float)(kRunHalf * sigma / g.pixel_width), d_stats);
   BAND_TRY(hipGetLastError());
   PlanStats st{};
   BAND_TRY(hipMemcpyAsync(&st, d_stats, sizeof(st), hipMemcpyDeviceToHost,
                           stream));
   BAND_TRY(hipStreamSynchronize(stream));
+  for (int i = 0; i < 2; ++i) max_extent[i] = std::max(st.max_extent[i], 1);
   const int64_t n_pairs = (int64_t)st.pairs;
   const double max_tan = (double)__builtin_bit_cast(float, st.max_tan);
   if (n_pairs <= 0 || n_pairs > 0x3fffffff || !(max_tan < 1e3) ||
@@ -1525,11 +1634,9 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
     return 0;
 
   // bins: half the reach for the vertex, half for the shear over a band
-  const double sigma = 1.0 / std::sqrt((double)g.inv_pow_sigma_z);
   const double iz = g.inv_pow_sigma_z, id = g.inv_pow_sigma_dl;
   const double k = 8.0 * iz * id / (4.0 * id + 2.0 * iz);
   const double half_width = 3.0 / std::sqrt(k);
-  const int n_bands = (g.n_y + R - 1) / R;
   MomentInstance d{};
   d.g = g;
   d.max_bands = std::max(st.max_bands, 1);
@@ -1578,9 +1685,19 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   }
   const int n_bins = d.nx * d.nt * n_bands;
 
-  // Only where the occupied bins can make the lists the faster form are they
-  // counted, before anything is sorted.
-  if (lists_faster(d.positions, (double)n_pairs, (double)n_bins, batch)) {
+  // Only where the occupied bins decide it are they counted, before anything is
+  // sorted.
+  const FormSizes sizes{
+      d.positions,
+      (double)n_pairs,
+      std::min((double)(st.max_group[0] * step), 2048.0),
+      std::min((double)(st.max_group[1] * step), 512.0),
+      max_tan * (double)g.pixel_height / (double)g.pixel_width,
+      st.max_extent[0] > 255,
+      (double)g.n_z * g.n_y};
+  if (lists_faster(sizes, (double)std::min<int64_t>(n_bins, n_pairs), batch)) {
+    // (a few pairs lie in nearly as many bins)
+    if (n_pairs <= 256) return 0;
     Scratch marks;
     const int n_words = (n_bins + 3) / 4;
     if (hipMalloc(&marks.p, sizeof(uint32_t) * (size_t)n_words) !=
@@ -1593,16 +1710,14 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
                        (uint32_t*)marks.p, (int64_t)n_words, 0u);
     hipLaunchKernelGGL(moment_mark_kernel, dim3(grid_of(n)), dim3(256), 0,
                        stream, d, ev.box, ev.a, n, (uint8_t*)marks.p);
-    int* d_total = reinterpret_cast<int*>(d_stats + 1) + 1;
     hipLaunchKernelGGL(moment_marked_kernel, dim3(256), dim3(256), 0, stream,
-                       (const uint32_t*)marks.p, n_words, d_total);
+                       (const uint32_t*)marks.p, n_words, &d_stats->occupied);
     BAND_TRY(hipGetLastError());
     int occupied = 0;
-    BAND_TRY(hipMemcpyAsync(&occupied, d_total, sizeof(int),
+    BAND_TRY(hipMemcpyAsync(&occupied, &d_stats->occupied, sizeof(int),
                             hipMemcpyDeviceToHost, stream));
     BAND_TRY(hipStreamSynchronize(stream));
-    if (lists_faster(d.positions, (double)n_pairs, (double)occupied, batch))
-      return 0;
+    if (lists_faster(sizes, (double)occupied, batch)) return 0;
   }
 
   // what building the plan needs
@@ -1759,9 +1874,8 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
       g.n_z + 2 * d.positions);
   const size_t merged_bytes = sizeof(float) * R * (size_t)merged_columns;
   const bool merged =
-      terms == 8 && d.positions <= kMergedPositions &&
-      totals[1] >= kMergedBins &&
-      (double)n_pairs < kMergedPairs * (double)totals[1] &&
+      terms == 8 &&
+      merge_bins(d.positions, (double)n_pairs, (double)totals[1]) &&
       table_bytes(d.positions, terms) + merged_bytes <= kLds;
   const int n_x_blocks = (d.nx + x_block - 1) / x_block;
   const int n_blocks = n_bands * n_x_blocks;
@@ -1820,7 +1934,7 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
                        dim3(256), 0, stream, d, pieces[0], n_blocks, x_block,
                        n_x_blocks, merged_chunk, max_shear, pieces[2],
                        plan.bwd_tasks);
-  int* d_status = reinterpret_cast<int*>(d_stats + 1);
+  int* d_status = &d_stats->status;
   hipLaunchKernelGGL(moment_pack_kernel,
                      dim3((unsigned)std::min(n_groups, 1 << 20)), dim3(256), 0,
                      stream, d, rec, groups, group_pair, vb.Current(),
@@ -1904,25 +2018,30 @@ int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
                          nullptr, stream, err);
 }
 
-int moment_fold(MomentPlan& plan, float* into, hipStream_t stream,
+int moment_fold(MomentPlan& plan, float* into, bool add, hipStream_t stream,
                 std::string* err) {
   if (plan.bpT == into) return 0;
   const int64_t n = (int64_t)plan.inst.g.n_z * plan.inst.g.n_y;
   hipLaunchKernelGGL(moment_fold_kernel,
                      dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)),
-                     dim3(256), 0, stream, n, plan.bp_images, plan.bpT, into);
+                     dim3(256), 0, stream, n, plan.bp_images, add ? 1 : 0,
+                     plan.bpT, into);
   BAND_TRY(hipGetLastError());
   return 0;
 }
 
 int moment_backward_into(MomentPlan& plan, const float* weights, float* into,
-                         hipStream_t stream, std::string* err) {
+                         bool add, hipStream_t stream, std::string* err) {
   const bool direct = plan.bp_images == 1;
+  if (direct && !add)
+    hipLaunchKernelGGL(
+        fill_words_kernel, dim3(1024), dim3(256), 0, stream, (uint32_t*)into,
+        (int64_t)plan.inst.g.n_z * plan.inst.g.n_y, 0u);
   if (launch_backward(plan.terms, plan.merged, plan.bwd_lds, plan.desc,
                       plan.bwd_tasks, plan.n_bwd, weights,
                       direct ? into : nullptr, stream, err))
     return -1;
-  return direct ? 0 : moment_fold(plan, into, stream, err);
+  return direct ? 0 : moment_fold(plan, into, add, stream, err);
 }
 
 int moment_gradient(MomentPlan& plan, const float* xT, int stride, float* out,

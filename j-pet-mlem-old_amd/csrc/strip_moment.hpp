@@ -113,11 +113,13 @@ bool moment_supported(const DeviceGeometry& g);
 
 // Builds the plan for the events.  *built = false (and 0) where the row-band
 // lists are the better choice (batch: among the members of a batch) or the plan
-// does not fit.
+// does not fit.  max_extent: the widest clamped bbox and the most rows of a
+// span-table slot, for the lists' plan; left alone where the events were not
+// looked at.
 int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
                    const EventSoA& ev, int64_t n_events, float* const rhoT[2],
                    float* bpT, bool batch, hipStream_t stream, bool* built,
-                   std::string* err);
+                   int max_extent[2], std::string* err);
 void moment_release(MomentPlan& plan);
 
 // The passes of an iteration reading image `cur`.
@@ -130,12 +132,12 @@ int moment_inverse(MomentPlan& plan, int guard, float* inv, float* denominators,
 int moment_backward(MomentPlan& plan, int cur, hipStream_t stream,
                     std::string* err);
 // The same with the caller's weights (record order), added to the column-major
-// image `into`.
+// image `into`, or put there.
 int moment_backward_into(MomentPlan& plan, const float* weights, float* into,
-                         hipStream_t stream, std::string* err);
-// The sum of the plan's images added to `into`, the images cleared (nothing
-// where `into` is where the back-projection adds).
-int moment_fold(MomentPlan& plan, float* into, hipStream_t stream,
+                         bool add, hipStream_t stream, std::string* err);
+// The sum of the plan's images added to `into`, or put there, and the images
+// cleared (nothing where `into` is where the back-projection adds).
+int moment_fold(MomentPlan& plan, float* into, bool add, hipStream_t stream,
                 std::string* err);
 // out[stride * (band of the record * n_events + record) + {0, 1, 2}] = sum K x,
 // sum K x Q, sum K x (w - Qd) of the column-major image xT (strip_adjoint.hip)

@@ -111,6 +111,36 @@ def test_moment_form_non_finite_pixels(pystrip_mod, phantom_mod, oracle_mod):
         assert np.max(np.abs(out[1][nz] - out[0][nz]) / out[0][nz]) < 1e-5
 
 
+# n_z, n_y, pixel, body half sizes, R, L, events, whether the moment form is the
+# faster one (an iteration over the lists and in the moment form, us); all of
+# them far from where the two are alike
+CHOICES = {
+    "few events, long lines": (512, 512, 1.0, 200.0, 200.0, 350.0, 700.0, 300,
+                               False),  # 20, 35
+    "spread events, long lines": (512, 512, 1.0, 200.0, 200.0, 350.0, 700.0,
+                                  10_000, False),  # 67, 202
+    "dense events, long lines": (512, 512, 1.0, 200.0, 200.0, 350.0, 700.0,
+                                 300_000, True),  # 808, 445
+    "short lines": (256, 160, 2.0, 80.0, 60.0, 350.0, 500.0, 3_000,
+                    True),  # 105, 34
+    "the shortest lines, one event": (61, 37, 5.0, 100.0, 60.0, 250.0, 700.0,
+                                      1, True),  # 12, 12; the shorter plan
+}
+
+
+@pytest.mark.parametrize("name", list(CHOICES))
+def test_choice_of_the_faster_form(pystrip_mod, phantom_mod, name):
+    print_case("choice of the form:", name)
+    n_z, n_y, w, a, b, R, L, n, moments = CHOICES[name]
+    ev = phantom_mod.generate_events([phantom_mod.Ellipse(0, 0, a, b, 0, 1)],
+                                     R, L, 10.0, 42.0, n, seed=7,
+                                     batch=1 << 16)
+    rec = pystrip_mod.Reconstruction(
+        pystrip_mod.Geometry.make(R, L, n_z, n_y, w, 10.0, 42.0))
+    rec.set_events(ev)
+    assert rec.plan_forms() == ((1, 0) if moments else (0, 1))
+
+
 def test_moment_form_knobs(pystrip_mod, phantom_mod, oracle_mod):
     # leaving a knob's default takes the lists, returning to it the moment
     # form again: the same reconstruction within rounding
