@@ -94,6 +94,7 @@ struct ModeFlags {
   int kernel;       // 0 gaussian, 1 analytic
   int sensitivity;  // 0 none, 1 denominator, 2 numerator
   int guard_zero;
+  int bp_images;  // images of the generic pass's back-projection
 };
 
 // Bounding-box wavefront kernel ("bbox" algorithm): one wave64 per event,
@@ -103,8 +104,8 @@ struct ModeFlags {
 // back-projection image with L2 float atomics.
 //  FAST = true: Gaussian kernel, no sensitivity, guarded inverse (CPU
 //  parity mode) with the row-hoisted prefactor and hardware exp2.
-//  FAST = false: generic semantics (legacy --gpu mode and variants), pass 1
-//  only (generic_event_kernel is their full pass).
+//  FAST = false: generic semantics (legacy --gpu mode and variants); their
+//  back-projection may go to several images (bp_images).
 template <bool FAST, bool BACKPROJECT>
 __global__ __launch_bounds__(256) void bbox_event_kernel(
     DeviceGeometry g, ModeFlags m, const float4* __restrict__ ev_a,
@@ -112,11 +113,12 @@ __global__ __launch_bounds__(256) void bbox_event_kernel(
     int64_t n_events, const float* __restrict__ rho,
     const float* __restrict__ sens, float* __restrict__ bp,
     float* __restrict__ denominators) {
-  static_assert(FAST || !BACKPROJECT, "generic_event_kernel");
   const int lane = threadIdx.x & 63;
   const int64_t waves_per_block = blockDim.x >> 6;
   const int64_t n_waves = (int64_t)gridDim.x * waves_per_block;
   const bool legacy_split = !FAST && m.kernel == 1;
+  if (!FAST && BACKPROJECT)
+    bp += (int64_t)(blockIdx.x % (unsigned)m.bp_images) * g.n_z * g.n_y;
   for (int64_t e = (int64_t)blockIdx.x * waves_per_block + (threadIdx.x >> 6);
        e < n_events; e += n_waves) {
     const float4 a = ev_a[e];
@@ -168,52 +170,62 @@ __global__ __launch_bounds__(256) void bbox_event_kernel(
       if (lane == 0) denominators[e] = d;
       continue;
     }
-    const float inv = (d > 0.0f) ? 1.0f / d : 0.0f;
+    float inv;
+    if (FAST || m.guard_zero)
+      inv = (d > 0.0f) ? 1.0f / d : 0.0f;
+    else
+      inv = 1.0f / d;
 
     for (int idx = lane; idx < n; idx += 64) {
-      const int r = idx / width, c = idx - r * width;
+      int r, c;
+      if (legacy_split) {
+        r = (int)(short)(int)((float)idx * inv_width_f);
+        c = idx - width * r;
+      } else {
+        r = idx / width;
+        c = idx - r * width;
+      }
       const int ix = x0 + c, iy = y0 + r;
+      // the float split can step one column outside the bbox; keep every
+      // access inside the image
+      if (!FAST && (ix < 0 || ix >= g.n_z || iy >= g.n_y)) continue;
       const float dz = pixel_center_z(g, ix) - z;
       const float dy = pixel_center_y(g, iy) - y;
       const float q = ellipse_q_exact(b.x, b.y, b.z, dy, dz);
       if (q <= 9.0f) {
         const int p = iy * g.n_z + ix;
-        const float k =
-            gauss_row_prefactor(g, dy + y, tan, sec) * gauss_exp(q);
+        float k;
+        if (FAST || m.kernel == 0)
+          k = gauss_row_prefactor(g, dy + y, tan, sec) * gauss_exp(q);
+        else
+          k = analytic_kernel(g, y, tan, sec, dz, dy);
         unsafeAtomicAdd(&bp[p], k * inv);
       }
     }
   }
 }
 
+// The same for the analytic kernel where boxes are small: K is kept in LDS
+// between the passes (the first kBboxCache pixels of a box; further ones are
+// evaluated again).  Its 32 KB leave 20 wavefronts to a CU in workgroups of
+// four.  Legacy semantics, 1e5 events on one image, K evaluated twice and kept:
+// boxes of 900 pixels 1.33 and 1.26 ms, 1400 pixels 1.26 and 1.18 ms, 2350 pixels
+// 1.84 and 1.93 ms, 5300 pixels 3.98 and 4.54 ms (workgroups of one wavefront: 5.3
+// and 12.7 ms).  With the Gaussian kernel, which costs less than its place in LDS,
+// 900 pixels 1.24 and 1.25 ms, 5300 pixels 2.45 and 3.64 ms.
 constexpr int kBboxCache = 2048;
-// Copies of the back-projection image, for modes that only this kernel serves:
-// workgroups go round the eight XCDs, so each copy is added to from one of
-// them and its lines stay in that XCD's L2.  At most 128 MB.
-constexpr int kBpCopies = 8;
-constexpr int kBpCopiesPixels = 1 << 22;
-
-// The generic semantics' event pass (legacy --gpu mode and variants).  K is kept
-// in LDS between the passes (the first kBboxCache pixels of the bbox; further
-// ones are evaluated again).  Bound by the atomic additions: legacy semantics,
-// 1e5 events, 256 x 160 at 2 mm 1.25 ms per iteration with K evaluated twice and
-// one image, 1.18 ms with K kept, 0.94 ms with kBpCopies images (0.75 ms
-// without any addition).
-__global__ __launch_bounds__(256) void generic_event_kernel(
+__global__ __launch_bounds__(256) void kept_event_kernel(
     DeviceGeometry g, ModeFlags m, const float4* __restrict__ ev_a,
     const float4* __restrict__ ev_b, const uint2* __restrict__ ev_box,
     int64_t n_events, const float* __restrict__ rho,
-    const float* __restrict__ sens, float* __restrict__ bp,
-    int bp_copies) {
+    const float* __restrict__ sens, float* __restrict__ bp) {
   __shared__ float cache[4 * kBboxCache];
   const int lane = threadIdx.x & 63;
   float* const kept = cache + (threadIdx.x >> 6) * kBboxCache;
-  const int64_t waves_per_block = blockDim.x >> 6;
-  const int64_t n_waves = (int64_t)gridDim.x * waves_per_block;
-  const bool legacy_split = m.kernel == 1;
-  bp += (int64_t)(blockIdx.x % bp_copies) * g.n_z * g.n_y;
-  for (int64_t e = (int64_t)blockIdx.x * waves_per_block + (threadIdx.x >> 6);
-       e < n_events; e += n_waves) {
+  const int64_t n_waves = (int64_t)gridDim.x * 4;
+  bp += (int64_t)(blockIdx.x % (unsigned)m.bp_images) * g.n_z * g.n_y;
+  for (int64_t e = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); e < n_events;
+       e += n_waves) {
     const float4 a = ev_a[e];
     const float4 b = ev_b[e];
     const uint2 box = ev_box[e];
@@ -225,19 +237,12 @@ __global__ __launch_bounds__(256) void generic_event_kernel(
     const float z = a.x, y = a.y, tan = a.z, sec = a.w;
     const float inv_width_f = 1.0f / (float)width;
 
-    // the pixel of bbox index idx, or -1 outside the image (the float split
-    // can step one column outside the bbox)
+    // the pixel of bbox index idx (warp_granularity.cuh:162-176, float
+    // reciprocal row split), or -1 outside the image: the split can step one
+    // column outside the bbox
     auto pixel = [&](int idx, int& ix, int& iy) {
-      int r, c;
-      if (legacy_split) {
-        // warp_granularity.cuh:162-176 (float reciprocal row split)
-        r = (int)(short)(int)((float)idx * inv_width_f);
-        c = idx - width * r;
-      } else {
-        r = idx / width;
-        c = idx - r * width;
-      }
-      ix = x0 + c;
+      const int r = (int)(short)(int)((float)idx * inv_width_f);
+      ix = x0 + idx - width * r;
       iy = y0 + r;
       if (ix < 0 || ix >= g.n_z || iy >= g.n_y) return -1;
       return iy * g.n_z + ix;
@@ -248,9 +253,7 @@ __global__ __launch_bounds__(256) void generic_event_kernel(
       const float dy = pixel_center_y(g, iy) - y;
       const float q = ellipse_q_exact(b.x, b.y, b.z, dy, dz);
       if (!(q <= 9.0f)) return -1.0f;
-      return m.kernel == 0
-                 ? gauss_row_prefactor(g, dy + y, tan, sec) * gauss_exp(q)
-                 : analytic_kernel(g, y, tan, sec, dz, dy);
+      return analytic_kernel(g, y, tan, sec, dz, dy);
     };
 
     float acc = 0.0f;
@@ -287,18 +290,31 @@ __global__ __launch_bounds__(256) void generic_event_kernel(
   }
 }
 
+// Images that the generic event pass adds to: workgroups go round the XCDs, so
+// that an image is added to from two of them and its lines wander less.  Legacy
+// and Gaussian with sensitivity, one, four and eight images: 1e5 events, 256 x 160
+// 1.18, 0.91, 0.92 and 1.19, 0.79, 0.81 ms; 1000 x 1000 3.89, 3.90, 3.90 and
+// 3.22, 2.84, 2.74 ms.  Summing and clearing them costs a short list more than
+// they give: 256 x 160, 100 and 1000 events 35.6, 36.4 and 37.1, 37.1 us; 1000 x
+// 1000, 1000 and 8000 events 155, 167 and 388, 389 us; 2000 x 2000, 8000 and
+// 30000 events 1.34, 1.36 and 4.20, 4.21 ms.  So from one event to 128 pixels, and
+// to 2^22 pixels (64 MB).
+constexpr int kBpImages = 4;
+constexpr int kBpImagesPixels = 1 << 22;
+constexpr int64_t kBpImagesPerEvent = 128;
+
 // rho'(p) = rho(p) * bp(p) [/ s(p) in numerator mode]; clears bp for the
 // next iteration (a fill kernel rather than hipMemsetAsync, so iterations can
 // be captured in a HIP graph).
 __global__ __launch_bounds__(256) void finalize_kernel(
     int n_pixels, const float* __restrict__ rho, float* __restrict__ bp,
-    int bp_copies, const float* __restrict__ sens, int divide_by_sens,
+    int bp_images, const float* __restrict__ sens, int divide_by_sens,
     float* __restrict__ rho_next) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n_pixels;
        i += gridDim.x * blockDim.x) {
     float sum = bp[i];
     bp[i] = 0.0f;
-    for (int c = 1; c < bp_copies; ++c) {
+    for (int c = 1; c < bp_images; ++c) {
       float* const at = bp + (int64_t)c * n_pixels + i;
       sum += *at;
       *at = 0.0f;
@@ -411,7 +427,10 @@ struct strip_mlem_ctx {
   float* rho[2] = {nullptr, nullptr};
   int cur = 0;
   float* bp = nullptr;
-  int bp_copies = 1;  // of bp, n_pixels apart (generic_event_kernel)
+  // images at bp, n_pixels apart and zero between iterations; false once more
+  // of them did not fit
+  int bp_allocated = 1;
+  bool bp_more = true;
   float* sens = nullptr;  // map used by the mode (only when it needs one)
   float* sens_out = nullptr;  // scratch for strip_mlem_get_sensitivity
   float* staging = nullptr;   // AoS staging for host uploads
@@ -638,25 +657,69 @@ int upload_events(strip_mlem_ctx* ctx, const float* responses, int64_t offset,
 }
 
 ModeFlags mode_flags(const strip_mlem_mode& m) {
-  return ModeFlags{m.kernel, m.sensitivity, m.guard_zero};
+  return ModeFlags{m.kernel, m.sensitivity, m.guard_zero, 1};
+}
+
+int fill(strip_mlem_ctx* ctx, float* ptr, int64_t n, float value);
+
+// Images the generic event pass adds to, allocated here when they are first
+// wanted, with the events or in the first pass on them (where they do not fit,
+// one serves as well).
+int bp_images(strip_mlem_ctx* ctx, int* images) {
+  *images = 1;
+  if ((ctx->mode.kernel == 0 && ctx->mode.sensitivity != 1) ||
+      ctx->n_pixels > kBpImagesPixels ||
+      ctx->n_events * kBpImagesPerEvent < ctx->n_pixels)
+    return STRIP_MLEM_OK;
+  if (ctx->bp_allocated < kBpImages && ctx->bp_more) {
+    float* more = nullptr;
+    const int64_t n = (int64_t)kBpImages * ctx->n_pixels;
+    if (hipMalloc(&more, sizeof(float) * n) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->bp_more = false;
+      return STRIP_MLEM_OK;
+    }
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    (void)hipFree(ctx->bp);
+    ctx->bp = more;
+    ctx->bp_allocated = kBpImages;
+    int rc = fill(ctx, ctx->bp, n, 0.0f);
+    if (rc) return rc;
+  }
+  *images = ctx->bp_allocated;
+  return STRIP_MLEM_OK;
+}
+
+// Whether most boxes (those of level events) fit kept_event_kernel's cache.
+bool small_boxes(const DeviceGeometry& g) {
+  const double half_z =
+      1.5 * std::sqrt(2.0 / g.inv_pow_sigma_z) / g.pixel_width;
+  const double half_y = 1.5 / std::sqrt(g.inv_pow_sigma_dl) / g.pixel_height;
+  return std::min(2.0 * half_z, (double)g.n_z) *
+             std::min(2.0 * half_y, (double)g.n_y) <= kBboxCache;
 }
 
 // One event pass: forward + back-projection of every resident event into bp.
-int launch_event_pass(strip_mlem_ctx* ctx, const float* rho) {
+int launch_event_pass(strip_mlem_ctx* ctx, const float* rho, int images) {
   if (ctx->n_events == 0) return STRIP_MLEM_OK;
   const int grid = grid_for_events(ctx, ctx->n_events);
+  ModeFlags m = mode_flags(ctx->mode);
+  m.bp_images = images;
   if (is_fast_mode(ctx->mode)) {
     hipLaunchKernelGGL((bbox_event_kernel<true, true>), dim3(grid),
-                       dim3(ctx->threads), 0, ctx->stream, ctx->g,
-                       mode_flags(ctx->mode), ctx->ev.a, ctx->ev.b,
-                       ctx->ev.box, ctx->n_events, rho, ctx->sens, ctx->bp,
-                       nullptr);
+                       dim3(ctx->threads), 0, ctx->stream, ctx->g, m,
+                       ctx->ev.a, ctx->ev.b, ctx->ev.box, ctx->n_events, rho,
+                       ctx->sens, ctx->bp, nullptr);
+  } else if (ctx->mode.kernel == 1 && ctx->threads == 256 &&
+             small_boxes(ctx->g)) {
+    hipLaunchKernelGGL(kept_event_kernel, dim3(grid), dim3(256), 0,
+                       ctx->stream, ctx->g, m, ctx->ev.a, ctx->ev.b,
+                       ctx->ev.box, ctx->n_events, rho, ctx->sens, ctx->bp);
   } else {
-    hipLaunchKernelGGL(generic_event_kernel, dim3(grid),
-                       dim3(ctx->threads), 0, ctx->stream, ctx->g,
-                       mode_flags(ctx->mode), ctx->ev.a, ctx->ev.b,
-                       ctx->ev.box, ctx->n_events, rho, ctx->sens, ctx->bp,
-                       ctx->bp_copies);
+    hipLaunchKernelGGL((bbox_event_kernel<false, true>), dim3(grid),
+                       dim3(ctx->threads), 0, ctx->stream, ctx->g, m,
+                       ctx->ev.a, ctx->ev.b, ctx->ev.box, ctx->n_events, rho,
+                       ctx->sens, ctx->bp, nullptr);
   }
   HIP_TRY(hipGetLastError());
   return STRIP_MLEM_OK;
@@ -698,12 +761,14 @@ int launch_iteration(strip_mlem_ctx* ctx) {
   const float* rho = ctx->rho[ctx->cur];
   float* rho_next = ctx->rho[ctx->cur ^ 1];
   hipEvent_t marks[4] = {nullptr, nullptr, nullptr, nullptr};
+  int images = 1;
+  int rc = bp_images(ctx, &images);
+  if (rc) return rc;
   if (ctx->timing) {
-    int rc = record_marks(ctx, marks);
-    if (rc) return rc;
+    if ((rc = record_marks(ctx, marks))) return rc;
     HIP_TRY(hipEventRecord(marks[0], ctx->stream));
   }
-  int rc = launch_event_pass(ctx, rho);
+  rc = launch_event_pass(ctx, rho, images);
   if (rc) return rc;
   if (ctx->timing) {
     HIP_TRY(hipEventRecord(marks[1], ctx->stream));
@@ -711,7 +776,7 @@ int launch_iteration(strip_mlem_ctx* ctx) {
   }
   const int blocks = std::max(1, std::min((ctx->n_pixels + 255) / 256, 4096));
   hipLaunchKernelGGL(finalize_kernel, dim3(blocks), dim3(256), 0, ctx->stream,
-                     ctx->n_pixels, rho, ctx->bp, ctx->bp_copies, ctx->sens,
+                     ctx->n_pixels, rho, ctx->bp, images, ctx->sens,
                      ctx->mode.sensitivity == 2 ? 1 : 0, rho_next);
   HIP_TRY(hipGetLastError());
   if (ctx->timing) HIP_TRY(hipEventRecord(marks[3], ctx->stream));
@@ -757,7 +822,6 @@ int band_iterations(strip_mlem_ctx* ctx, int n_iterations) {
 }
 
 // Differentiation needs the CPU-path semantics on the row-band plan.
-int fill(strip_mlem_ctx* ctx, float* ptr, int64_t n, float value);
 int ensure_subsets(strip_mlem_ctx* ctx);
 
 int adjoint_ready(strip_mlem_ctx* ctx, bool full_plan = true) {
@@ -1152,28 +1216,13 @@ int strip_mlem_create(const strip_mlem_geometry* geometry,
   if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) !=
       hipSuccess)
     return cleanup(strip::fail(STRIP_MLEM_ERR_HIP, "hipStreamCreate failed"));
-  if ((m.kernel != 0 || m.sensitivity == 1) &&
-      ctx->n_pixels <= kBpCopiesPixels)
-    ctx->bp_copies = kBpCopies;
-  if (hipMalloc(&ctx->bp, sizeof(float) * ctx->n_pixels * ctx->bp_copies) !=
-      hipSuccess) {
-    ctx->bp = nullptr;
-    // where the copies do not fit, one serves as well
-    if (ctx->bp_copies > 1) {
-      (void)hipGetLastError();
-      ctx->bp_copies = 1;
-      if (hipMalloc(&ctx->bp, sizeof(float) * ctx->n_pixels) != hipSuccess)
-        ctx->bp = nullptr;
-    }
-  }
   if (hipMalloc(&ctx->rho[0], sizeof(float) * ctx->n_pixels) != hipSuccess ||
       hipMalloc(&ctx->rho[1], sizeof(float) * ctx->n_pixels) != hipSuccess ||
-      !ctx->bp ||
+      hipMalloc(&ctx->bp, sizeof(float) * ctx->n_pixels) != hipSuccess ||
       hipMalloc(&ctx->counter, sizeof(unsigned long long)) != hipSuccess)
     return cleanup(strip::fail(STRIP_MLEM_ERR_ALLOC, "cannot allocate images"));
   if ((rc = fill(ctx, ctx->rho[0], ctx->n_pixels, 1.0f)) ||
-      (rc = fill(ctx, ctx->bp, (int64_t)ctx->n_pixels * ctx->bp_copies,
-                 0.0f)) ||
+      (rc = fill(ctx, ctx->bp, ctx->n_pixels, 0.0f)) ||
       (rc = ensure_mode_sensitivity(ctx)))
     return cleanup(rc);
   if (hipStreamSynchronize(ctx->stream) != hipSuccess)
@@ -1228,7 +1277,8 @@ int strip_mlem_set_events(strip_mlem_ctx* ctx, const float* responses,
   ctx->subsets_dirty = true;
   if ((rc = upload_events(ctx, responses, 0, n))) return rc;
   ctx->n_events = n;
-  return STRIP_MLEM_OK;
+  int images = 0;
+  return bp_images(ctx, &images);
 }
 
 int strip_mlem_reserve_events(strip_mlem_ctx* ctx, int64_t n_events) {
@@ -1269,7 +1319,8 @@ int strip_mlem_set_events_device(strip_mlem_ctx* ctx,
   ctx->n_events = n;
   ctx->band_dirty = true;
   ctx->subsets_dirty = true;
-  return STRIP_MLEM_OK;
+  int images = 0;
+  return bp_images(ctx, &images);
 }
 
 int64_t strip_mlem_n_events(const strip_mlem_ctx* ctx) {

@@ -81,8 +81,18 @@ struct MomentInstance {
   int64_t n_events;
 };
 
+// The row-band tiling that a plan's events would have as lists.
+struct ListTiling {
+  bool known = false;
+  int forward_group = 0, backward_group = 0;
+  int forward_rows = 0, backward_rows = 0;
+  int window_columns = 0;
+  int64_t forward_pairs = 0, backward_pairs = 0;
+};
+
 struct MomentPlan {
   bool ready = false;
+  ListTiling tiling;  // looked up when a caller first asks for it
   int64_t n_events = 0, n_pairs = 0;
   int n_bins = 0, n_groups = 0;
   int n_fwd = 0, n_bwd = 0;
