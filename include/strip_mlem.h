@@ -215,7 +215,8 @@ int strip_mlem_set_backprojection_occupancy(strip_mlem_ctx* ctx,
  * and the table takes at most half the free device memory), 0 = each
  * iteration solves the runs again.  Same pixels either way.  Takes effect at
  * the next upload-time plan (next iteration).  strip_mlem_get_span_table
- * reports whether the plan in use has the table (1) or not (0). */
+ * reports whether the plan in use keeps its rows' runs (1) or not (0): in the
+ * table, or, in the moment form, with its pairs. */
 int strip_mlem_set_span_table(strip_mlem_ctx* ctx, int enable);
 int strip_mlem_get_span_table(strip_mlem_ctx* ctx, int* in_use);
 
@@ -229,8 +230,11 @@ int strip_mlem_get_plan_forms(strip_mlem_ctx* ctx, int* moment_plans,
 
 /* The row-band tiling: band rows of both kernels, the widest
  * back-projection task window (columns) and the number of (event, band) pairs
- * of both kernels (where the moment form is in use, those its events would
- * have). */
+ * of both kernels.  Where the moment form is in use (strip_mlem_get_plan_forms),
+ * the tiling its events would have as lists, as with strip_mlem_get_band_groups:
+ * the first call on a plan builds those lists and releases them, which takes the
+ * time of building a plan and, where memory is short, drops the moment form's
+ * plan, which the next iteration builds again. */
 int strip_mlem_get_band_tiling(strip_mlem_ctx* ctx, int* forward_rows,
                                int* backward_rows, int* window_columns,
                                int64_t* forward_pairs,

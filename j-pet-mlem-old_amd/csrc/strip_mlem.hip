@@ -973,13 +973,12 @@ int unrolled_gradient_device(strip_mlem_ctx* ctx, const float* d_rho0,
 
 // The plans the iterations run: the subset (or split) plans when there are
 // several (they share one tuning), else the whole-list plan.
-int active_plans(strip_mlem_ctx* ctx,
-                 std::vector<const strip::BandPlan*>& plans) {
+int active_plans(strip_mlem_ctx* ctx, std::vector<strip::BandPlan*>& plans) {
   plans.clear();
   if (plan_parts(ctx) > 1) {
     int rc = ensure_subsets(ctx);
     if (rc) return rc;
-    for (const strip::BandPlan& p : ctx->subsets) plans.push_back(&p);
+    for (strip::BandPlan& p : ctx->subsets) plans.push_back(&p);
   } else {
     int rc = ensure_band(ctx);
     if (rc) return rc;
@@ -988,55 +987,78 @@ int active_plans(strip_mlem_ctx* ctx,
   return STRIP_MLEM_OK;
 }
 
-// The row-band tiling that the resident events' plans have, or, for plans in
-// the moment form, would have: those plans' lists are built, described and
-// released again.
-int describe_tiling(strip_mlem_ctx* ctx, int* forward_group,
-                    int* backward_group, int* forward_rows,
-                    int* backward_rows, int* window_columns,
-                    int64_t* forward_pairs, int64_t* backward_pairs) {
-  std::vector<const strip::BandPlan*> plans;
+// The row-band tiling of a plan, or, in the moment form, the one that its events
+// (`view`) would have: their lists are built, described and released again, once
+// per plan.  Where they do not fit beside the moment form, it makes room for them
+// and is built again when it is next needed.
+int plan_tiling(strip_mlem_ctx* ctx, strip::BandPlan& p, const EventSoA& view,
+                strip::ListTiling* t) {
+  if (p.moment.ready && p.moment.tiling.known) {
+    *t = p.moment.tiling;
+    return STRIP_MLEM_OK;
+  }
+  strip::BandPlan lists;
+  const strip::BandPlan* described = &p;
+  if (p.moment.ready) {
+    lists.tuning = p.tuning;
+    lists.tuning.moments = 0;
+    for (;;) {
+      lists.rhoT[0] = p.rhoT[0];
+      lists.rhoT[1] = p.rhoT[1];
+      lists.bpT = p.bpT;
+      lists.owns_images = false;
+      std::string err;
+      if (!strip::band_prepare(lists, ctx->g, view, p.n_events, ctx->stream,
+                               &err))
+        break;
+      strip::band_release(lists);
+      (void)hipGetLastError();
+      if (!p.moment.ready)
+        return strip::fail(STRIP_MLEM_ERR_HIP, "band plan: " + err);
+      strip::moment_release(p.moment);
+      p.ready = false;
+    }
+    described = &lists;
+  }
+  *t = strip::ListTiling{true,
+                         described->fwd_group,
+                         described->bwd_group,
+                         described->fwd.H,
+                         described->bwd.H,
+                         described->bwd.Wt,
+                         described->fwd.n_pairs,
+                         described->bwd.n_pairs};
+  if (described == &lists) {
+    strip::band_release(lists);
+    if (p.moment.ready) p.moment.tiling = *t;
+  }
+  return STRIP_MLEM_OK;
+}
+
+// The tiling of the resident events: the first plan's groups and rows, the widest
+// window, all plans' pairs.
+int describe_tiling(strip_mlem_ctx* ctx, strip::ListTiling* all) {
+  std::vector<strip::BandPlan*> plans;
   int rc = active_plans(ctx, plans);
   if (rc) return rc;
-  int wt = 0;
-  int64_t nf = 0, nb = 0;
-  for (size_t i = 0; i < plans.size(); ++i) {
-    const strip::BandPlan* p = plans[i];
-    strip::BandPlan lists;
-    if (p->moment.ready) {
-      std::string err;
-      const int64_t parts = (int64_t)plans.size();
-      const int64_t lo = ctx->n_events * (int64_t)i / parts;
-      const EventSoA view{ctx->ev.a + lo, ctx->ev.b + lo, ctx->ev.c + lo,
-                          ctx->ev.box + lo};
-      lists.tuning = p->tuning;
-      lists.tuning.moments = 0;
-      lists.rhoT[0] = p->rhoT[0];
-      lists.rhoT[1] = p->rhoT[1];
-      lists.bpT = p->bpT;
-      lists.owns_images = false;
-      const int failed = strip::band_prepare(lists, ctx->g, view, p->n_events,
-                                             ctx->stream, &err);
-      p = &lists;
-      if (failed) {
-        strip::band_release(lists);
-        return strip::fail(STRIP_MLEM_ERR_HIP, "band plan: " + err);
-      }
-    }
+  *all = strip::ListTiling{};
+  const int64_t parts = (int64_t)plans.size();
+  for (int64_t i = 0; i < parts; ++i) {
+    const int64_t lo = ctx->n_events * i / parts;
+    strip::ListTiling t;
+    if ((rc = plan_tiling(ctx, *plans[i],
+                          EventSoA{ctx->ev.a + lo, ctx->ev.b + lo,
+                                   ctx->ev.c + lo, ctx->ev.box + lo},
+                          &t)))
+      return rc;
     if (i == 0) {
-      if (forward_group) *forward_group = p->fwd_group;
-      if (backward_group) *backward_group = p->bwd_group;
-      if (forward_rows) *forward_rows = p->fwd.H;
-      if (backward_rows) *backward_rows = p->bwd.H;
+      *all = t;
+      continue;
     }
-    wt = std::max(wt, p->bwd.Wt);
-    nf += p->fwd.n_pairs;
-    nb += p->bwd.n_pairs;
-    if (p == &lists) strip::band_release(lists);
+    all->window_columns = std::max(all->window_columns, t.window_columns);
+    all->forward_pairs += t.forward_pairs;
+    all->backward_pairs += t.backward_pairs;
   }
-  if (window_columns) *window_columns = wt;
-  if (forward_pairs) *forward_pairs = nf;
-  if (backward_pairs) *backward_pairs = nb;
   return STRIP_MLEM_OK;
 }
 
@@ -1656,8 +1678,12 @@ int strip_mlem_get_band_groups(strip_mlem_ctx* ctx, int* forward_group,
   CTX_CHECK(ctx);
   if (effective_algorithm(ctx) != 2)
     return strip::fail(STRIP_MLEM_ERR_STATE, "row-band algorithm not in use");
-  return describe_tiling(ctx, forward_group, backward_group, nullptr, nullptr,
-                         nullptr, nullptr, nullptr);
+  strip::ListTiling t;
+  int rc = describe_tiling(ctx, &t);
+  if (rc) return rc;
+  if (forward_group) *forward_group = t.forward_group;
+  if (backward_group) *backward_group = t.backward_group;
+  return STRIP_MLEM_OK;
 }
 
 int strip_mlem_set_backprojection_waves(strip_mlem_ctx* ctx, int waves) {
@@ -1716,7 +1742,7 @@ int strip_mlem_get_span_table(strip_mlem_ctx* ctx, int* in_use) {
   if (!in_use) return strip::fail(STRIP_MLEM_ERR_ARGUMENT, "NULL output");
   *in_use = 0;
   if (effective_algorithm(ctx) != 2) return STRIP_MLEM_OK;
-  std::vector<const strip::BandPlan*> plans;
+  std::vector<strip::BandPlan*> plans;
   int rc = active_plans(ctx, plans);
   if (rc) return rc;
   bool any = false, all = true;
@@ -1737,7 +1763,7 @@ int strip_mlem_get_plan_forms(strip_mlem_ctx* ctx, int* moment_plans,
     return strip::fail(STRIP_MLEM_ERR_ARGUMENT, "NULL output");
   *moment_plans = *list_plans = 0;
   if (effective_algorithm(ctx) != 2) return STRIP_MLEM_OK;
-  std::vector<const strip::BandPlan*> plans;
+  std::vector<strip::BandPlan*> plans;
   int rc = active_plans(ctx, plans);
   if (rc) return rc;
   for (const strip::BandPlan* p : plans)
@@ -1752,8 +1778,15 @@ int strip_mlem_get_band_tiling(strip_mlem_ctx* ctx, int* forward_rows,
   CTX_CHECK(ctx);
   if (effective_algorithm(ctx) != 2)
     return strip::fail(STRIP_MLEM_ERR_STATE, "row-band algorithm not in use");
-  return describe_tiling(ctx, nullptr, nullptr, forward_rows, backward_rows,
-                         window_columns, forward_pairs, backward_pairs);
+  strip::ListTiling t;
+  int rc = describe_tiling(ctx, &t);
+  if (rc) return rc;
+  if (forward_rows) *forward_rows = t.forward_rows;
+  if (backward_rows) *backward_rows = t.backward_rows;
+  if (window_columns) *window_columns = t.window_columns;
+  if (forward_pairs) *forward_pairs = t.forward_pairs;
+  if (backward_pairs) *backward_pairs = t.backward_pairs;
+  return STRIP_MLEM_OK;
 }
 
 int strip_mlem_kernel_evaluations(strip_mlem_ctx* ctx, int64_t* count) {

@@ -448,7 +448,8 @@ class Reconstruction:
         _check(self._lib.strip_mlem_set_span_table(self._ctx, int(bool(enable))))
 
     def span_table(self) -> bool:
-        """Whether the plan in use has the span table."""
+        """Whether the plan in use keeps its rows' runs (span table, or with
+        the pairs in the moment form)."""
         v = ctypes.c_int()
         _check(self._lib.strip_mlem_get_span_table(self._ctx, ctypes.byref(v)))
         return bool(v.value)

@@ -22,7 +22,16 @@ struct Launch {
   void* first;  // first eight bytes of the arguments
 };
 
+// What a kernel would have written: `bytes` to the memory its argument `arg`
+// points to.
+struct Effect {
+  std::string part;
+  int arg;
+  std::vector<char> bytes;
+};
+
 std::mutex lock;
+std::vector<Effect> effects;
 std::map<const void*, std::string> names;
 std::vector<Launch> launches;
 std::set<void*> live;
@@ -47,6 +56,11 @@ void stub_fail_in(long k) { fail_in = k; }
 long stub_allocations() { return allocations; }
 long stub_live() { return (long)live.size(); }
 void stub_clear_launches() { launches.clear(); }
+// launches of kernels whose name holds `part` write n bytes to the memory that
+// their argument `arg` points to
+void stub_effect(const char* part, int arg, const char* bytes, size_t n) {
+  effects.push_back({part, arg, std::vector<char>(bytes, bytes + n)});
+}
 // launches of kernels whose name holds `part`; null_first: only those whose
 // first argument is a null pointer; over: only those of more work-items
 long stub_launches(const char* part, int null_first, unsigned long long over) {
@@ -102,6 +116,10 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args,
   Launch l{names.count(f) ? names[f] : "?", grid, block, nullptr};
   std::memcpy(&l.first, args[0], sizeof(void*));
   launches.push_back(l);
+  for (const Effect& e : effects)
+    if (l.kernel.find(e.part) != std::string::npos)
+      std::memcpy(*static_cast<void**>(args[e.arg]), e.bytes.data(),
+                  e.bytes.size());
   return hipSuccess;
 }
 

@@ -22,6 +22,8 @@ stub.stub_launches.argtypes = [ctypes.c_char_p, ctypes.c_int,
 stub.stub_launches.restype = ctypes.c_long
 stub.stub_work_items.argtypes = [ctypes.c_char_p]
 stub.stub_work_items.restype = ctypes.c_ulonglong
+stub.stub_effect.argtypes = [ctypes.c_char_p, ctypes.c_int, ctypes.c_char_p,
+                             ctypes.c_size_t]
 sys.path.insert(0, {package!r})
 import pystrip
 result = None
