@@ -31,6 +31,9 @@ thread_local std::string g_last_error;
 
 int fail(int code, const std::string& message) {
   g_last_error = message;
+  // (the runtime's own note of it would be taken for an error of the next
+  // kernel launch)
+  (void)hipGetLastError();
   return code;
 }
 
