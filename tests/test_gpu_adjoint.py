@@ -22,7 +22,8 @@ pytestmark = pytest.mark.gpu
 CFG = "strip-256x160-2mm-1e6"
 
 
-def _case(pystrip_mod, phantom_mod, oracle_mod, n, sigma_scale=1.0, seed=21):
+def _case(pystrip_mod, phantom_mod, oracle_mod, n, sigma_scale=1.0, seed=21,
+          algorithm=0):
     w = phantom_mod.WORKLOADS[CFG]
     ev = w.events(n, seed=seed)
     g = w.geometry()
@@ -33,15 +34,21 @@ def _case(pystrip_mod, phantom_mod, oracle_mod, n, sigma_scale=1.0, seed=21):
     t[7] *= sigma_scale
     og = oracle_mod.geometry(*t)
     rec = pystrip_mod.Reconstruction(g, pystrip_mod.MODE_CPU)
+    rec.set_algorithm(algorithm)
     rec.set_events(ev)
+    # 0: these events take the moment form; 2: the lists
+    assert rec.plan_forms() == ((0, 1) if algorithm else (1, 0))
     return w, ev, g, og, rec
 
 
+@pytest.mark.parametrize("algorithm", [0, 2])
 @pytest.mark.parametrize("sigma_scale", [1.0, 1.4])
-def test_loglik_gradient(pystrip_mod, phantom_mod, oracle_mod, sigma_scale):
-    print_case("log-likelihood gradient, sigma scale", sigma_scale)
+def test_loglik_gradient(pystrip_mod, phantom_mod, oracle_mod, sigma_scale,
+                         algorithm):
+    print_case("log-likelihood gradient, sigma scale", sigma_scale,
+               "algorithm", algorithm)
     w, ev, g, og, rec = _case(pystrip_mod, phantom_mod, oracle_mod, 20000,
-                              sigma_scale)
+                              sigma_scale, algorithm=algorithm)
     rng = np.random.default_rng(2)
     rho = rng.uniform(0.5, 1.5, size=rec.shape).astype(np.float32)
     value, grad, gs = rec.loglik_gradient(rho)
@@ -66,11 +73,14 @@ def test_loglik_gradient_current_image(pystrip_mod, phantom_mod, oracle_mod):
     assert np.allclose(s0, s1, rtol=1e-6)
 
 
+@pytest.mark.parametrize("algorithm", [0, 2])
 @pytest.mark.parametrize("iterations", [1, 4])
-def test_unrolled_gradient(pystrip_mod, phantom_mod, oracle_mod, iterations):
-    print_case("unrolled MLEM gradient, iterations", iterations)
+def test_unrolled_gradient(pystrip_mod, phantom_mod, oracle_mod, iterations,
+                           algorithm):
+    print_case("unrolled MLEM gradient, iterations", iterations, "algorithm",
+               algorithm)
     w, ev, g, og, rec = _case(pystrip_mod, phantom_mod, oracle_mod, 3000,
-                              sigma_scale=1.4)
+                              sigma_scale=1.4, algorithm=algorithm)
     rng = np.random.default_rng(5)
     rho0 = rng.uniform(0.5, 1.5, size=rec.shape).astype(np.float32)
     target = rng.uniform(0.0, 2.0, size=rec.shape).astype(np.float32)

@@ -18,8 +18,8 @@ from conftest import print_case
 pytestmark = pytest.mark.gpu
 
 # n_z, n_y, pixel width, height, sigma_z, sigma_dl, R, L, phantom half sizes,
-# events.  All of them take the moment form: where bins hold few pairs, wide lines
-# and many bins stay on the lists.
+# events.  All of them take the moment form (asserted): where bins hold few pairs,
+# wide lines and many bins stay on the lists.
 CASES = {
     "command line defaults, sigma 1.5 px": (
         100, 100, 0.01, 0.01, 0.015, 0.06, 0.5, 1.0, 0.3, 0.3, 20_011),
@@ -33,9 +33,9 @@ CASES = {
         12, 200, 2.0, 2.0, 12.0, 42.0, 300.0, 500.0, 20.0, 150.0, 4_000),
     "steep events": (
         200, 64, 2.0, 2.0, 10.0, 30.0, 70.0, 1200.0, 150.0, 40.0, 5_000),
-    "one event": (256, 160, 2.0, 2.0, 10.0, 42.0, 350.0, 500.0, 80.0, 60.0, 1),
+    "one event": (128, 80, 4.0, 4.0, 10.0, 42.0, 350.0, 500.0, 80.0, 60.0, 1),
     "seventeen events": (
-        256, 160, 2.0, 2.0, 10.0, 42.0, 350.0, 500.0, 80.0, 60.0, 17),
+        128, 80, 4.0, 4.0, 10.0, 42.0, 350.0, 500.0, 80.0, 60.0, 17),
     "wide line, dense bins": (
         300, 200, 1.0, 1.0, 10.0, 42.0, 250.0, 500.0, 40.0, 30.0, 30_000),
     # more than 12000 bins of few pairs on short lines: merged
@@ -66,6 +66,7 @@ def test_moment_form_against_oracle(pystrip_mod, phantom_mod, oracle_mod,
     ev, g, og = _case(pystrip_mod, phantom_mod, oracle_mod, name)
     rec = pystrip_mod.Reconstruction(g)
     rec.set_events(ev)
+    assert rec.plan_forms() == (1, 0)
     _, ne = oracle_mod.support_counts(og, ev)
     assert rec.kernel_evaluations() == int(ne.sum())
     rho = np.random.default_rng(3).uniform(0.5, 2.0, rec.shape).astype(
@@ -101,6 +102,7 @@ def test_moment_form_non_finite_pixels(pystrip_mod, phantom_mod, oracle_mod):
             rec = pystrip_mod.Reconstruction(g)
             rec.set_algorithm(algorithm)
             rec.set_events(ev)
+            assert rec.plan_forms() == (1 - algorithm, 0)
             rec.rho = rho
             out.append(rec.forward())
         fine = np.isfinite(out[0])
@@ -153,38 +155,116 @@ def test_moment_form_knobs(pystrip_mod, phantom_mod, oracle_mod):
     tiling = rec.band_tiling()
     assert tiling[:2] == (32, 16) and rec.band_groups() == (2, 4)
     assert rec.span_table()
-    for change in (lambda: None, lambda: rec.set_exp_mode(0),
-                   lambda: rec.set_exp_mode(1),
-                   lambda: rec.set_span_table(False),
-                   lambda: rec.set_span_table(True),
-                   lambda: rec.set_algorithm(2),
-                   lambda: rec.set_algorithm(0)):
+    for change, forms in ((lambda: None, (1, 0)),
+                          (lambda: rec.set_exp_mode(0), (0, 1)),
+                          (lambda: rec.set_exp_mode(1), (1, 0)),
+                          (lambda: rec.set_span_table(False), (0, 1)),
+                          (lambda: rec.set_span_table(True), (1, 0)),
+                          (lambda: rec.set_algorithm(2), (0, 1)),
+                          (lambda: rec.set_algorithm(0), (1, 0))):
         change()
+        assert rec.plan_forms() == forms
         rec.rho = np.ones(rec.shape, np.float32)
         rec.iterate(2)
         assert oracle_mod.rel_l2(rec.rho, ref) <= 1e-4
         assert rec.band_tiling()[:2] == tiling[:2]
 
 
-def test_moment_form_in_a_batch(pystrip_mod, phantom_mod, oracle_mod):
-    # members of every kind of task (few and many terms, merged, one and four
-    # wavefronts) and one that stays on the lists, iterated together, eagerly
-    # and replayed
-    names = ["full bins", "many small bins", "wide line, dense bins",
-             "command line defaults, sigma 1.5 px", "one event"]
+@pytest.mark.parametrize("name", list(CASES))
+def test_moment_form_gradient_against_oracle(pystrip_mod, phantom_mod,
+                                             oracle_mod, name):
+    # the log-likelihood and its derivatives in FP64.  An event's log D is
+    # within 1e-5 (above), its share of d ln sigma, of a size of one, within
+    # 2e-5; images as everywhere against FP64: 1e-4.
+    print_case("moment form, gradient:", name)
+    ev, g, og = _case(pystrip_mod, phantom_mod, oracle_mod, name)
+    rec = pystrip_mod.Reconstruction(g)
+    rec.set_events(ev)
+    assert rec.plan_forms() == (1, 0)
+    rho = np.random.default_rng(8).uniform(0.5, 2.0, rec.shape).astype(
+        np.float32)
+    value, grad, gs = rec.loglik_gradient(rho)
+    rv, rg, rs = oracle_mod.loglik_grad(og, ev.astype(np.float64),
+                                        rho.astype(np.float64))
+    print("value", value, rv, "image", oracle_mod.rel_l2(grad, rg), "sigma",
+          gs, rs)
+    assert abs(value - rv) <= 1e-5 * len(ev) + 2e-6 * abs(rv)
+    assert oracle_mod.rel_l2(grad, rg) <= 1e-4
+    sigma = np.array([g.sigma_z, g.sigma_dl])
+    assert np.all(np.abs(gs - rs) <= 1e-3 * np.abs(rs) + 2e-5 * len(ev) / sigma)
+
+
+def test_moment_form_gradient_non_finite_pixels(pystrip_mod, phantom_mod,
+                                                oracle_mod):
+    # as the lists give it: the events whose support holds the pixel drop out
+    # of the image derivative, and no others
+    ev, g, og = _case(pystrip_mod, phantom_mod, oracle_mod,
+                      "object beyond every edge")
+    for value in (np.inf, np.nan):
+        print_case("moment form, gradient, pixel =", value)
+        rho = np.ones((g.n_y_pixels, g.n_z_pixels), np.float32)
+        rho[20, 30] = value
+        rho[5, 1] = value
+        out = []
+        for algorithm in (2, 0):
+            rec = pystrip_mod.Reconstruction(g)
+            rec.set_algorithm(algorithm)
+            rec.set_events(ev)
+            assert rec.plan_forms() == ((0, 1) if algorithm else (1, 0))
+            out.append(rec.loglik_gradient(rho))
+        for a, b in zip(*out):
+            a, b = np.asarray(a), np.asarray(b)
+            assert np.array_equal(np.isnan(a), np.isnan(b))
+            assert np.array_equal(np.isinf(a), np.isinf(b))
+        assert np.all(np.isfinite(out[0][1]))
+        assert oracle_mod.rel_l2(out[1][1], out[0][1]) <= 1e-5
+
+
+# members of a batch in the moment form, which has to be a seventh faster than the
+# lists there: as CASES
+DENSE = {
+    # 90 pairs to a bin: one wavefront to a forward task
+    "eight terms, one wavefront": (300, 200, 1.0, 1.0, 10.0, 42.0, 250.0,
+                                   500.0, 40.0, 30.0, 60_000),
+    # 180: four
+    "eight terms, four wavefronts": (300, 200, 1.0, 1.0, 10.0, 42.0, 250.0,
+                                     500.0, 40.0, 30.0, 120_000),
+    # 15 cells, 30000 bins of under 100 pairs
+    "merged tasks": (381, 203, 1.25, 1.25, 7.5, 35.0, 300.0, 700.0, 150.0,
+                     90.0, 450_000),
+    # more than 400 pairs to every bin, in two sizes of LDS
+    "six terms": (60, 32, 2.0, 2.0, 30.0, 42.0, 200.0, 200.0, 50.0, 25.0,
+                  300_000),
+    "six terms, shorter lines": (60, 32, 2.5, 2.5, 30.0, 42.0, 200.0, 200.0,
+                                 50.0, 25.0, 300_000),
+}
+
+
+@pytest.mark.parametrize("names", [
+    ["six terms", "eight terms, one wavefront", "merged tasks",
+     "wide line, dense bins", "eight terms, four wavefronts",
+     "six terms, shorter lines", "one event"],
+    # no member over lists, the same kind twice
+    ["six terms, shorter lines", "six terms"],
+    ["eight terms, one wavefront"]])
+def test_moment_form_in_a_batch(pystrip_mod, phantom_mod, oracle_mod, names,
+                                monkeypatch):
+    # members of every kind of task, several to a launch, among members over
+    # lists, iterated together, eagerly and replayed
     print_case("moment form in a batch:", names)
+    monkeypatch.setattr("test_gpu_moment.CASES", {**CASES, **DENSE})
     cases = [_case(pystrip_mod, phantom_mod, oracle_mod, n) for n in names]
-    ev, g, og = cases[2]
-    cases.append((ev[:300], g, og))  # wide lines, sparse: lists
+    refs = [oracle_mod.mlem(og, ev, iterations=5) for ev, _, og in cases]
     for graph in (False, True):
         b = pystrip_mod.Batch()
         b.set_graph(graph)
         for ev, g, _ in cases:
             b.add(g, ev)
         b.iterate(2)
-        b.iterate(5)
-        for i, (ev, g, og) in enumerate(cases):
-            ref = oracle_mod.mlem(og, ev, iterations=7)
-            e = oracle_mod.rel_l2(b.rho(i), ref)
-            print(i, e)
+        b.iterate(3)
+        for i, name in enumerate(names):
+            e = oracle_mod.rel_l2(b.rho(i), refs[i])
+            print(name, b.member(i).plan_forms(), e)
+            assert b.member(i).plan_forms() == ((1, 0) if name in DENSE
+                                                else (0, 1))
             assert e <= 1e-4
