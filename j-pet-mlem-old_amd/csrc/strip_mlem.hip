@@ -1241,13 +1241,17 @@ int strip_mlem_create(const strip_mlem_geometry* geometry,
   if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) !=
       hipSuccess)
     return cleanup(strip::fail(STRIP_MLEM_ERR_HIP, "hipStreamCreate failed"));
+  // small images are allocated together, others when they are wanted
+  if ((m.kernel != 0 || m.sensitivity == 1) && ctx->n_pixels <= 1 << 18)
+    ctx->bp_allocated = kBpImages;
+  const int64_t bp_pixels = (int64_t)ctx->n_pixels * ctx->bp_allocated;
   if (hipMalloc(&ctx->rho[0], sizeof(float) * ctx->n_pixels) != hipSuccess ||
       hipMalloc(&ctx->rho[1], sizeof(float) * ctx->n_pixels) != hipSuccess ||
-      hipMalloc(&ctx->bp, sizeof(float) * ctx->n_pixels) != hipSuccess ||
+      hipMalloc(&ctx->bp, sizeof(float) * bp_pixels) != hipSuccess ||
       hipMalloc(&ctx->counter, sizeof(unsigned long long)) != hipSuccess)
     return cleanup(strip::fail(STRIP_MLEM_ERR_ALLOC, "cannot allocate images"));
   if ((rc = fill(ctx, ctx->rho[0], ctx->n_pixels, 1.0f)) ||
-      (rc = fill(ctx, ctx->bp, ctx->n_pixels, 0.0f)) ||
+      (rc = fill(ctx, ctx->bp, bp_pixels, 0.0f)) ||
       (rc = ensure_mode_sensitivity(ctx)))
     return cleanup(rc);
   if (hipStreamSynchronize(ctx->stream) != hipSuccess)
