@@ -1407,10 +1407,9 @@ constexpr size_t kLds = 160 * 1024;
 // offsets round decides their kernel values.
 constexpr double kMinSigmaPixels = 1.4;
 constexpr int kFwdChunk = 2048;  // pairs of a forward workgroup's task
-// back-projection tasks of several bins (moment_prepare says when)
+// back-projection tasks of several bins (merge_bins says when)
 constexpr int kMergedPositions = 16;
-constexpr int kMergedBins = 12000;
-constexpr double kMergedPairs = 100.0;
+constexpr int kMergedBins = 10500;
 constexpr double kMergedSpan = 6.0;  // columns of a merged task's vertices
 constexpr int kMergedTasks = 4096;   // tasks aimed at, of 8 to 64 groups
 constexpr int kBwdChunk = 1024;  // pairs of a back-projection wavefront's task
@@ -1435,10 +1434,22 @@ size_t table_bytes(int positions, int terms) {
          (2 * (size_t)(positions + 1) * R * terms + (terms == 6 ? 32 : 0));
 }
 
-// Whether back-projection tasks hold several bins (of 8 terms).
+// Whether back-projection tasks hold several bins (of 8 terms).  Their pixels are
+// summed in LDS first: 16 x 2 cells per bin added to the images one by one
+// outweigh a few pairs' own work.  It takes bins for full tasks, and short lines,
+// as the pixels' LDS comes on top of the cells'; with more pairs to a bin the
+// wavefronts that this LDS costs count for more.  An iteration with one bin to a
+// task and merged (cells, bins, pairs per bin):
+//   5, 18100, 3.3: 42, 41 us       5, 25800, 15: 66, 65 us    5, 27800, 29: 82, 94
+//   7, 6400, 1.2: 24, 30 us        7, 32700, 16: 95, 94 us    7, 34300, 30: 115, 137
+//   9, 15000, 1.1: 66, 53 us       9, 147000, 15: 588, 471    9, 157000, 35: 753, 736
+//   10, 10300, 3.2: 46, 45 us      10, 12500, 7.9: 54, 53     10, 13500, 24: 66, 78
+//   13, 5600, 8.3: 40, 48 us       13, 98000, 18: 592, 472    13, 105000, 41: 753, 749
+//   15, 10400, 1.6: 68, 55 us      15, 27400, 21: 190, 161    15, 29500, 77: 274, 339
+//   19, 57700, 4.1: 342, 322 us    20, 30700, 21: 224, 246 us
 bool merge_bins(int positions, double pairs, double bins) {
   return positions <= kMergedPositions && bins >= kMergedBins &&
-         pairs < kMergedPairs * bins;
+         pairs < std::min(bins / 1000.0, 2.4 * positions) * bins;
 }
 
 // What the time of an iteration in either form depends on.
@@ -1456,13 +1467,14 @@ struct FormSizes {
 // than walking the runs' pixels, and more so the more cells a line has: it takes
 // longer, and its LDS leaves fewer wavefronts to a CU.  The lists take as long as
 // all their pairs at full throughput or as the chains of their largest tasks,
-// which are short where events are few to a band and bucket.  Times in us, fitted
-// to 1790 contexts (20 to 1600 by 24 to 800 pixels of 0.5 to 2.5 mm, sigma_z 5 to
-// 14 mm, 3 to 1e6 events); for 1690 others, at 5 and 95 %, the lists' lie at 0.87
-// and 1.19 of those measured and the moments' at 0.86 and 1.14.  There the moment
-// form is taken 1236 times, 17 times where it is more than 3 % slower (at most
-// 1.18 times), and the lists where they are more than 10 % slower 8 times (at
-// most 1.48 times).  Some of them (cells, pairs, occupied bins: lists, moments):
+// which are short where events are few to a band and bucket, and longer where they
+// solve every row's run anew.  Times in us, fitted to 1880 contexts (20 to 1600
+// by 24 to 800 pixels of 0.5 to 2.5 mm, sigma_z 5 to 14 mm, 3 to 1e6 events); for
+// 1810 others, at 5 and 95 %, the lists' lie at 0.87 and 1.18 of those measured
+// and the moments' at 0.86 and 1.14.  There the moment form is taken 1240 times,
+// 18 times where it is more than 3 % slower (at most 1.20 times), and the lists
+// where they are more than 10 % slower 8 times (at most 1.44 times).  Some of them
+// (cells, pairs, occupied bins: lists, moments):
 //   24, 3997, 3335: 25, 60 us            57, 1022, 683: 26, 58 us
 //   32, 1.2e5, 1.8e4: 189, 311 us        17, 1.8e5, 4.2e4: 237, 338 us
 //   45, 9056, 589: 420, 29 us            24, 1.2e6, 3.4e4: 488, 375 us
@@ -1479,12 +1491,14 @@ bool lists_faster(const FormSizes& s, double bins, bool batch) {
   if (batch)
     return 1.15 * (s.pairs * 0.07 + bins * 8.0 * std::pow(P / 24.0, 1.6)) >
            s.pairs * (0.04 + 0.0065 * P);
-  const double wide = s.wide ? 2.08 : 1.0;
+  const double wide = s.wide ? 1.0 : 0.0;
   const double line = std::max(P - 7.0, 0.0);
-  const double chain = (s.fwd_group * (0.0333 + 0.00343 * P) +
-                        s.bwd_group * 0.00623 * (P + 8.0 * s.slope)) * wide;
-  const double work = s.pairs * (1.015e-4 + 6.28e-6 * P) * wide;
-  const double lists = 12.4 + 0.0925 * line + 5.92e-6 * s.pixels +
+  const double chain =
+      s.fwd_group * (0.0342 + 0.00323 * P + 0.135 * wide) +
+      s.bwd_group * (0.00641 * (P + 8.0 * s.slope) + 0.135 * wide);
+  const double work = s.pairs * (9.67e-5 + 6.62e-6 * P +
+                                 (5.9e-5 + 2.58e-4 * s.slope) * wide);
+  const double lists = 12.4 + 0.0955 * line + 5.54e-6 * s.pixels +
                        std::hypot(chain, work);
   // a bin's line at the wavefronts that its cells leave room for; the chain of
   // the fullest bin
@@ -1673,9 +1687,12 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   // Six terms about lines 2.3 times closer leave room for eight instead of six
   // back-projection wavefronts per CU (24 cells) and save arithmetic, but make
   // five times the bins, each with its table and its expansion: taken where
-  // the bins stay full.  Measured per iteration with 8 and 6 terms: 947 pairs
-  // per bin (occupied or not) 12.1 and 10.8 ms, 100 pairs 0.40 and 0.44 ms, 83
-  // pairs of 48 cells 2.8 and 4.5 ms.
+  // the bins stay full.  An iteration with 8 and 6 terms (cells, pairs per bin,
+  // occupied or not):
+  //   13, 100: 0.357, 0.361 ms    13, 300: 0.905, 0.866 ms  15, 354: 2.16, 2.35 ms
+  //   24, 142: 1.99, 2.43 ms      24, 285: 3.74, 3.84 ms    24, 947: 12.1, 10.8 ms
+  //   34, 256: 1.21, 1.17 ms      34, 767: 3.17, 2.59 ms    36, 703: 0.113, 0.119
+  //   48, 155: 0.74, 0.94 ms      48, 517: 1.94, 1.82 ms    66, 447: 0.78, 0.63 ms
   if ((double)n_pairs >= 400.0 * n_bins_f) {
     terms = 6;
     if (!set_bins()) {
@@ -1853,15 +1870,6 @@ int moment_prepare(MomentPlan& plan, const DeviceGeometry& g,
   BAND_TRY(hipStreamSynchronize(stream));
   const int n_groups = totals[0];
   int merged_chunk = 0;
-  // Bins of few pairs are back-projected several to a task, whose pixels are
-  // summed in LDS first: the atomic additions to the image, 16 x 2 cells per
-  // bin, would otherwise outweigh the pairs' own work.  It
-  // takes enough bins for full tasks, and short lines, as the pixels' LDS comes
-  // on top of the cells'.  Back-projection, one bin to a task and merged: 5
-  // cells, 2.5 pairs per bin, 15700 bins 0.051 and 0.032 ms; 15 cells, 20 pairs,
-  // 27500 bins 0.182 and 0.107 ms, 58 pairs 0.212 and 0.195 ms, 185 pairs 0.35
-  // and 0.41 ms; 13 cells, 62 pairs, 7500 bins 0.050 and 0.063 ms; 24 cells, 25
-  // pairs, 31400 bins 0.185 and 0.211 ms.
   const double row_step = 0.5 * (R - 1) * (double)g.pixel_height;
   const float max_shear =
       (float)(row_step * ((double)d.nt * 0.5) * (double)d.dt);
