@@ -6,7 +6,7 @@ shows; the events are ones whose pixels in FP32 and in FP64 are nearly the same
 
 The errors differ by 2 % from run to run (the order of the additions): the
 moment form may have 1.05 times the lists'.  With all tasks adding to one image
-it has 1.19 to 1.27 times the lists'.
+it has 1.17 to 1.75 times the lists'.
 """
 import numpy as np
 import pytest
@@ -17,12 +17,15 @@ pytestmark = pytest.mark.gpu
 
 # n_z, n_y, pixel, sigma_z, sigma_dl, R, L, half sizes of the body, events, seed
 CASES = {
-    "merged tasks, few rows": (203, 56, 2.5, 10.0, 42.0, 200.0, 640.0, 150.0,
-                               40.0, 96_151, 2),
-    "one bin to a task": (476, 197, 1.5, 12.0, 42.0, 250.0, 850.0, 200.0,
-                          80.0, 150_000, 3),
+    "few rows": (203, 56, 2.5, 10.0, 42.0, 200.0, 640.0, 150.0, 40.0, 96_151,
+                 2),
+    "long lines": (476, 197, 1.5, 12.0, 42.0, 250.0, 850.0, 200.0, 80.0,
+                   150_000, 3),
+    "short lines": (194, 136, 2.5, 10.0, 30.0, 260.0, 600.0, 150.0, 100.0,
+                    137_443, 1),
+    # 17348 bins of 15.5 pairs: back-projection tasks of several bins
     "merged tasks": (194, 136, 2.5, 10.0, 30.0, 260.0, 600.0, 150.0, 100.0,
-                     137_443, 1),
+                     90_000, 1),
 }
 
 
