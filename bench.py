@@ -32,7 +32,8 @@ PEAK_FP32_TFLOPS = 157.3
 # exp2 (1), K = pre*e (1), D += K*rho (2); again Q (4), exp2 (1), K (1),
 # K*inv (1) and the image add (1).  The moment form gets the same sums with
 # fewer operations (a row costs the same whatever its run's length), so the
-# rate this gives is one of the algorithm's work, not of instructions issued.
+# rate this gives is one of the algorithm's work, not of instructions issued
+# (VALU_INSTRUCTIONS below).
 FLOPS_PER_KERNEL_EVAL = 16
 # HBM bytes per launch (read + written) of the moment kernels on the default
 # workload, from two rocprofv3 --pmc runs (FETCH_SIZE, WRITE_SIZE) each scaled
@@ -43,6 +44,10 @@ MEASURED_TRAFFIC_BYTES = {
     "forward projection": (10.36 + 1.32) * 1e9,
 }
 TRAFFIC_WORKLOAD = "strip-1000x400-1mm-2e7"
+# VALU wavefront instructions per launch there (SQ_INSTS_VALU, the same file),
+# and the nominal issue rate: one per CU and cycle, 256 CUs at 2.4 GHz
+VALU_INSTRUCTIONS = {"back-projection": 2.57e9, "forward projection": 2.23e9}
+VALU_ISSUE_PER_S = 256 * 2.4e9
 
 
 def usable_cores():
@@ -488,6 +493,10 @@ def main():
         dom_flops = n_evals * FLOPS_PER_KERNEL_EVAL
     kernel_avg_ms = kernel_ms / n_timed
     achieved_tflops = dom_flops / (dom_ms * 1e-3) / 1e12
+    # what was counted on this very workload in the moment form
+    moments, lists = rec.plan_forms()
+    counted = (w.name == TRAFFIC_WORKLOAD and n_events == w.n_events
+               and moments and not lists)
 
     rho = rec.rho
     mass = float(rho.astype(np.float64).sum())
@@ -528,10 +537,14 @@ def main():
             "peak": PEAK_FP32_TFLOPS,
             "unit": "TFLOP/s",
             "frac": achieved_tflops / PEAK_FP32_TFLOPS,
-            "traffic": (MEASURED_TRAFFIC_BYTES.get(dom_name)
-                        if w.name == TRAFFIC_WORKLOAD and
-                        n_events == w.n_events and args.algorithm == 0
-                        else None),
+            "flops_counted": "pixel by pixel; the moment form gets the same "
+                             "sums with fewer operations" if moments
+            else "pixel by pixel, as issued",
+            "plan_forms": {"moments": moments, "lists": lists},
+            "valu_issue_frac": VALU_INSTRUCTIONS[dom_name] / (dom_ms * 1e-3)
+            / VALU_ISSUE_PER_S if counted else None,
+            "traffic": MEASURED_TRAFFIC_BYTES.get(dom_name) if counted
+            else None,
             "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE + "
                             "WRITE_SIZE, copy-calibrated)",
             "kernel": dom_name,
